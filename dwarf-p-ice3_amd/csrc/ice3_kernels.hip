@@ -8,10 +8,9 @@
 // Kernels:
 //   k_ice_adjust   one thread per (level, column) point, pointwise ICE_ADJUST;
 //   k_adjust_sedim one thread per column: ICE_ADJUST and the sedimentation in one
-//                  top-down walk (the FP64 fused step);
-//   k_sedim<R>     one thread per column, walking the levels top-down: the
-//                  statistical sedimentation flux recurrence, whose fluxes
-//                  never leave registers, and the surface precipitation;
+//                  top-down walk (the FP64 fused step over many columns);
+//   k_sedim<R>     (ice3_sedim.hip) the statistical sedimentation and the surface
+//                  precipitation, a wavefront per 64 columns and species;
 //   k_micro<R>     persistent, one workgroup per compute unit, lookup tables in LDS:
 //                  the ICE4 time-split microphysics, total tendencies and negativity
 //                  correction per point, with the points still being time-stepped
@@ -22,7 +21,7 @@
 //                  decode, water and sign checks per point.  Points it rejects are
 //                  queued for k_micro_segments, the plain FP64 microphysics over the queue.
 // rain_ice is k_sedim then k_micro on one stream; the fused time step is
-// k_ice_adjust, k_sedim, k_micro.  R is the arithmetic of the process rates
+// k_ice_adjust, k_sedim, k_micro, or k_adjust_sedim, k_micro.  R is the arithmetic of the process rates
 // and lookups (double, or float for the mixed path).
 #include <hip/hip_runtime.h>
 
@@ -36,6 +35,7 @@
 #include "ice3_physics.hpp"
 #include "ice3_stages.hpp"
 #include "ice3_mlp.hpp"
+#include "ice3_sedim.hpp"
 
 namespace ice3 {
 
@@ -63,27 +63,13 @@ __global__ void __launch_bounds__(64) k_adjust_sedim(AdjustArgs aa, SedimArgs a)
   adjust_sedim_column<double>(aa, a, i);
 }
 
-template <class R, bool ZZZ = false>
-__global__ void __launch_bounds__(256) k_sedim(SedimArgs a) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.ncol) return;
-  sedim_column<R, ZZZ>(a, i);
-}
-
 // ---- hail (KRR=7), FP64: ICE_ADJUST with the hail heat capacity (one thread per point),
-// the sedimentation with hail (one thread per column), the two in one column walk for the
-// fused step; the microphysics is k_micro<double, false, true> (k_micro_points<double, false,
+// and that and the sedimentation with hail in one column walk for the fused step; the microphysics is k_micro<double, false, true> (k_micro_points<double, false,
 // true> when the context sets another sub-step cap).
 __global__ void __launch_bounds__(256) k_ice_adjust_hail(AdjustArgs a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.ncol) return;
   adjust_at<false, true>(a, i, (size_t)blockIdx.y * a.ld + i);
-}
-
-__global__ void __launch_bounds__(256) k_sedim_hail(SedimArgs a) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.ncol) return;
-  sedim_column<double, false, true>(a, i);
 }
 
 __global__ void __launch_bounds__(64) k_adjust_sedim_hail(AdjustArgs aa, SedimArgs a) {
@@ -1210,6 +1196,27 @@ extern "C" int ice3_ice_adjust_ocnd2(ice3_ctx *ctx, int ncol, int nlev, int ld, 
   return ICE3_OK;
 }
 
+// ICE_ADJUST and the statistical sedimentation of the FP64 fused step; aa.rh (with sa.src_rh)
+// selects hail.  One column walk when there are enough columns to hide its latency: a lone
+// wavefront takes 6 us a level, so that 1,024 to 65,536 columns of 90 levels all take 0.53 to
+// 0.60 ms, against 0.08 to 0.44 ms for ICE_ADJUST point by point followed by k_sedim.  From
+// SEDIM_WALK_COLS (1.7 wavefronts per SIMD) on the walk saves more traffic than it waits: at
+// 98,304 columns 0.76 against 0.64 ms, at 114,688 0.78 against 0.75 (hail: 0.93 against 0.96),
+// at 131,072 0.81 against 0.85, at 262,144 1.51 against 1.72.
+static hipError_t launch_adjust_sedim(const ice3_ctx *ctx, const AdjustArgs &aa, const SedimArgs &sa,
+                                      hipStream_t s) {
+  const dim3 gw((aa.ncol + 63) / 64), gp((aa.ncol + 255) / 256, aa.nlev);
+  if (aa.ncol >= SEDIM_WALK_COLS * ctx->ncu) {
+    if (aa.rh) hipLaunchKernelGGL(k_adjust_sedim_hail, gw, dim3(64), 0, s, aa, sa);
+    else hipLaunchKernelGGL(k_adjust_sedim, gw, dim3(64), 0, s, aa, sa);
+    return hipGetLastError();
+  }
+  if (aa.rh) hipLaunchKernelGGL(k_ice_adjust_hail, gp, dim3(256), 0, s, aa);
+  else hipLaunchKernelGGL(k_ice_adjust, gp, dim3(256), 0, s, aa);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : sedim_launch<double>(sa, ctx->ncu, s);
+}
+
 // Launch k_micro: one workgroup of eight wavefronts per compute unit (its LDS holds the
 // tables and the parked points, so one workgroup fits a CU).
 static hipError_t launch_micro(const ice3_ctx *ctx, int prec, const MicroArgs &m, hipStream_t s) {
@@ -1307,11 +1314,9 @@ static int launch_split_keep(ice3_ctx *ctx, int nlev, int ld, const SedimArgs &s
 static int launch_rain_ice(ice3_ctx *ctx, int prec, const SedimArgs &sa, const MicroArgs &ma,
                            void *stream) {
   hipStream_t s = (hipStream_t)stream;
-  const dim3 gs((sa.ncol + 255) / 256);
   if (ctx->sedim == ICE3_SEDIM_SPLI) HIPCHK(launch_split(ctx, sa, ma, s));
-  else if (prec == ICE3_PREC_FP64) hipLaunchKernelGGL(k_sedim<double>, gs, dim3(256), 0, s, sa);
-  else hipLaunchKernelGGL(k_sedim<float>, gs, dim3(256), 0, s, sa);
-  HIPCHK(hipGetLastError());
+  else if (prec == ICE3_PREC_FP64) HIPCHK(sedim_launch<double>(sa, ctx->ncu, s));
+  else HIPCHK(sedim_launch<float>(sa, ctx->ncu, s));
   MARK(2);
   HIPCHK(launch_micro(ctx, prec, ma, s));
   MARK(3); MARK(4); MARK(5); MARK(6);
@@ -1369,8 +1374,7 @@ extern "C" int ice3_rain_ice_ocnd2(ice3_ctx *ctx, int ncol, int nlev, int ld, do
   if (ctx->sedim == ICE3_SEDIM_SPLI)
     HIPCHK(launch_split(ctx, sa, m, s));
   else
-    hipLaunchKernelGGL((k_sedim<double, true>), dim3((ncol + 255) / 256), dim3(256), 0, s, sa);
-  HIPCHK(hipGetLastError());
+    HIPCHK(sedim_launch<double>(sa, ctx->ncu, s));
   MARK(2);
   HIPCHK(launch_micro_ocnd2(ctx, m, s));
   MARK(3); MARK(4); MARK(5); MARK(6);
@@ -1412,15 +1416,14 @@ extern "C" int ice3_adjust_rain_ice_stages(ice3_ctx *ctx, int prec, int ncol, in
   pipeline_args(ncol, nlev, ld, dt, ctx->d_tab, in, out, stats, aa, sa, m);
   m.max_calls = ctx->max_calls; m.capped = ctx->d_capped;
   hipStream_t s = (hipStream_t)stream;
-  const dim3 gs((ncol + 255) / 256), gp((ncol + 255) / 256, nlev);
+  const dim3 gp((ncol + 255) / 256, nlev);
   const bool split = ctx->sedim == ICE3_SEDIM_SPLI;
   MARK(0);
   if (prec == ICE3_PREC_FP64 && !split && (stages & ICE3_STAGE_ADJUST) &&
       (stages & ICE3_STAGE_SEDIMENTATION)) {
     // one column walk for both stages (in the mixed path the float sedimentation is cheap
     // and the two kernels are faster apart)
-    hipLaunchKernelGGL(k_adjust_sedim, dim3((ncol + 63) / 64), dim3(64), 0, s, aa, sa);
-    HIPCHK(hipGetLastError());
+    HIPCHK(launch_adjust_sedim(ctx, aa, sa, s));
     stages &= ~ICE3_STAGE_SEDIMENTATION;
   } else if (stages & ICE3_STAGE_ADJUST) {
     hipLaunchKernelGGL(k_ice_adjust, gp, dim3(256), 0, s, aa);
@@ -1433,9 +1436,11 @@ extern "C" int ice3_adjust_rain_ice_stages(ice3_ctx *ctx, int prec, int ncol, in
       if (rc != ICE3_OK) return rc;
     } else if (split) {
       HIPCHK(launch_split(ctx, sa, m, s));
-    } else if (prec == ICE3_PREC_FP64) hipLaunchKernelGGL(k_sedim<double>, gs, dim3(256), 0, s, sa);
-    else hipLaunchKernelGGL(k_sedim<float>, gs, dim3(256), 0, s, sa);
-    HIPCHK(hipGetLastError());
+    } else if (prec == ICE3_PREC_FP64) {
+      HIPCHK(sedim_launch<double>(sa, ctx->ncu, s));
+    } else {
+      HIPCHK(sedim_launch<float>(sa, ctx->ncu, s));
+    }
   }
   MARK(2);
   if (stages & ICE3_STAGE_MICROPHYSICS) {
@@ -1485,9 +1490,8 @@ extern "C" int ice3_adjust_rain_ice_ocnd2(ice3_ctx *ctx, int ncol, int nlev, int
     const int rc = launch_split_keep(ctx, nlev, ld, sa, m, s);
     if (rc != ICE3_OK) return rc;
   } else {
-    hipLaunchKernelGGL((k_sedim<double, true>), dim3((ncol + 255) / 256), dim3(256), 0, s, sa);
+    HIPCHK(sedim_launch<double>(sa, ctx->ncu, s));
   }
-  HIPCHK(hipGetLastError());
   MARK(2);
   HIPCHK(launch_micro_ocnd2(ctx, m, s));
   MARK(3); MARK(4); MARK(5); MARK(6);
@@ -1587,11 +1591,8 @@ extern "C" int ice3_rain_ice_branches(ice3_ctx *ctx, int ncol, int nlev, int ld,
   hipStream_t s = (hipStream_t)stream;
   if (ctx->sedim == ICE3_SEDIM_SPLI)
     HIPCHK(launch_split(ctx, sa, m, s));
-  else if (hail)
-    hipLaunchKernelGGL(k_sedim_hail, dim3((ncol + 255) / 256), dim3(256), 0, s, sa);
   else
-    hipLaunchKernelGGL(k_sedim<double>, dim3((ncol + 255) / 256), dim3(256), 0, s, sa);
-  HIPCHK(hipGetLastError());
+    HIPCHK(sedim_launch<double>(sa, ctx->ncu, s));
   const unsigned int npts = (unsigned int)nlev * (unsigned int)ncol;
   if (hail)
     hipLaunchKernelGGL(k_micro_branches<true>, dim3((npts + 255) / 256), dim3(256), 0, s, m);
@@ -1628,8 +1629,7 @@ extern "C" int ice3_rain_ice_hail(ice3_ctx *ctx, int ncol, int nlev, int ld, dou
   if (ctx->sedim == ICE3_SEDIM_SPLI)
     HIPCHK(launch_split(ctx, sa, m, s));
   else
-    hipLaunchKernelGGL(k_sedim_hail, dim3((ncol + 255) / 256), dim3(256), 0, s, sa);
-  HIPCHK(hipGetLastError());
+    HIPCHK(sedim_launch<double>(sa, ctx->ncu, s));
   MARK(2);
   HIPCHK(launch_micro_hail(ctx, m, s));
   MARK(3); MARK(4); MARK(5); MARK(6);
@@ -1664,8 +1664,7 @@ extern "C" int ice3_adjust_rain_ice_hail(ice3_ctx *ctx, int ncol, int nlev, int 
     const int rc = launch_split_keep(ctx, nlev, ld, sa, m, s);
     if (rc != ICE3_OK) return rc;
   } else {
-    hipLaunchKernelGGL(k_adjust_sedim_hail, dim3((ncol + 63) / 64), dim3(64), 0, s, aa, sa);
-    HIPCHK(hipGetLastError());
+    HIPCHK(launch_adjust_sedim(ctx, aa, sa, s));
     MARK(1);
   }
   MARK(2);
@@ -1740,8 +1739,7 @@ static int surrogate_step(ice3_ctx *ctx, int ncol, int nlev, int ld, double dt,
   const unsigned int ntiles = (npts + MLP_TILE - 1) / MLP_TILE;
   const unsigned int nblk = ntiles < (unsigned int)ncu ? ntiles : (unsigned int)ncu;
   MARK(0);
-  hipLaunchKernelGGL(k_adjust_sedim, dim3((ncol + 63) / 64), dim3(64), 0, s, aa, sa);
-  HIPCHK(hipGetLastError());
+  HIPCHK(launch_adjust_sedim(ctx, aa, sa, s));
   MARK(1);
   MARK(2);
   hipLaunchKernelGGL(k_sg_features, dim3((npts + 255) / 256), dim3(256), 0, s, g);

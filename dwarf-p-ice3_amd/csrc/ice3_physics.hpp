@@ -36,6 +36,20 @@ enum { ITH = 0, IRV = 1, IRC = 2, IRR = 3, IRI = 4, IRS = 5, IRG = 6, IRH = 7 };
 // built with -fapprox-func, under which the device divides by a reciprocal refined with
 // Newton steps (within 1 ulp; in practice the IEEE quotient).
 
+// One Horner step p z + c of the two polynomials.  With ICE3_SCALAR_COEF (a source that is
+// bound by the VALU issue rate defines it) the coefficient is a scalar operand of one
+// v_fma_f64; the compiler's own choice moves it into two vector registers first.  The same
+// fused operation either way.
+__host__ __device__ __forceinline__ double horner(double p, double z, double c) {
+#if defined(__HIP_DEVICE_COMPILE__) && defined(ICE3_SCALAR_COEF)
+  double r;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(p), "v"(z), "s"(c));
+  return r;
+#else
+  return fma(p, z, c);
+#endif
+}
+
 // log x: x = 2^e m with m in [sqrt(1/2), sqrt(2)); log m = 2 atanh(s) = 2s + s z p(z),
 // s = (m - 1)/(m + 1), z = s^2 <= 0.0295; p is a degree-6 near-minimax fit of
 // (log m - 2s)/(s z) on that interval (interpolation at Chebyshev nodes in 60-digit
@@ -55,12 +69,12 @@ __host__ __device__ __forceinline__ double log_f64(double x) {
   const double s = f / (2.0 + f);
   const double z = s * s;
   double p = 0x1.2b5900de53b32p-3;
-  p = fma(p, z, 0x1.39fe51a7c18f9p-3);
-  p = fma(p, z, 0x1.7462b51cb66b1p-3);
-  p = fma(p, z, 0x1.c71c62e3f11e6p-3);
-  p = fma(p, z, 0x1.2492492df281ap-2);
-  p = fma(p, z, 0x1.99999999952d7p-2);
-  p = fma(p, z, 0x1.5555555555558p-1);
+  p = horner(p, z, 0x1.39fe51a7c18f9p-3);
+  p = horner(p, z, 0x1.7462b51cb66b1p-3);
+  p = horner(p, z, 0x1.c71c62e3f11e6p-3);
+  p = horner(p, z, 0x1.2492492df281ap-2);
+  p = horner(p, z, 0x1.99999999952d7p-2);
+  p = horner(p, z, 0x1.5555555555558p-1);
   const double r = fma(s * z, p, s + s);  // log m
   const double de = (double)e;
   const double y = fma(de, LN2_HI, fma(de, LN2_LO, r));
@@ -81,17 +95,17 @@ __host__ __device__ __forceinline__ double exp_f64(double x) {
   double r = fma(-n, LN2_HI, xc);  // exact: n LN2_HI is exact and close to xc
   r = fma(-n, LN2_LO, r);
   double p = 0x1.af236857dc4b7p-26;
-  p = fma(p, r, 0x1.28803f36ecdd5p-22);
-  p = fma(p, r, 0x1.71de17e4e5d5dp-19);
-  p = fma(p, r, 0x1.a019c9a6c2942p-16);
-  p = fma(p, r, 0x1.a01a01a4b2f7fp-13);
-  p = fma(p, r, 0x1.6c16c1738faf6p-10);
-  p = fma(p, r, 0x1.1111111110e6ap-7);
-  p = fma(p, r, 0x1.5555555554cb7p-5);
-  p = fma(p, r, 0x1.5555555555555p-3);
-  p = fma(p, r, 0.5);
-  p = fma(p, r, 1.0);
-  p = fma(p, r, 1.0);
+  p = horner(p, r, 0x1.28803f36ecdd5p-22);
+  p = horner(p, r, 0x1.71de17e4e5d5dp-19);
+  p = horner(p, r, 0x1.a019c9a6c2942p-16);
+  p = horner(p, r, 0x1.a01a01a4b2f7fp-13);
+  p = horner(p, r, 0x1.6c16c1738faf6p-10);
+  p = horner(p, r, 0x1.1111111110e6ap-7);
+  p = horner(p, r, 0x1.5555555554cb7p-5);
+  p = horner(p, r, 0x1.5555555555555p-3);
+  p = horner(p, r, 0.5);
+  p = horner(p, r, 1.0);
+  p = horner(p, r, 1.0);
   const double y = ldexp(p, (int)n);
   return x == x ? y : x;  // NaN stays NaN
 }
@@ -1341,48 +1355,70 @@ __device__ __forceinline__ int stepping_point(double dt, double exn, double rhod
   return st < 0 ? -calls : calls;
 }
 
-// Fall speed of one species at one level, OTHER_SPECIES / PRISTINE_ICE
+// Fall speed law of one species, OTHER_SPECIES / PRISTINE_ICE
 // (micro/mode_ice4_sedimentation_stat.F90:295-431); jrr = 3 (r), 4 (i), 5 (s), 6 (g),
-// 7 (h, :184-188).  lnrho = ln(rhodref) of the level; the powers are evaluated as exp(c*ln x).
-template <class R>
-__device__ __forceinline__ R fall_speed(int jrr, double rx, R lnrho) {
-  if (jrr == 4) {
-    if (!(rx > dmax(P.XRTMIN[4], 1.0E-7))) return (R)0;
-    const R lnrx = rlog<R>((R)rx);
-    return (R)P.XFSEDI * rexp<R>(-(R)P.XCEXVT * lnrho) *
-           rexp<R>((R)P.XEXCSEDI *
-                   rlog<R>(dmax((R)0.05E6, (R)-0.15319E6 - (R)0.021454E6 * (lnrho + lnrx))));
-  }
-  if (!(rx > P.XRTMIN[jrr])) return (R)0;
+// 7 (h, :184-188).  A literal jrr folds to constants; a wavefront-uniform one (k_sedim) is a
+// set of scalars.
+template <class R> struct FallLaw {
+  bool ice;
+  double thr;        // no fall at or below this mixing ratio
+  R fsed, exr, exrho;  // fsed r^exr rho^exrho (the power-law species)
+};
+template <class R> __device__ __forceinline__ FallLaw<R> fall_law(int jrr) {
+  if (jrr == 4) return {true, dmax(P.XRTMIN[4], 1.0E-7), (R)0, (R)0, (R)0};
   const double fsed = jrr == 3 ? P.XFSEDR : (jrr == 5 ? P.XFSEDS : (jrr == 6 ? P.XFSEDG : P.XFSEDH));
   const double exsed = jrr == 3 ? P.XEXSEDR : (jrr == 5 ? P.XEXSEDS : (jrr == 6 ? P.XEXSEDG : P.XEXSEDH));
-  return (R)fsed * rexp<R>((R)(exsed - 1) * rlog<R>((R)rx) + (R)(exsed - P.XCEXVT - 1) * lnrho);
+  return {false, P.XRTMIN[jrr], (R)fsed, (R)(exsed - 1), (R)(exsed - P.XCEXVT - 1)};
 }
 
-// One species at one level of ICE4_SEDIMENTATION_STAT (:143-229) for one column:
-// flux holds the flux leaving the level above on entry and this level's on exit
-// (double); rs is the species' source, updated by the flux divergence.
-// jrr = 3 (r), 4 (i), 5 (s), 6 (g), 7 (h); the species are independent, so the
-// reference's species-outer loop order and this level-outer order agree.
+// Fall speed at mixing ratio rx > law.thr; lnrho = ln(rhodref) of the level; the powers are
+// evaluated as exp(c*ln x).  rhoc (read for pristine ice only) is rho^-XCEXVT.
 template <class R>
-__device__ __forceinline__ void sediment_species(int jrr, double dt, double rho, R lnrho, double dz,
+__device__ __forceinline__ R fall_speed_above(const FallLaw<R> &law, double rx, R lnrho, R rhoc) {
+  const R lnrx = rlog<R>((R)rx);
+  if (law.ice)
+    return (R)P.XFSEDI * rhoc *
+           rexp<R>((R)P.XEXCSEDI *
+                   rlog<R>(dmax((R)0.05E6, (R)-0.15319E6 - (R)0.021454E6 * (lnrho + lnrx))));
+  return law.fsed * rexp<R>(law.exr * lnrx + law.exrho * lnrho);
+}
+template <class R> __device__ __forceinline__ R fall_rhoc(R lnrho) { return rexp<R>(-(R)P.XCEXVT * lnrho); }
+
+// The flux a level's own content sends down (w1 the fall speed of rx = rs * dt).
+__device__ __forceinline__ double sediment_own(double zinv, double rho, double dz, double rx, double w1) {
+  return dmin(rho * dz * rx * zinv, w1 * rho * rx);
+}
+
+// The rest of one level of ICE4_SEDIMENTATION_STAT (:143-229): the part of the flux from
+// above that goes through the level, added to f1; rs is the species' source, updated by the
+// flux divergence; flux holds the flux leaving the level above on entry, this level's on exit.
+template <class R>
+__device__ __forceinline__ void sediment_through(const FallLaw<R> &law, double dt, double zinv, R lnrho,
+                                                 R rhoc, double dz, double tsorhodz, double f1,
                                                  double &rs, double &flux) {
-  const double zinv = 1. / dt;
-  const double tsorhodz = dt / (rho * dz);
-  const double rx = rs * dt;
   const double qp = flux * tsorhodz;
-  const double thr = P.XRTMIN[jrr];
-  double cur;
-  if (rx > thr || qp > thr) {
-    const double w1 = (double)fall_speed<R>(jrr, rx, lnrho);
-    const double w2 = (double)fall_speed<R>(jrr, qp, lnrho);
-    const double f1 = dmin(rho * dz * rx * zinv, w1 * rho * rx);
-    cur = w2 != 0. ? f1 + dmax(0., 1. - dz / (dt * w2)) * flux : f1;
-  } else {
-    cur = dmin(rho * dz * rx * zinv, 0. * rho * rx);
+  double cur = f1;
+  if (qp > law.thr) {
+    const double w2 = (double)fall_speed_above<R>(law, qp, lnrho, rhoc);
+    if (w2 != 0.) cur = f1 + dmax(0., 1. - dz / (dt * w2)) * flux;
   }
   rs = rs + tsorhodz * (flux - cur) * zinv;
   flux = cur;
+}
+
+// One species at one level of ICE4_SEDIMENTATION_STAT (:143-229) for one column (flux as
+// above, double).  The species are independent, so the reference's species-outer loop order
+// and a level-outer order agree.
+template <class R>
+__device__ __forceinline__ void sediment_species(int jrr, double dt, double rho, R lnrho, double dz,
+                                                 double &rs, double &flux) {
+  const FallLaw<R> law = fall_law<R>(jrr);
+  const double zinv = 1. / dt;
+  const double rx = rs * dt;
+  const R rhoc = law.ice ? fall_rhoc<R>(lnrho) : (R)0;
+  const double w1 = rx > law.thr ? (double)fall_speed_above<R>(law, rx, lnrho, rhoc) : 0.;
+  sediment_through<R>(law, dt, zinv, lnrho, rhoc, dz, dt / (rho * dz),
+                      sediment_own(zinv, rho, dz, rx, w1), rs, flux);
 }
 
 }  // namespace ice3

@@ -11,7 +11,7 @@ CSRC = os.path.join(PKG, "csrc")
 OUT = os.path.join(HERE, "_lib", "libice3_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ("ice3_kernels.hip", "ice3_mlp.hip", "ice3_params.cpp")
+SOURCES = ("ice3_kernels.hip", "ice3_sedim.hip", "ice3_mlp.hip", "ice3_params.cpp")
 # -ffp-contract=off keeps FP64 a*b+c as two roundings, the sequence of the CPU reference.
 # Packed FP32 instructions (v_pk_*_f32) are disabled for the device code: some of their
 # forms have given wrong results on this hardware without any error.
@@ -25,7 +25,9 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
 # SIMD (each polynomial step of a log became a dependent scratch reload); rebuilding the
 # constants at their uses is cheaper (k_micro<double>: 256 VGPRs + 104 B/lane of spills ->
 # 216 VGPRs, none; -10 %).  The matrix-core kernels (ice3_mlp.hip) keep it: their hoisted
-# LDS addresses pay.
+# LDS addresses pay.  So does the sedimentation (ice3_sedim.hip), whose hoisted constants are
+# scalars; it takes the default scheduler (iterative-ilp: the same times, and the register
+# allocator has failed on it).
 # The iterative ILP scheduler, for both: the kernels run at a fixed two (k_micro), four
 # (k_adjust_sedim) or one (k_mlp_infer) wavefronts per SIMD and hide latency mostly within
 # a wavefront (k_micro -7 %, k_mlp_infer -5 %; results bit for bit the same).
@@ -38,6 +40,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
 ILP = ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]
 SOURCE_FLAGS = {"ice3_kernels.hip": ["-mllvm", "-disable-machine-licm", "-Xarch_device", "-fapprox-func",
                                      *ILP],
+                "ice3_sedim.hip": ["-Xarch_device", "-fapprox-func"],
                 "ice3_mlp.hip": ILP}
 
 
