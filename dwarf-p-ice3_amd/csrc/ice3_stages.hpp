@@ -37,9 +37,10 @@ struct Ocnd2Args {
 // adjusted ris.  With OCND2 the branch's extra fields come from x: the layer thickness is
 // ZDZ(k) = PZZ(kp) - PZZ(kp-1), kp = min(k+1, nlev-1) (condensation.F90:366,376-378).
 // HAIL (KRR=7): a.rh enters the heat capacity.
+// c0 is the offset of the column's lowest level, a.ld the step to the next one.
 template <bool OCND2 = false, bool HAIL = false>
-__device__ __forceinline__ double adjust_at(const AdjustArgs &a, int i, size_t j, int k = 0,
-                                            const Ocnd2Args *x = nullptr, unsigned *br = nullptr) {
+__device__ __forceinline__ double adjust_at(const AdjustArgs &a, int i, size_t j, int k,
+                                            const Ocnd2Args *x, unsigned *br, size_t c0) {
   const ice3_ice_adjust_in &in = a.in;
   double rvs = in.rvs[j], rcs = in.rcs[j], ris = in.ris[j], ths = in.ths[j];
   AdjustOut o;
@@ -49,7 +50,7 @@ __device__ __forceinline__ double adjust_at(const AdjustArgs &a, int i, size_t j
     const double *zz = x->in.zz;
     xp.tiwmx = x->tiwmx;
     xp.z = zz[j];
-    xp.dz = zz[(size_t)kp * a.ld + i] - zz[(size_t)(kp - 1) * a.ld + i];
+    xp.dz = zz[(size_t)kp * a.ld + c0] - zz[(size_t)(kp - 1) * a.ld + c0];
     xp.cld_wgt = x->in.ice_cld_wgt[i];
     xp.bottom = k == 0;
   }
@@ -84,6 +85,13 @@ __device__ __forceinline__ double adjust_at(const AdjustArgs &a, int i, size_t j
   if (out.srcs) out.srcs[j] = o.srcs;
   if (a.ris_copy) a.ris_copy[j] = ris;
   return ris;
+}
+
+// Fields (nlev, ld): the lowest level of column i at offset i.
+template <bool OCND2 = false, bool HAIL = false>
+__device__ __forceinline__ double adjust_at(const AdjustArgs &a, int i, size_t j, int k = 0,
+                                            const Ocnd2Args *x = nullptr, unsigned *br = nullptr) {
+  return adjust_at<OCND2, HAIL>(a, i, j, k, x, br, (size_t)i);
 }
 
 // Sedimentation stage arguments.  src_* are the sources entering RAIN_ICE,

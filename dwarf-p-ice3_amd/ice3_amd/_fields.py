@@ -24,6 +24,26 @@ def as_columns(x, layout: str, *, device, name: str) -> torch.Tensor:
     return t.reshape(-1, t.shape[-1]).t().contiguous()
 
 
+def in_rows(fields: dict) -> bool:
+    """Whether "jax" layout fields (device float64 tensors) are better taken as (ncol, nlev) rows,
+    the vertical contiguous, than as (nlev, ncol) columns: True unless more of them already have
+    the columns' memory order (results of a columns call are such views)."""
+    score = 0
+    for t in fields.values():
+        if t.is_contiguous():
+            score += 1
+        elif t.dim() >= 2 and t.movedim(-1, 0).is_contiguous():
+            score -= 1
+    return score >= 0
+
+
+def as_rows(t: torch.Tensor, name: str) -> torch.Tensor:
+    """A "jax" layout device tensor as contiguous (ncol, nlev) rows (no copy when it is)."""
+    if t.dim() < 2:
+        raise ValueError(f"{name}: expected a (..., nz) array, got {tuple(t.shape)}")
+    return t.reshape(-1, t.shape[-1]).contiguous()
+
+
 def from_columns(t: torch.Tensor, layout: str, shape) -> torch.Tensor:
     """Inverse of as_columns for results: a (nlev, ncol) field back to ``shape``, or a
     per-column (ncol,) result to ``shape[:-1]`` (the JAX layout without its vertical axis)."""

@@ -80,7 +80,7 @@ class Surrogate(ctypes.Structure):
 
 EXPORTS = ("ice3_ctx_create", "ice3_ctx_destroy", "ice3_strerror", "ice3_dump_constants",
            "ice3_ctx_set_substep_cap", "ice3_ctx_status", "ice3_ctx_set_sedimentation",
-           "ice3_ice_adjust", "ice3_ice_adjust_ocnd2", "ice3_rain_ice", "ice3_adjust_rain_ice",
+           "ice3_ice_adjust", "ice3_ice_adjust_rows", "ice3_ice_adjust_ocnd2", "ice3_rain_ice", "ice3_adjust_rain_ice",
            "ice3_rain_ice_ocnd2", "ice3_adjust_rain_ice_ocnd2",
            "ice3_ice_adjust_hail", "ice3_rain_ice_hail", "ice3_adjust_rain_ice_hail",
            "ice3_rain_ice_branches", "ice3_ice_adjust_branches",
@@ -118,6 +118,9 @@ def load():
         lib.ice3_ice_adjust.argtypes = common + [ctypes.POINTER(AdjustIn), ctypes.POINTER(AdjustOut), _P]
         lib.ice3_ice_adjust_ocnd2.argtypes = [
             _P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_double, ctypes.POINTER(AdjustIn),
+            ctypes.POINTER(Ocnd2In), ctypes.POINTER(AdjustOut), ctypes.POINTER(Ocnd2Out), _P]
+        lib.ice3_ice_adjust_rows.argtypes = [
+            _P, ctypes.c_int, ctypes.c_int, ctypes.c_double, ctypes.POINTER(AdjustIn), _P,
             ctypes.POINTER(Ocnd2In), ctypes.POINTER(AdjustOut), ctypes.POINTER(Ocnd2Out), _P]
         lib.ice3_rain_ice.argtypes = common + [ctypes.POINTER(RainIn), ctypes.POINTER(RainIO),
                                                ctypes.POINTER(RainOut), ctypes.POINTER(Stats), _P]

@@ -20,7 +20,7 @@ import ctypes
 import torch
 
 from . import _lib
-from ._fields import as_columns, check_layout, from_columns, ptr, resolve_layout, stream_ptr
+from ._fields import as_columns, as_rows, check_layout, from_columns, in_rows, ptr, resolve_layout, stream_ptr
 
 _PREC = {"fp64": _lib.PREC_FP64, "mixed": _lib.PREC_MIXED}
 _OUT_ORDER = ("t", "rv_out", "rc_out", "ri_out", "cldfr", "hlc_hrc", "hlc_hcf", "hli_hri",
@@ -110,14 +110,35 @@ class IceAdjust:
         self._ctx = _lib.context(self.device.index)
 
     def _inputs(self, sigqsat, args, layout):
-        """Columns-layout device tensors of the fields and the per-column sigqsat."""
-        f = {k: as_columns(v, layout, device=self.device, name=k) for k, v in args.items()}
-        nlev, ncol = f["th"].shape
+        """Device tensors of the fields, the per-column sigqsat, the domain and whether the fields
+        are (ncol, nlev) rows ("jax" arrays as they are) instead of (nlev, ncol) columns."""
+        rows = False
+        if layout == "jax":
+            args = {k: torch.as_tensor(v, dtype=torch.float64, device=self.device) for k, v in args.items()}
+            rows = in_rows(args)
+        if rows:
+            f = {k: as_rows(v, k) for k, v in args.items()}
+            ncol, nlev = f["th"].shape
+        else:
+            f = {k: as_columns(v, layout, device=self.device, name=k) for k, v in args.items()}
+            nlev, ncol = f["th"].shape
         for k, v in f.items():
-            if tuple(v.shape) != (nlev, ncol):
-                raise ValueError(f"{k}: shape {tuple(v.shape)} != {(nlev, ncol)}")
+            have = tuple(v.shape[::-1]) if rows else tuple(v.shape)
+            if have != (nlev, ncol):
+                raise ValueError(f"{k}: shape {have} != {(nlev, ncol)}")
         sq = self._per_column(sigqsat, "sigqsat", ncol, layout)
-        return f, sq, nlev, ncol
+        return f, sq, nlev, ncol, rows
+
+    def _check_finite(self, f, per_column, nlev, ncol):
+        """require_finite counts per field, so rows may be read as if they were columns."""
+        _lib.require_finite({**{k: v.view(nlev, ncol) for k, v in f.items()}, **per_column}, self.device)
+
+    def _results(self, out, names, layout, rows, shape):
+        return tuple(out[k].reshape(shape) if rows else from_columns(out[k], layout, shape) for k in names)
+
+    def _outputs(self, names, nlev, ncol, rows):
+        shape = (ncol, nlev) if rows else (nlev, ncol)
+        return {k: torch.empty(shape, dtype=torch.float64, device=self.device) for k in names}
 
     def _per_column(self, x, name, ncol, layout):
         t = torch.as_tensor(x, dtype=torch.float64, device=self.device)
@@ -136,22 +157,24 @@ class IceAdjust:
                     rvs=rvs, rcs=rcs, ris=ris, ths=ths)
         shape = tuple(th.shape) if hasattr(th, "shape") else tuple(torch.as_tensor(th).shape)
         layout = resolve_layout(self.layout, th)
-        f, sq, nlev, ncol = self._inputs(sigqsat, args, layout)
+        f, sq, nlev, ncol, rows = self._inputs(sigqsat, args, layout)
         if check_inputs:
-            _lib.require_finite({**f, "sigqsat": sq}, self.device)
-        out = {k: torch.empty((nlev, ncol), dtype=torch.float64, device=self.device) for k in _OUT_ORDER}
-        srcs = torch.empty((nlev, ncol), dtype=torch.float64, device=self.device) if return_srcs else None
+            self._check_finite(f, {"sigqsat": sq}, nlev, ncol)
+        names = _OUT_ORDER + (("srcs",) if return_srcs else ())
+        out = self._outputs(names, nlev, ncol, rows)
         cin = _lib.AdjustIn(*[ptr(f[k]) for k in _lib.ADJ_IN_FIELDS[:-1]], ptr(sq))
-        cout = _lib.AdjustOut(*[ptr(out[k]) for k in _lib.ADJ_OUT_FIELDS[:-1]], ptr(srcs))
+        cout = _lib.AdjustOut(*[ptr(out[k]) for k in _lib.ADJ_OUT_FIELDS[:-1]], ptr(out.get("srcs")))
         with torch.cuda.device(self.device):
-            rc_ = self._lib.ice3_ice_adjust(self._ctx, _PREC[precision], ncol, nlev, ncol, float(timestep),
-                                            ctypes.byref(cin), ctypes.byref(cout), stream_ptr(self.device))
+            prec = _PREC[precision]
+            if rows:
+                rc_ = self._lib.ice3_ice_adjust_rows(self._ctx, ncol, nlev, float(timestep), ctypes.byref(cin),
+                                                     None, None, ctypes.byref(cout), None,
+                                                     stream_ptr(self.device))
+            else:
+                rc_ = self._lib.ice3_ice_adjust(self._ctx, prec, ncol, nlev, ncol, float(timestep),
+                                                ctypes.byref(cin), ctypes.byref(cout), stream_ptr(self.device))
         _lib.check(rc_, "ice3_ice_adjust")
-        res = [out[k] for k in _OUT_ORDER]
-        res = [from_columns(r, layout, shape) for r in res]
-        if srcs is not None:
-            srcs = from_columns(srcs, layout, shape)
-        return (*res, srcs) if return_srcs else tuple(res)
+        return self._results(out, names, layout, rows, shape)
 
 
 class IceAdjustOCND2(IceAdjust):
@@ -179,28 +202,29 @@ class IceAdjustOCND2(IceAdjust):
                     rvs=rvs, rcs=rcs, ris=ris, ths=ths, zz=zz)
         shape = tuple(th.shape) if hasattr(th, "shape") else tuple(torch.as_tensor(th).shape)
         layout = resolve_layout(self.layout, th)
-        f, sq, nlev, ncol = self._inputs(sigqsat, args, layout)
+        f, sq, nlev, ncol, rows = self._inputs(sigqsat, args, layout)
         wgt = self._per_column(ice_cld_wgt, "ice_cld_wgt", ncol, layout)
         if nlev == 1:
             raise ValueError("the OCND2 branch needs at least two levels")
         if check_inputs:
-            _lib.require_finite({**f, "sigqsat": sq, "ice_cld_wgt": wgt}, self.device)
-        names = _OUT_ORDER + _lib.OCND2_OUT_FIELDS
-        out = {k: torch.empty((nlev, ncol), dtype=torch.float64, device=self.device) for k in names}
-        srcs = torch.empty((nlev, ncol), dtype=torch.float64, device=self.device) if return_srcs else None
+            self._check_finite(f, {"sigqsat": sq, "ice_cld_wgt": wgt}, nlev, ncol)
+        names = _OUT_ORDER + _lib.OCND2_OUT_FIELDS + (("srcs",) if return_srcs else ())
+        out = self._outputs(names, nlev, ncol, rows)
         cin = _lib.AdjustIn(*[ptr(f[k]) for k in _lib.ADJ_IN_FIELDS[:-1]], ptr(sq))
         cin2 = _lib.Ocnd2In(ptr(f["zz"]), ptr(wgt))
-        cout = _lib.AdjustOut(*[ptr(out[k]) for k in _lib.ADJ_OUT_FIELDS[:-1]], ptr(srcs))
+        cout = _lib.AdjustOut(*[ptr(out[k]) for k in _lib.ADJ_OUT_FIELDS[:-1]], ptr(out.get("srcs")))
         cout2 = _lib.Ocnd2Out(*[ptr(out[k]) for k in _lib.OCND2_OUT_FIELDS])
         with torch.cuda.device(self.device):
-            rc_ = self._lib.ice3_ice_adjust_ocnd2(self._ctx, ncol, nlev, ncol, float(timestep),
-                                                  ctypes.byref(cin), ctypes.byref(cin2), ctypes.byref(cout),
-                                                  ctypes.byref(cout2), stream_ptr(self.device))
+            if rows:
+                rc_ = self._lib.ice3_ice_adjust_rows(self._ctx, ncol, nlev, float(timestep), ctypes.byref(cin),
+                                                     None, ctypes.byref(cin2), ctypes.byref(cout),
+                                                     ctypes.byref(cout2), stream_ptr(self.device))
+            else:
+                rc_ = self._lib.ice3_ice_adjust_ocnd2(self._ctx, ncol, nlev, ncol, float(timestep),
+                                                      ctypes.byref(cin), ctypes.byref(cin2), ctypes.byref(cout),
+                                                      ctypes.byref(cout2), stream_ptr(self.device))
         _lib.check(rc_, "ice3_ice_adjust_ocnd2")
-        res = [from_columns(out[k], layout, shape) for k in names]
-        if srcs is not None:
-            srcs = from_columns(srcs, layout, shape)
-        return (*res, srcs) if return_srcs else tuple(res)
+        return self._results(out, names, layout, rows, shape)
 
 
 class IceAdjustHail(IceAdjust):
@@ -220,19 +244,21 @@ class IceAdjustHail(IceAdjust):
                     rvs=rvs, rcs=rcs, ris=ris, ths=ths, rh=rh)
         shape = tuple(th.shape) if hasattr(th, "shape") else tuple(torch.as_tensor(th).shape)
         layout = resolve_layout(self.layout, th)
-        f, sq, nlev, ncol = self._inputs(sigqsat, args, layout)
+        f, sq, nlev, ncol, rows = self._inputs(sigqsat, args, layout)
         if check_inputs:
-            _lib.require_finite({**f, "sigqsat": sq}, self.device)
-        out = {k: torch.empty((nlev, ncol), dtype=torch.float64, device=self.device) for k in _OUT_ORDER}
-        srcs = torch.empty((nlev, ncol), dtype=torch.float64, device=self.device) if return_srcs else None
+            self._check_finite(f, {"sigqsat": sq}, nlev, ncol)
+        names = _OUT_ORDER + (("srcs",) if return_srcs else ())
+        out = self._outputs(names, nlev, ncol, rows)
         cin = _lib.AdjustIn(*[ptr(f[k]) for k in _lib.ADJ_IN_FIELDS[:-1]], ptr(sq))
-        cout = _lib.AdjustOut(*[ptr(out[k]) for k in _lib.ADJ_OUT_FIELDS[:-1]], ptr(srcs))
+        cout = _lib.AdjustOut(*[ptr(out[k]) for k in _lib.ADJ_OUT_FIELDS[:-1]], ptr(out.get("srcs")))
         with torch.cuda.device(self.device):
-            rc_ = self._lib.ice3_ice_adjust_hail(self._ctx, ncol, nlev, ncol, float(timestep),
-                                                 ctypes.byref(cin), ptr(f["rh"]), ctypes.byref(cout),
-                                                 stream_ptr(self.device))
+            if rows:
+                rc_ = self._lib.ice3_ice_adjust_rows(self._ctx, ncol, nlev, float(timestep), ctypes.byref(cin),
+                                                     ptr(f["rh"]), None, ctypes.byref(cout), None,
+                                                     stream_ptr(self.device))
+            else:
+                rc_ = self._lib.ice3_ice_adjust_hail(self._ctx, ncol, nlev, ncol, float(timestep),
+                                                     ctypes.byref(cin), ptr(f["rh"]), ctypes.byref(cout),
+                                                     stream_ptr(self.device))
         _lib.check(rc_, "ice3_ice_adjust_hail")
-        res = [from_columns(out[k], layout, shape) for k in _OUT_ORDER]
-        if srcs is not None:
-            srcs = from_columns(srcs, layout, shape)
-        return (*res, srcs) if return_srcs else tuple(res)
+        return self._results(out, names, layout, rows, shape)

@@ -154,6 +154,15 @@ int ice3_ice_adjust_ocnd2(ice3_ctx *ctx, int ncol, int nlev, int ld, double dt,
                           const ice3_ice_adjust_out *out, const ice3_ocnd2_out *out2,
                           void *stream);
 
+/* ICE_ADJUST of fields (ncol, nlev) with the vertical contiguous, element (column i, level k) at
+ * p[i*nlev + k]: the JAX components' (nx, ny, nz) arrays as they are (the stage is pointwise).
+ * FP64 in both precisions.  rh (or NULL): the hail mixing ratio, as ice3_ice_adjust_hail; in2
+ * and out2 (both or neither): as ice3_ice_adjust_ocnd2, not with rh. */
+int ice3_ice_adjust_rows(ice3_ctx *ctx, int ncol, int nlev, double dt,
+                         const ice3_ice_adjust_in *in, const double *rh,
+                         const ice3_ocnd2_in *in2, const ice3_ice_adjust_out *out,
+                         const ice3_ocnd2_out *out2, void *stream);
+
 /* ---- rain_ice: RAIN_ICE (micro/rain_ice.F90:7) with statistical sedimentation,
  *      total tendencies and negativity correction ---- */
 typedef struct {
