@@ -5,6 +5,8 @@ import ctypes
 
 import torch
 
+from . import _lib
+
 
 def as_columns(x, layout: str, *, device, name: str) -> torch.Tensor:
     """Return a contiguous float64 CUDA tensor of shape (nlev, ncol).
@@ -22,6 +24,59 @@ def as_columns(x, layout: str, *, device, name: str) -> torch.Tensor:
     if t.dim() < 2:
         raise ValueError(f"{name}: expected a (..., nz) array, got {tuple(t.shape)}")
     return t.reshape(-1, t.shape[-1]).t().contiguous()
+
+
+def columns_of(fields: dict, layout: str, *, device):
+    """as_columns of every field of a call, and the names of those that are fresh copies (the
+    others share the caller's memory).  "jax" fields whose memory is (..., nz) in order are
+    transposed together, one launch for each shape among them."""
+    out, fresh, batches = {}, set(), {}
+    f64 = torch.float64
+    for k, x in fields.items():
+        if type(x) is torch.Tensor and x.dtype is f64 and x.device == device:
+            t = x
+            if layout == "columns" and x.dim() == 2 and x.is_contiguous():
+                out[k] = x
+                continue
+        else:
+            t = torch.as_tensor(x, dtype=f64, device=device)
+        if layout == "jax" and t.dim() >= 2 and t.is_contiguous() and t.device.type == "cuda":
+            v = t.reshape(-1, t.shape[-1])
+            if not v.t().is_contiguous() and max(v.shape) < 2 ** 31:
+                batches.setdefault(tuple(v.shape), []).append((k, v))
+                out[k] = None  # keeps the order of the names
+                continue
+        out[k] = as_columns(t, layout, device=device, name=k)
+        if out[k].data_ptr() != t.data_ptr():
+            fresh.add(k)
+    for (rows, cols), items in batches.items():
+        for i in range(0, len(items), _lib.ICE3_MAX_CHECK_FIELDS):
+            part = items[i:i + _lib.ICE3_MAX_CHECK_FIELDS]
+            new = [torch.empty((cols, rows), dtype=torch.float64, device=device) for _ in part]
+            arr = ctypes.c_void_p * len(part)
+            with torch.cuda.device(device):
+                _lib.check(_lib.load().ice3_transpose_fields(
+                    len(part), arr(*[v.data_ptr() for _, v in part]), arr(*[n.data_ptr() for n in new]), rows, cols,
+                    stream_ptr(device)), "ice3_transpose_fields")
+            for (k, _), n in zip(part, new):
+                out[k] = n
+                fresh.add(k)
+    return out, fresh
+
+
+def column_shape(x, layout: str, name: str) -> tuple:
+    """The (nlev, ncol) shape as_columns(x) would have, without making it."""
+    shape = tuple(x.shape) if hasattr(x, "shape") else tuple(torch.as_tensor(x).shape)
+    if layout == "columns":
+        if len(shape) != 2:
+            raise ValueError(f"{name}: expected a (nlev, ncol) array, got {shape}")
+        return shape
+    if len(shape) < 2:
+        raise ValueError(f"{name}: expected a (..., nz) array, got {shape}")
+    n = 1
+    for d in shape[:-1]:
+        n *= d
+    return shape[-1], n
 
 
 def in_rows(fields: dict) -> bool:

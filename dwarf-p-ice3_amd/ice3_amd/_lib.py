@@ -60,6 +60,7 @@ Hail = _struct("ice3_hail", HAIL_FIELDS)
 PipeHail = _struct("ice3_pipeline_hail", PIPE_HAIL_FIELDS)
 
 STAGE_ADJUST, STAGE_SEDIMENTATION, STAGE_MICROPHYSICS = 1, 2, 4
+RainSrc = _struct("ice3_rain_ice_src", RAIN_IO_FIELDS + ("rhs",))
 SEDIM = {"STAT": 0, "SPLI": 1}   # ICE3_SEDIM_STAT, ICE3_SEDIM_SPLI
 NFEAT, NTARG = 18, 8
 
@@ -81,7 +82,7 @@ class Surrogate(ctypes.Structure):
 EXPORTS = ("ice3_ctx_create", "ice3_ctx_destroy", "ice3_strerror", "ice3_dump_constants",
            "ice3_ctx_set_substep_cap", "ice3_ctx_status", "ice3_ctx_set_sedimentation",
            "ice3_ice_adjust", "ice3_ice_adjust_rows", "ice3_ice_adjust_ocnd2", "ice3_rain_ice", "ice3_adjust_rain_ice",
-           "ice3_rain_ice_ocnd2", "ice3_adjust_rain_ice_ocnd2",
+           "ice3_rain_ice_ocnd2", "ice3_adjust_rain_ice_ocnd2", "ice3_rain_ice_from", "ice3_transpose_fields",
            "ice3_ice_adjust_hail", "ice3_rain_ice_hail", "ice3_adjust_rain_ice_hail",
            "ice3_rain_ice_branches", "ice3_ice_adjust_branches",
            "ice3_stage_timing",
@@ -124,6 +125,11 @@ def load():
             ctypes.POINTER(Ocnd2In), ctypes.POINTER(AdjustOut), ctypes.POINTER(Ocnd2Out), _P]
         lib.ice3_rain_ice.argtypes = common + [ctypes.POINTER(RainIn), ctypes.POINTER(RainIO),
                                                ctypes.POINTER(RainOut), ctypes.POINTER(Stats), _P]
+        lib.ice3_rain_ice_from.argtypes = common + [
+            ctypes.POINTER(RainIn), ctypes.POINTER(RainOcnd2In), ctypes.POINTER(RainSrc), ctypes.POINTER(RainIO),
+            ctypes.POINTER(RainOut), ctypes.POINTER(Hail), ctypes.POINTER(Stats), _P]
+        lib.ice3_transpose_fields.argtypes = [ctypes.c_int, ctypes.POINTER(_P), ctypes.POINTER(_P), ctypes.c_int,
+                                              ctypes.c_int, _P]
         lib.ice3_adjust_rain_ice.argtypes = common + [ctypes.POINTER(PipeIn), ctypes.POINTER(PipeOut),
                                                       ctypes.POINTER(Stats), _P]
         c5 = [_P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_double]

@@ -43,7 +43,8 @@ import ctypes
 import torch
 
 from . import _lib
-from ._fields import as_columns, check_layout, from_columns, ptr, resolve_layout, stream_ptr
+from ._fields import (as_columns, check_layout, column_shape, columns_of, from_columns, ptr, resolve_layout,
+                      stream_ptr)
 from .ice_adjust import check_configuration, sedimentation_of
 
 _PREC = {"fp64": _lib.PREC_FP64, "mixed": _lib.PREC_MIXED}
@@ -106,17 +107,26 @@ class RainIce(_Base):
     """RAIN_ICE on MI355X (see module docstring)."""
 
     _ENTRY = "ice3_rain_ice"
+    # argument of the C ABI -> state key: what the kernels read, what they read if the state
+    # has it, and what the interface takes without reading
+    _READ = dict(exn="exn", dzz="dzz", rhodref="rhodref", pabs="pres", tht="th_t", rvt="rv_t", rct="rc_t",
+                 rrt="rr_t", rit="ri_t", rst="rs_t", rgt="rg_t", ths="ths", rvs="rvs", rcs="rcs", rrs="rrs",
+                 ris="ris", rss="rss", rgs="rgs", ci="ci_t")
+    _READ_OPTIONAL = dict(exn_ref="exnref", cldfr="cf", sigs="sigs")
+    _UNREAD = dict(rhodj="rhodj", hlc_hrc="hlc_hrc", hlc_hcf="hlc_hcf", hli_hri="hli_hri", hli_hcf="hli_hcf")
+    _EXTRA = {}  # of the OCND2 and hail variants
 
-    def _extra_inputs(self, state, layout, nlev, ncol):
-        return {}
+    def _extra_arrays(self, extra, fresh, nlev, ncol):
+        return extra
 
     def _extra_results(self, extra, new, diags, layout, shape):
         pass
 
-    def _launch(self, precision, ncol, nlev, dt, cin, extra, cio, cout, st):
-        return self._lib.ice3_rain_ice(self._ctx, _PREC[precision], ncol, nlev, ncol, float(dt),
-                                       ctypes.byref(cin), ctypes.byref(cio), ctypes.byref(cout),
-                                       ctypes.byref(st), stream_ptr(self.device))
+    def _launch(self, precision, ncol, nlev, dt, cin, csrc, extra, cio, cout, st, in2=None, hail=None):
+        return self._lib.ice3_rain_ice_from(self._ctx, _PREC[precision], ncol, nlev, ncol, float(dt),
+                                            ctypes.byref(cin), in2 and ctypes.byref(in2), ctypes.byref(csrc),
+                                            ctypes.byref(cio), ctypes.byref(cout), hail and ctypes.byref(hail),
+                                            ctypes.byref(st), stream_ptr(self.device))
 
     def __call__(self, state: dict, dt: float, lsedim_after: bool = False, ldeposc: bool = False,
                  ldsoft: bool = False, lfeedbackt: bool = True, max_iterations: int | None = None,
@@ -125,38 +135,44 @@ class RainIce(_Base):
             raise ValueError("only LSEDIM_AFTER=F, LDEPOSC=F, LFEEDBACKT=T are implemented")
         shape = self._shape(state["th_t"])
         layout = resolve_layout(self.layout, state["th_t"])
-        g = lambda k: self._col(state[k], k, layout)  # noqa: E731
-        th = g("th_t")
-        nlev, ncol = th.shape
-        z = torch.zeros((nlev, ncol), dtype=torch.float64, device=self.device)
-        opt = lambda k, d: self._col(state[k], k, layout) if k in state else d  # noqa: E731
-        exn = g("exn")
-        rhodref = g("rhodref")
-        inp = dict(exn=exn, dzz=g("dzz"), rhodj=opt("rhodj", rhodref), rhodref=rhodref,
-                   exn_ref=opt("exnref", exn), pabs=g("pres"), cldfr=opt("cf", z),
-                   hlc_hrc=opt("hlc_hrc", z), hlc_hcf=opt("hlc_hcf", z), hli_hri=opt("hli_hri", z),
-                   hli_hcf=opt("hli_hcf", z), sigs=opt("sigs", z), tht=th, rvt=g("rv_t"), rct=g("rc_t"),
-                   rrt=g("rr_t"), rit=g("ri_t"), rst=g("rs_t"), rgt=g("rg_t"))
-        # sources and ci are updated in place on private copies
-        io = {k: g(k).clone() for k in ("ths", "rvs", "rcs", "rrs", "ris", "rss", "rgs")}
-        io["ci"] = g("ci_t").clone()
+        read = {**self._READ, **{k: v for k, v in self._READ_OPTIONAL.items() if v in state}}
+        if check_inputs:
+            read.update({k: v for k, v in self._UNREAD.items() if v in state})
+        read.update(self._EXTRA)
+        f, fresh = columns_of({v: state[v] for v in read.values()}, layout, device=self.device)
+        f = {k: f[v] for k, v in read.items()}
+        fresh = {k for k, v in read.items() if v in fresh}
+        nlev, ncol = f["tht"].shape
+        for k, v in self._UNREAD.items():  # taken for the interface: the kernels read none of them
+            if v in state and k not in f and column_shape(state[v], layout, v) != (nlev, ncol):
+                raise ValueError(f"{k}: shape {column_shape(state[v], layout, v)} != {(nlev, ncol)}")
+        for k, v in f.items():
+            if tuple(v.shape) != (nlev, ncol):
+                raise ValueError(f"{k}: shape {tuple(v.shape)} != {(nlev, ncol)}")
+        extra = {k: f.pop(k) for k in self._EXTRA}
+        f.setdefault("exn_ref", f["exn"])
+        if "cldfr" not in f or "sigs" not in f:
+            z = torch.zeros((nlev, ncol), dtype=torch.float64, device=self.device)
+            f.setdefault("cldfr", z)
+            f.setdefault("sigs", z)
+        inp = {k: f.get(k, f["rhodref"]) for k in _lib.RAIN_IN_FIELDS}
+        src = {k: f[k] for k in _lib.RAIN_IO_FIELDS}
+        # the sources and ci are updated in the copies made above, or apart from the caller's arrays
+        io = {k: v if k in fresh else torch.empty_like(v) for k, v in src.items()}
         out = {k: torch.empty((nlev, ncol), dtype=torch.float64, device=self.device) for k in ("evap3d", "rainfr")}
         out.update({k: torch.empty(ncol, dtype=torch.float64, device=self.device)
                     for k in ("inprc", "inprr", "inpri", "inprs", "inprg")})
-        for k, v in list(inp.items()) + list(io.items()):
-            if tuple(v.shape) != (nlev, ncol):
-                raise ValueError(f"{k}: shape {tuple(v.shape)} != {(nlev, ncol)}")
         if check_inputs:
-            _lib.require_finite({**inp, **io}, self.device)
-        extra = self._extra_inputs(state, layout, nlev, ncol)
-        if check_inputs:
+            _lib.require_finite(f, self.device)
             _lib.require_finite(extra, self.device)
+        extra = self._extra_arrays(extra, fresh, nlev, ncol)
         counters, calls, st = self._stats(nlev * ncol, return_calls)
         cin = _lib.RainIn(*[ptr(inp[k]) for k in _lib.RAIN_IN_FIELDS])
+        csrc = _lib.RainSrc(*[ptr(src[k]) for k in _lib.RAIN_IO_FIELDS], ptr(extra.get("rhs")))
         cio = _lib.RainIO(*[ptr(io[k]) for k in _lib.RAIN_IO_FIELDS])
         cout = _lib.RainOut(*[ptr(out[k]) for k in _lib.RAIN_OUT_FIELDS])
         with torch.cuda.device(self.device), self._scheme():
-            rc = self._launch(precision, ncol, nlev, dt, cin, extra, cio, cout, st)
+            rc = self._launch(precision, ncol, nlev, dt, cin, csrc, extra, cio, cout, st)
         _lib.check(rc, self._ENTRY)
         self._finish_counters(counters)
         new = dict(state)
@@ -187,21 +203,23 @@ class AdjustRainIce(_Base):
     def _fused(self, f, dt, precision, return_calls, check_inputs, ocnd2=False, hail=False):
         shape = self._shape(f["th"])
         layout = resolve_layout(self.layout, f["th"])
-        g = {k: self._col(f[k], k, layout) for k in _lib.PIPE_IN_FIELDS if k != "sigqsat"}
+        names = [k for k in _lib.PIPE_IN_FIELDS if k not in ("rhodj", "sigqsat")]
+        more = (["zz"] if ocnd2 else []) + (["rh", "rhs"] if hail else [])
+        # rhodj: taken for the interface, read by no kernel
+        g, _ = columns_of({k: f[k] for k in names + more + (["rhodj"] if check_inputs else [])}, layout,
+                          device=self.device)
         nlev, ncol = g["th"].shape
         sq = self._per_column(f["sigqsat"], "sigqsat", ncol, layout)
-        extra = {}
         if ocnd2:
-            extra["zz"] = self._col(f["zz"], "zz", layout)
             wgt = self._per_column(f["ice_cld_wgt"], "ice_cld_wgt", ncol, layout)
             if nlev < 2:
                 raise ValueError("the OCND2 branch needs at least two levels")
-        if hail:
-            extra["rh"] = self._col(f["rh"], "rh", layout)
-            extra["rhs"] = self._col(f["rhs"], "rhs", layout)
-        for k, v in list(g.items()) + list(extra.items()):
-            if tuple(v.shape) != (nlev, ncol):
-                raise ValueError(f"{k}: shape {tuple(v.shape)} != {(nlev, ncol)}")
+        for k, v in {**{k: tuple(v.shape) for k, v in g.items()},
+                     "rhodj": column_shape(f["rhodj"], layout, "rhodj")}.items():
+            if v != (nlev, ncol):
+                raise ValueError(f"{k}: shape {v} != {(nlev, ncol)}")
+        g.setdefault("rhodj", g["rhodref"])
+        extra = {k: g.pop(k) for k in more}
         if check_inputs:
             _lib.require_finite({**g, **extra, "sigqsat": sq, **({"ice_cld_wgt": wgt} if ocnd2 else {})},
                                 self.device)
@@ -272,20 +290,13 @@ class RainIceOCND2(RainIce):
         super().__init__({}, layout, device, sedimentation or sedim,
                          cfl if split_max_cfl is None else split_max_cfl)
 
-    def _extra_inputs(self, state, layout, nlev, ncol):
-        x = {k: self._col(state[k], k, layout) for k in _lib.RAIN_OCND2_IN_FIELDS}
-        for k, v in x.items():
-            if tuple(v.shape) != (nlev, ncol):
-                raise ValueError(f"{k}: shape {tuple(v.shape)} != {(nlev, ncol)}")
-        return x
+    _EXTRA = {k: k for k in _lib.RAIN_OCND2_IN_FIELDS}
 
-    def _launch(self, precision, ncol, nlev, dt, cin, extra, cio, cout, st):
+    def _launch(self, precision, ncol, nlev, dt, cin, csrc, extra, cio, cout, st):
         if precision != "fp64":
             raise ValueError("the OCND2 branch is implemented in FP64 only")
-        cin2 = _lib.RainOcnd2In(*[ptr(extra[k]) for k in _lib.RAIN_OCND2_IN_FIELDS])
-        return self._lib.ice3_rain_ice_ocnd2(self._ctx, ncol, nlev, ncol, float(dt), ctypes.byref(cin),
-                                             ctypes.byref(cin2), ctypes.byref(cio), ctypes.byref(cout),
-                                             ctypes.byref(st), stream_ptr(self.device))
+        return super()._launch(precision, ncol, nlev, dt, cin, csrc, extra, cio, cout, st,
+                               in2=_lib.RainOcnd2In(*[ptr(extra[k]) for k in _lib.RAIN_OCND2_IN_FIELDS]))
 
 
 class AdjustRainIceOCND2(AdjustRainIce):
@@ -318,25 +329,21 @@ class RainIceHail(RainIce):
 
     _ENTRY = "ice3_rain_ice_hail"
 
-    def _extra_inputs(self, state, layout, nlev, ncol):
-        x = {"rht": self._col(state["rh_t"], "rh_t", layout),
-             "rhs": self._col(state["rhs"], "rhs", layout).clone()}
-        for k in ("rht", "rhs"):
-            if tuple(x[k].shape) != (nlev, ncol):
-                raise ValueError(f"{k}: shape {tuple(x[k].shape)} != {(nlev, ncol)}")
-        return x
+    _EXTRA = {"rht": "rh_t", "rhs": "rhs"}
 
-    def _launch(self, precision, ncol, nlev, dt, cin, extra, cio, cout, st):
+    def _extra_arrays(self, extra, fresh, nlev, ncol):
+        extra["rhs_out"] = extra["rhs"] if "rhs" in fresh else torch.empty_like(extra["rhs"])
+        extra["inprh"] = torch.empty(ncol, dtype=torch.float64, device=self.device)
+        return extra
+
+    def _launch(self, precision, ncol, nlev, dt, cin, csrc, extra, cio, cout, st):
         if precision != "fp64":
             raise ValueError("the hail path is implemented in FP64 only")
-        extra["inprh"] = torch.empty(ncol, dtype=torch.float64, device=self.device)
-        h = _lib.Hail(ptr(extra["rht"]), ptr(extra["rhs"]), ptr(extra["inprh"]))
-        return self._lib.ice3_rain_ice_hail(self._ctx, ncol, nlev, ncol, float(dt), ctypes.byref(cin),
-                                            ctypes.byref(cio), ctypes.byref(cout), ctypes.byref(h),
-                                            ctypes.byref(st), stream_ptr(self.device))
+        return super()._launch(precision, ncol, nlev, dt, cin, csrc, extra, cio, cout, st,
+                               hail=_lib.Hail(ptr(extra["rht"]), ptr(extra["rhs_out"]), ptr(extra["inprh"])))
 
     def _extra_results(self, extra, new, diags, layout, shape):
-        new["rhs"] = from_columns(extra["rhs"], layout, shape)
+        new["rhs"] = from_columns(extra["rhs_out"], layout, shape)
         diags["inprh"] = from_columns(extra["inprh"], layout, shape)
 
 

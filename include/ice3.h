@@ -112,6 +112,13 @@ long ice3_dump_constants(const ice3_ctx *ctx, char *buf, long buflen);
 int ice3_count_nonfinite(int nfield, const double *const *fields, const int *rows, int ncol,
                          int ld, unsigned long long *counts, void *stream);
 
+/* nfield (at most ICE3_MAX_CHECK_FIELDS) float64 device arrays (rows, cols), contiguous, written
+ * transposed: dst[q][c*rows + r] = src[q][r*cols + c].  One launch; src and dst are host arrays
+ * of device pointers, and no dst overlaps a src.  The Python drop-ins bring (..., nz) fields to
+ * the (nlev, ncol) layout with it. */
+int ice3_transpose_fields(int nfield, const double *const *src, double *const *dst, int rows,
+                          int cols, void *stream);
+
 /* ---- ice_adjust: ICE_ADJUST (micro/ice_adjust.F90:7) with CONDENSATION ---- */
 typedef struct {
   const double *pabs, *sigs, *th, *exn, *exn_ref, *rho_dry_ref;
@@ -232,6 +239,21 @@ int ice3_ice_adjust_hail(ice3_ctx *ctx, int ncol, int nlev, int ld, double dt,
 /* RAIN_ICE with KRR=7: as ice3_rain_ice, plus the hail arrays. */
 int ice3_rain_ice_hail(ice3_ctx *ctx, int ncol, int nlev, int ld, double dt,
                        const ice3_rain_ice_in *in, const ice3_rain_ice_inout *io,
+                       const ice3_rain_ice_out *out, const ice3_hail *hail,
+                       const ice3_stats *stats, void *stream);
+
+/* RAIN_ICE with the sources read from src and written to io (and hail->rhs): ice3_rain_ice
+ * without the copies that a caller who keeps the sources at entry would make.  Any array of src
+ * may be the one io (hail) writes.  in2 (or NULL): as ice3_rain_ice_ocnd2; hail (or NULL): as
+ * ice3_rain_ice_hail, its source read from src->rhs; not both, and in FP64. */
+typedef struct {
+  const double *ths, *rvs, *rcs, *rrs, *ris, *rss, *rgs, *ci;
+  const double *rhs;    /* with hail; else NULL */
+} ice3_rain_ice_src;
+
+int ice3_rain_ice_from(ice3_ctx *ctx, int prec, int ncol, int nlev, int ld, double dt,
+                       const ice3_rain_ice_in *in, const ice3_rain_ocnd2_in *in2,
+                       const ice3_rain_ice_src *src, const ice3_rain_ice_inout *io,
                        const ice3_rain_ice_out *out, const ice3_hail *hail,
                        const ice3_stats *stats, void *stream);
 

@@ -84,3 +84,58 @@ def test_ice_adjust_orders_bitwise(kind, shape):
     bad["rc"][0, 0, 0] = float("nan")
     with pytest.raises(ValueError, match=r"rc \(1\)"):
         call(sq, *[bad[k] for k in ARGS], timestep=DT, check_inputs=True, **{k: bad[k] for k in extra})
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [(2, 2), (31, 5), (32, 128), (33, 129), (1000, 90), (65, 300), (300, 2)])
+def test_transposing_launch(rows, cols):
+    """Every field of a call in one launch: tile edges, more than one column tile, a field that needs no
+    transposing among them."""
+    from ice3_amd._fields import columns_of
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    t = {f"f{q}": torch.rand((rows, cols), dtype=torch.float64, device="cuda").reshape(1, rows, cols) for q in range(3)}
+    t["view"] = _column_view(t["f0"])
+    out, fresh = columns_of(t, "jax", device=torch.device("cuda", 0))
+    assert list(out) == list(t) and fresh == {"f0", "f1", "f2"}
+    for k, v in out.items():
+        assert v.is_contiguous() and torch.equal(v, t[k].reshape(rows, cols).t()), k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sedimentation", ["STAT", "SPLI"])
+@pytest.mark.parametrize("kind", ["plain", "hail", "ocnd2"])
+def test_rain_ice_orders_bitwise(kind, sedimentation):
+    """RainIce in every order of its state, against the columns call; the caller's arrays stay as they were."""
+    from ice3_amd import RainIce, RainIceHail, RainIceOCND2, synthetic
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    shape = (5, 13, 40)
+    f = synthetic.generate(65, 40, seed=20260330, variant="pipeline")
+    names = dict(exn="exn", exnref="exn_ref", rhodref="rho_dry_ref", rhodj="rhodj", pres="pabs", dzz="dzz",
+                 th_t="th", rv_t="rv", rc_t="rc", rr_t="rr", ri_t="ri", rs_t="rs", rg_t="rg", ci_t="ci", sigs="sigs")
+    names.update({k: k for k in ("ths", "rvs", "rcs", "rrs", "ris", "rss", "rgs")})
+    cols = {k: f[v] for k, v in names.items()}
+    cols["cf"] = (f["rc"] > 0) * 0.5
+    if kind == "hail":
+        cols["rh_t"], cols["rhs"] = f["rg"] * 0.7, f["rg"] * 0.7 / DT
+    if kind == "ocnd2":
+        rng = np.random.Generator(np.random.Philox(5))
+        cols.update(icldfr=rng.uniform(0, 1, f["th"].shape), ssio=rng.uniform(0, 0.2, f["th"].shape),
+                    ssiu=rng.uniform(-0.2, 0, f["th"].shape), ifr=np.full(f["th"].shape, 10.0))
+    cols = {k: torch.from_numpy(np.ascontiguousarray(v)).cuda() for k, v in cols.items()}
+    call = {"plain": RainIce, "hail": RainIceHail, "ocnd2": RainIceOCND2}[kind](sedimentation=sedimentation)
+    rows = lambda k, v: v.t().contiguous().reshape(shape)  # noqa: E731
+    view = lambda k, v: v.t().reshape(shape)  # noqa: E731
+    ref, ref_d = call(cols, DT)
+    keys = ["ths", "rvs", "rcs", "rrs", "ris", "rss", "rgs", "ci_t", "evap3d", "rainfr"] + ["rhs"] * (kind == "hail")
+    orders = {"rows": rows, "columns": view, "mixed": lambda k, v: (view if k in ("ths", "rv_t", "ci_t") else rows)(k, v)}
+    for name, to in orders.items():
+        state = {k: to(k, v.clone()) for k, v in cols.items()}
+        new, diags = call(state, DT)
+        for k in keys:
+            assert new[k].shape == shape and torch.equal(new[k].reshape(65, 40).t(), ref[k]), (name, k)
+        for k in ref_d:
+            assert torch.equal(diags[k].reshape(-1), ref_d[k]), (name, k)
+        for k, v in state.items():
+            assert torch.equal(v.reshape(65, 40).t(), cols[k]), (name, k)
