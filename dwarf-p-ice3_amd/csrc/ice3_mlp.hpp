@@ -92,6 +92,56 @@ __device__ __forceinline__ void mlp_layer(const __bf16 *sIn, int row0, const bf1
   }
 }
 
+// ---- Activations in registers.  With the weights as the first matrix operand and the
+// activations as the second (the packed W fragments are the A fragments of W^T), a product of a
+// layer leaves lane l with units 4*(l/16) .. +3 of point l % 16 of each 16-unit tile; rounded to
+// bf16 that is two dwords, and the next layer's operand wants units 8*(l/16) .. +7 of the same
+// point of each 32-unit block.  Two lane swaps a dword pair bring the one to the other, so the
+// activations of a wavefront never leave its registers.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ u32x2 pack4(float a, float b, float c, float d) {
+  return u32x2{__builtin_bit_cast(unsigned int, bf16x2{(__bf16)a, (__bf16)b}),
+               __builtin_bit_cast(unsigned int, bf16x2{(__bf16)c, (__bf16)d})};
+}
+
+// The operand fragment of 32 units from its two 16-unit tiles: rows r0..r3 (16 lanes each) of t0
+// hold units 0-3, 4-7, 8-11, 12-15, of t1 16-19 .. 28-31; the halves swap gives (t0 r0 r1, t1 r0 r1)
+// and (t0 r2 r3, t1 r2 r3), the rows swap units 8r .. 8r+3 and 8r+4 .. 8r+7 in row r.  Every lane
+// of the wavefront must be active.
+__device__ __forceinline__ bf16x8 operand_of(const u32x2 &t0, const u32x2 &t1) {
+  u32x4 f;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const auto h = __builtin_amdgcn_permlane32_swap(t0[q], t1[q], false, false);
+    const auto r = __builtin_amdgcn_permlane16_swap(h[0], h[1], false, false);
+    f[q] = r[0];
+    f[2 + q] = r[1];
+  }
+  return __builtin_bit_cast(bf16x8, f);
+}
+
+// acc[mt][nn]: 16 units (tile nn) x 16 points (tile mt) of W^T X, W as packed fragments in LDS (NT
+// unit tiles wide, the first N / 16 of them taken), X as operand fragments.
+template <int K, int N, int NT, int MT>
+__device__ __forceinline__ void mlp_product(const bf16x8 *sWpk, const bf16x8 (&x)[MT][K / 32],
+                                            f32x4 (&acc)[MT][N / 16], int lane) {
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nn = 0; nn < N / 16; ++nn) acc[mt][nn] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kk = 0; kk < K / 32; ++kk)
+#pragma unroll
+    for (int nn = 0; nn < N / 16; ++nn) {
+      const bf16x8 w = sWpk[(kk * NT + nn) * 64 + lane];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[mt][nn] = mfma_bf16(w, x[mt][kk], acc[mt][nn]);
+    }
+}
+
 // Copy n elements global -> LDS with the whole workgroup (16-byte granules).
 __device__ __forceinline__ void block_copy16(void *dst, const void *src, int bytes) {
   const int4 *s = (const int4 *)src;

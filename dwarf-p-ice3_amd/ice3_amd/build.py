@@ -28,9 +28,10 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
 # LDS addresses pay.  So does the sedimentation (ice3_sedim.hip), whose hoisted constants are
 # scalars; it takes the default scheduler (iterative-ilp: the same times, and the register
 # allocator has failed on it).
-# The iterative ILP scheduler, for both: the kernels run at a fixed two (k_micro), four
-# (k_adjust_sedim) or one (k_mlp_infer) wavefronts per SIMD and hide latency mostly within
-# a wavefront (k_micro -7 %, k_mlp_infer -5 %; results bit for bit the same).
+# The iterative ILP scheduler for the physics kernels: they run at a fixed two (k_micro) or four
+# (k_adjust_sedim) wavefronts per SIMD and hide latency mostly within a wavefront (k_micro
+# -7 %; results bit for bit the same).  k_mlp_infer, bound by the VALU, is faster with the
+# default one (4.27 against 4.46 ms at 512x512x90).
 # -fapprox-func for the physics kernels' device code: divisions become a reciprocal and
 # Newton steps (FP64: two steps and a residual correction, within 1 ulp and in practice
 # correctly rounded; FP32: the hardware reciprocal, 1 ulp) instead of the scaled IEEE
@@ -41,7 +42,7 @@ ILP = ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]
 SOURCE_FLAGS = {"ice3_kernels.hip": ["-mllvm", "-disable-machine-licm", "-Xarch_device", "-fapprox-func",
                                      *ILP],
                 "ice3_sedim.hip": ["-Xarch_device", "-fapprox-func"],
-                "ice3_mlp.hip": ILP}
+                "ice3_mlp.hip": []}
 
 
 def build(verbose: bool = False) -> str:
