@@ -321,7 +321,7 @@ __device__ __forceinline__ double split_species(const SplitArgs &a, int lane, co
                                                 const double (&dz)[L], const double (&oorhodz)[L],
                                                 double (&r)[L], double (&s)[L], bool *capped) {
   constexpr double thr = JRR == 4 ? (P.XRTMIN[4] > 1.0E-7 ? P.XRTMIN[4] : 1.0E-7) : P.XRTMIN[JRR];
-  const double dt = a.dt, zinv = 1. / dt;
+  const double dt = a.dt, zinv = 1. / by(dt);
   bool any = false;
 #pragma unroll
   for (int q = 0; q < L; ++q) any = any || (lane + 64 * q < a.nlev && r[q] > thr);
@@ -349,11 +349,11 @@ __device__ __forceinline__ double split_species(const SplitArgs &a, int lane, co
       const bool in = lane + 64 * q < a.nlev;
       w[q] = in && r[q] > thr ? split_flux<JRR>(r[q], rho[q], rf[q]) : 0.;
       if (in && r[q] > P.XRTMIN[JRR] && w[q] > 1.E-20)
-        m = dmin(m, a.maxcfl * rho[q] * r[q] * dz[q] / w[q]);  // :795-808
+        m = dmin(m, a.maxcfl * rho[q] * r[q] * dz[q] / by(w[q]));  // :795-808
     }
     const double step = dmin(remaint, wave_min(m));
     remaint = remaint - step;  // :814-815
-    inpr = inpr + lane0_f64(w[0]) / P.XRHOLW * (step * zinv);
+    inpr = inpr + lane0_f64(w[0]) / by(P.XRHOLW) * (step * zinv);
 #pragma unroll
     for (int q = 0; q < L; ++q) {  // :820-824; level k + 1 is the next lane (or slot)
       const double next = q + 1 < L ? lane0_f64(w[q + 1 < L ? q + 1 : q]) : 0.;
@@ -442,7 +442,7 @@ __global__ void __launch_bounds__(64 * SPLIT_COLS)
   double oorhodz[L];
 #pragma unroll
   for (int q = 0; q < L; ++q)
-    oorhodz[q] = lane + 64 * q < a.nlev ? 1. / (rho[q] * dz[q]) : 0.;  // ZW (:263)
+    oorhodz[q] = lane + 64 * q < a.nlev ? 1. / by(rho[q] * dz[q]) : 0.;  // ZW (:263)
   if (i < a.ncol) {
     bool capped = false;
     const double pr = split_species<L, 3>(a, lane, rho, dz, oorhodz, r[0], src[IRR], &capped);

@@ -26,6 +26,37 @@ namespace ice3 {
 
 enum { ITH = 0, IRV = 1, IRC = 2, IRR = 3, IRI = 4, IRS = 5, IRG = 6, IRH = 7 };
 
+// ---------------------------------------------------------------- FP64 division
+// a / by(b).  On the device: the hardware reciprocal (relative error under 4.7e-8), one Newton
+// step, and the residual correction of the quotient, which squares the reciprocal's remaining
+// error (2e-15): the IEEE quotient but for operands within 1e-29 of a rounding boundary (equal to
+// it on 6.3e9 random pairs over 2^+-300).  Two fused operations fewer than the compiler's own
+// -fapprox-func sequence, which takes a second Newton step; and a divisor shared by several
+// quotients is one reciprocal wherever they stand.  A zero, infinite or NaN divisor gives NaN, as
+// the compiler's sequence does.  Divisions are a quarter of k_micro's VALU time: with this form
+// k_micro takes 2.85 ms at 512x512x90 instead of 2.95, results bit for bit the same.
+template <class T> struct By {
+  T b, r;
+};
+__host__ __device__ __forceinline__ By<double> by(double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double r = __builtin_amdgcn_rcp(b);
+  return {b, fma(fma(-b, r, 1.0), r, r)};
+#else
+  return {b, 0.};
+#endif
+}
+__host__ __device__ __forceinline__ double operator/(double a, const By<double> &d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double q = a * d.r;
+  return fma(fma(-d.b, q, a), d.r, q);
+#else
+  return a / d.b;
+#endif
+}
+__host__ __device__ __forceinline__ By<float> by(float b) { return {b, 0.f}; }
+__host__ __device__ __forceinline__ float operator/(float a, const By<float> &d) { return a / d.b; }
+
 // ---------------------------------------------------------------- FP64 exp and log
 // The physics evaluates about ten FP64 logarithms and as many exponentials per point and
 // sedimentation level, and more in a hard tendency call.  The library versions keep
@@ -66,7 +97,7 @@ __host__ __device__ __forceinline__ double log_f64(double x) {
     e = e - 1;
   }
   const double f = m - 1.0;  // exact
-  const double s = f / (2.0 + f);
+  const double s = f / by(2.0 + f);
   const double z = s * s;
   double p = 0x1.2b5900de53b32p-3;
   p = horner(p, z, 0x1.39fe51a7c18f9p-3);
@@ -180,37 +211,37 @@ __device__ __forceinline__ void icecloud(double p, double z, double dz, double t
   const double sigx = 3.E-4, sigy = 3.E-4, sigz = 1.E-2, xdist = 2500., ydist = 2500.;
   const double r = dmax(0., rv * 1.);
   double s = 0.;
-  const double za = r * p / (P.XEPSILO + r);
-  const double rhw = za / esw, rhi = za / esi, i2w = esw / esi;
+  const double za = r * p / by(P.XEPSILO + r);
+  const double rhw = za / by(esw), rhi = za / by(esi), i2w = esw / by(esi);
   double su = dmin(i2w, rhi), so = su;
   if (t > 273.1 || r <= 0. || esi >= p * 0.5) {
     su = su - 1.;
     so = su;
   } else {
     const double rhin = dmax(0.05, dmin(1., rhw));
-    const double drhdz = rhin * P.XG / (t * P.XRD) * (P.XEPSILO * P.XLVTT / (P.XCPD * t) - 1.);
+    const double drhdz = rhin * P.XG / by(t * P.XRD) * (P.XEPSILO * P.XLVTT / by(P.XCPD * t) - 1.);
     const double zz = dmin(1., dmax(0., z * 0.001));  // PPBLH < 0
     double rhdist = sqrt(xdist * sq(sigx) + ydist * sq(sigy) + (1. - zz) * sq(dz * drhdz) +
                          zz * dz * sq(sigz));
-    if (zz > 0.1) rhdist = rhdist / (1. + rhdist);
+    if (zz > 0.1) rhdist = rhdist / by(1. + rhdist);
     const double rhlim = dmax(0.5, dmin(0.99, 1. - 0.5 * rhdist));
-    double rhdif = (1. - rhw) / (1.0 - rhlim);        // PWCLD < 0
+    double rhdif = (1. - rhw) / by(1.0 - rhlim);        // PWCLD < 0
     rhdif = 1. - sqrt(dmax(0., rhdif));
     const double wcld = dmin(1., dmax(rhdif, 0.0));
     s = wcld;
     const double rhlimice = 1. + i2w * (rhlim - 1.);
     if (rhlim <= 0.999) {
-      rhdif = (rhi - rhlimice) * (1. / (1. - rhlimice));
+      rhdif = (rhi - rhlimice) * (1. / by(1. - rhlimice));
       if (wcld == 0.) {
         s = dmin(1., 0.5 * dmax(0., rhdif));
       } else {
-        s = dmin(1., (1. - 1. / i2w) * 0.5 / (1. - rhlim));
+        s = dmin(1., (1. - 1. / by(i2w)) * 0.5 / by(1. - rhlim));
         s = dmin(1., wcld + s);
       }
     }
     if (s > 0.01) {
       su = s + rhlimice * (1. - s);
-      so = (rhi - (1. - s) * su) / s;
+      so = (rhi - (1. - s) * su) / by(s);
     } else {
       s = 0.;
       su = dmax(0., s + rhlimice * (1. - s) + 2. * dmin(0., rhi - rhlimice));
@@ -258,20 +289,20 @@ __device__ __forceinline__ void ice_adjust_point(double dt, double sigqsat, doub
     frac = 0.;
   } else {
     const double logt = log_f64(zt);
-    pv = dmin(exp_f64(P.XALPW - P.XBETAW / zt - P.XGAMW * logt), .99 * pabs);
-    piv = dmin(exp_f64(P.XALPI - P.XBETAI / zt - P.XGAMI * logt), .99 * pabs);
-    frac = dmax(0., dmin(1., ((P.XTMAXMIX - zt) / (P.XTMAXMIX - P.XTMINMIX))));
+    pv = dmin(exp_f64(P.XALPW - P.XBETAW / by(zt) - P.XGAMW * logt), .99 * pabs);
+    piv = dmin(exp_f64(P.XALPI - P.XBETAI / by(zt) - P.XGAMI * logt), .99 * pabs);
+    frac = dmax(0., dmin(1., ((P.XTMAXMIX - zt) / by(P.XTMAXMIX - P.XTMINMIX))));
   }
-  double qsl = P.XRD / P.XRV * pv / (pabs - pv);
-  const double qsi = P.XRD / P.XRV * piv / (pabs - piv);
+  double qsl = P.XRD / P.XRV * pv / by(pabs - pv);
+  const double qsi = P.XRD / P.XRV * piv / by(pabs - piv);
   qsl = (1. - frac) * qsl + frac * qsi;
   const double lvs = (1. - frac) * lv + frac * ls;
-  const double ah = lvs * qsl / (P.XRV * sq(zt)) * (P.XRV * qsl / P.XRD + 1.);
-  const double a = 1. / (1. + lvs / cph * ah);
-  const double sbar = a * (rt - qsl + ah * lvs * (rc + ri * prifact) / cph);
+  const double ah = lvs * qsl / by(P.XRV * sq(zt)) * (P.XRV * qsl / by(P.XRD) + 1.);
+  const double a = 1. / by(1. + lvs / by(cph) * ah);
+  const double sbar = a * (rt - qsl + ah * lvs * (rc + ri * prifact) / by(cph));
   double sigma = sigqsat != 0. ? sqrt(sq(2 * sigs) + sq(sigqsat * qsl * a)) : 2 * sigs;
   sigma = dmax(1.E-10, sigma);
-  const double q1 = sbar / sigma;
+  const double q1 = sbar / by(sigma);
   double cond;
   if (q1 > 0. && q1 <= 2)
     cond = dmin(exp(-1.) + .66 * q1 + .086 * sq(q1), 2.);
@@ -300,58 +331,58 @@ __device__ __forceinline__ void ice_adjust_point(double dt, double sigqsat, doub
       rc_out = cond - 0.;
     }
     x->wcldfr = cldfr;
-    const double dum1 = dmin(1.0, 20. * rc_out * sqrt(x->dz) / qsl);
+    const double dum1 = dmin(1.0, 20. * rc_out * sqrt(x->dz) / by(qsl));
     const double dum3 = dmax(0., x->icldfr - x->wcldfr);
     double dum4 = x->bottom ? ri : ri + rs * 0.5 + rg * 0.25;
-    dum4 = dmax(0., dmin(1., x->cld_wgt * dum4 * sqrt(x->dz) / qsi));
+    dum4 = dmax(0., dmin(1., x->cld_wgt * dum4 * sqrt(x->dz) / by(qsi)));
     const double dum2 = (0.8 * cldfr + 0.2) * dmin(1., dum1 + dum4 * cldfr);
     cldfr = dmin(1., dum2 + (0.5 * dum3 + 0.5) * dum4);
     ri_out = ri;
-    zt = zt + ((rc_out - rcold) * lv + (ri_out - ri) * ls) / cph;
+    zt = zt + ((rc_out - rcold) * lv + (ri_out - ri) * ls) / by(cph);
   } else {
-    zt = zt + ((rc_out - rc) * lv + (ri_out - ri) * ls) / cph;
+    zt = zt + ((rc_out - rc) * lv + (ri_out - ri) * ls) / by(cph);
   }
   double rv_out = rt - rc_out - ri_out * prifact;
   sigrc = sigrc * dmin(3., dmax(1., 1. - q1));
   // 5.0-5.1 sources
-  double w1 = (rc_out - rc) / dt;
-  double w2 = (ri_out - ri) / dt;
+  double w1 = (rc_out - rc) / by(dt);
+  double w2 = (ri_out - ri) / by(dt);
   if (br) *br |= (w1 < 0.0 ? 1u << ICE3_ABR_ZW1NEG : 0u) | (w2 < 0.0 ? 1u << ICE3_ABR_ZW2NEG : 0u);
   w1 = w1 < 0.0 ? dmax(w1, -rcs) : dmin(w1, rvs);
   rvs = rvs - w1;
   rcs = rcs + w1;
-  ths = ths + w1 * lv / (cph * exnref);
+  ths = ths + w1 * lv / by(cph * exnref);
   w2 = w2 < 0.0 ? dmax(w2, -ris) : dmin(w2, rvs);
   rvs = rvs - w2;
   ris = ris + w2;
-  ths = ths + w2 * ls / (cph * exnref);
+  ths = ths + w2 * ls / by(cph * exnref);
   // 5.2 subgrid: mass-flux contribution, TRIANGLE pdf
-  w1 = rc_mf / dt;
-  w2 = ri_mf / dt;
+  w1 = rc_mf / by(dt);
+  w2 = ri_mf / by(dt);
   if (w1 + w2 > rvs) {
     if (br) *br |= 1u << ICE3_ABR_MFLIMIT;
-    w1 = w1 * rvs / (w1 + w2);
+    w1 = w1 * rvs / by(w1 + w2);
     w2 = rvs - w1;
   }
   cldfr = dmin(1., cldfr + cf_mf);
   rcs = rcs + w1;
   ris = ris + w2;
   rvs = rvs - (w1 + w2);
-  ths = ths + (w1 * lv + w2 * ls) / cph / exnref;
+  ths = ths + (w1 * lv + w2 * ls) / by(cph) / by(exnref);
   double hlc_hcf = 0., hlc_hrc = 0., hli_hcf = 0., hli_hri = 0.;
   {
-    const double criaut = P.XCRIAUTC / rhodref, x = w1 * dt, c = criaut * cf_mf;
+    const double criaut = P.XCRIAUTC / by(rhodref), x = w1 * dt, c = criaut * cf_mf;
     double hcf, hr;
     if (br) *br |= (x > cf_mf * criaut ? 0u : 2. * w1 * dt <= cf_mf * criaut ? 1u : 2u) << ICE3_ABR_PDFC;
     if (x > cf_mf * criaut) {
-      hcf = 1. - .5 * sq(criaut * cf_mf / dmax(1.E-20, x));
-      hr = x - (c * c * c) / (3 * sq(dmax(1.E-20, x)));
+      hcf = 1. - .5 * sq(criaut * cf_mf / by(dmax(1.E-20, x)));
+      hr = x - (c * c * c) / by(3 * sq(dmax(1.E-20, x)));
     } else if (2. * w1 * dt <= cf_mf * criaut) {
       hcf = 0.;
       hr = 0.;
     } else {
-      hcf = sq(2. * w1 * dt - criaut * cf_mf) / (2. * sq(dmax(1.E-20, x)));
-      hr = (4. * (x * x * x) - 3. * w1 * dt * sq(c) + (c * c * c)) / (3 * sq(dmax(1.E-20, x)));
+      hcf = sq(2. * w1 * dt - criaut * cf_mf) / by(2. * sq(dmax(1.E-20, x)));
+      hr = (4. * (x * x * x) - 3. * w1 * dt * sq(c) + (c * c * c)) / by(3 * sq(dmax(1.E-20, x)));
     }
     hlc_hcf = dmin(1., hlc_hcf + hcf * cf_mf);
     hlc_hrc = hlc_hrc + hr;
@@ -365,14 +396,14 @@ __device__ __forceinline__ void ice_adjust_point(double dt, double sigqsat, doub
     double hcf, hr;
     if (br) *br |= (x > cf_mf * criaut ? 0u : 2. * w2 * dt <= cf_mf * criaut ? 1u : 2u) << ICE3_ABR_PDFI;
     if (x > cf_mf * criaut) {
-      hcf = 1. - .5 * sq(criaut * cf_mf / x);
-      hr = x - (c * c * c) / (3 * sq(x));
+      hcf = 1. - .5 * sq(criaut * cf_mf / by(x));
+      hr = x - (c * c * c) / by(3 * sq(x));
     } else if (2. * w2 * dt <= cf_mf * criaut) {
       hcf = 0.;
       hr = 0.;
     } else {
-      hcf = sq(2. * w2 * dt - criaut * cf_mf) / (2. * sq(x));
-      hr = (4. * (x * x * x) - 3. * w2 * dt * sq(c) + (c * c * c)) / (3 * sq(x));
+      hcf = sq(2. * w2 * dt - criaut * cf_mf) / by(2. * sq(x));
+      hr = (4. * (x * x * x) - 3. * w2 * dt * sq(c) + (c * c * c)) / by(3 * sq(x));
     }
     hli_hcf = dmin(1., hli_hcf + hcf * cf_mf);
     hli_hri = hli_hri + hr;
@@ -381,13 +412,13 @@ __device__ __forceinline__ void ice_adjust_point(double dt, double sigqsat, doub
     double v1 = rc_mf, v2 = ri_mf;
     if (br && v1 + v2 > rv_out) *br |= 1u << ICE3_ABR_MFOUT;
     if (v1 + v2 > rv_out) {
-      v1 = v1 * rv_out / (v1 + v2);
+      v1 = v1 * rv_out / by(v1 + v2);
       v2 = rv_out - v1;
     }
     rc_out = rc_out + v1;
     ri_out = ri_out + v2;
     rv_out = rv_out - (v1 + v2);
-    zt = zt + (v1 * lv + v2 * ls) / cph;
+    zt = zt + (v1 * lv + v2 * ls) / by(cph);
   }
   o.t = zt; o.rv = rv_out; o.rc = rc_out; o.ri = ri_out; o.cldfr = cldfr;
   o.hlc_hrc = hlc_hrc; o.hlc_hcf = hlc_hcf; o.hli_hri = hli_hri; o.hli_hcf = hli_hcf;
@@ -409,12 +440,12 @@ __device__ __forceinline__ double tiwmx_at(const double *tiwmx, int table, doubl
   return tiwmx[table * ICE3_TIWMX_N + tiwmx_index(t)];
 }
 
-// ICE4_NUCLEATION (micro/ice4_nucleation.func.h:68-143), LFEEDBACKT.  With OCND2 (FP64 only)
+// ICE4_NUCLEATION (micro/ice4_nucleation.func.h:68-143), LFEEDBACKT; tt_exn is XTT / exn.  With OCND2 (FP64 only)
 // the nucleated concentration is the Meyers function of the tables, reduced between 0 and
 // -20 C and with height, times the ice cloud fraction, and no vapour is taken (:127-139).
 template <class R, bool OCND2 = false>
 __device__ __forceinline__ void nucleation(bool ldcompute, double tht, double pabst, double rhodref,
-                                  double exn, double lsfact, double t, double rvt, double &cit,
+                                  double tt_exn, double lsfact, double t, double rvt, double &cit,
                                   double &rvheni_mr, const MicroOcnd2 *x = nullptr) {
   const bool gnegt = ldcompute && t < P.XTT && rvt > P.XRTMIN[1];
   rvheni_mr = 0.;
@@ -430,25 +461,25 @@ __device__ __forceinline__ void nucleation(bool ldcompute, double tht, double pa
   }
   const R rt = (R)t;
   const R lt = rlog<R>(rt);
-  R usw = rexp<R>((R)P.XALPW - (R)P.XBETAW / rt - (R)P.XGAMW * lt);
-  R zzw = rexp<R>((R)P.XALPI - (R)P.XBETAI / rt - (R)P.XGAMI * lt);
+  R usw = rexp<R>((R)P.XALPW - (R)P.XBETAW / by(rt) - (R)P.XGAMW * lt);
+  R zzw = rexp<R>((R)P.XALPI - (R)P.XBETAI / by(rt) - (R)P.XGAMI * lt);
   const R pab = (R)pabst;
   zzw = dmin(pab / (R)2., zzw);
-  R ssi = (R)rvt * (pab - zzw) / ((R)P.XEPSILO * zzw) - (R)1.0;
+  R ssi = (R)rvt * (pab - zzw) / by((R)P.XEPSILO * zzw) - (R)1.0;
   usw = dmin(pab / (R)2., usw);
-  usw = (usw / zzw) * ((pab - zzw) / (pab - usw)) - (R)1.0;
+  usw = (usw / by(zzw)) * ((pab - zzw) / by(pab - usw)) - (R)1.0;
   ssi = dmin(ssi, usw);
   R nn = 0.;
   if (t < P.XTT - 5.0 && ssi > (R)0.0)
     nn = (R)P.XNU20 * rexp<R>((R)P.XALPHA2 * ssi - (R)P.XBETA2);
   else if (t <= P.XTT - 2.0 && t >= P.XTT - 5.0 && ssi > (R)0.0)
     nn = dmax((R)P.XNU20 * rexp<R>(-(R)P.XBETA2),
-              (R)P.XNU10 * rexp<R>(-(R)P.XBETA1 * (rt - (R)P.XTT)) * rpow<R>(ssi / usw, (R)P.XALPHA1));
+              (R)P.XNU10 * rexp<R>(-(R)P.XBETA1 * (rt - (R)P.XTT)) * rpow<R>(ssi / by(usw), (R)P.XALPHA1));
   double zz = (double)nn - cit;
   zz = dmin(zz, 50.E3);
-  double rv_mr = dmax(zz, 0.0) * P.XMNU0 / rhodref;
+  double rv_mr = dmax(zz, 0.0) * P.XMNU0 / by(rhodref);
   rv_mr = dmin(rvt, rv_mr);
-  const double zw = dmin(rv_mr, dmax(0., (P.XTT / exn - tht) / lsfact)) / dmax(rv_mr, 1.E-20);
+  const double zw = dmin(rv_mr, dmax(0., (tt_exn - tht) / by(lsfact))) / by(dmax(rv_mr, 1.E-20));
   rvheni_mr = rv_mr * zw;
   zz = zz * zw;
   cit = dmax(zz + cit, cit);
@@ -558,8 +589,8 @@ template <class R> __device__ __forceinline__ R powl_(R lnx, R c) { return rexp<
 // (micro/mode_ice4_fast_rh.F90) and their PA / PB terms (:619-716); htab then holds the
 // wet-growth kernels of hail (the block that follows the ICE3 tables, ICE3_T_ICE3 on).
 template <class R, bool OCND2 = false, bool HAIL = false, class TB, class SS>
-__device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref, double lvfact,
-                                  double lsfact, double pres, double cf, double sigma_rc,
+__device__ __forceinline__ void tendencies(bool soft, double exn, double tt_exn, double rhodref,
+                                  double lvfact, double lsfact, double pres, double cf, double sigma_rc,
                                   double &cit, double pt, const double *pvart,
                                   SS &S, const PointConst<R> &pc,
                                   const TB *__restrict__ tab, double *pa, double *pb,
@@ -575,17 +606,18 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
   for (int jv = 0; jv < NV; ++jv) { zv[jv] = pvart[jv]; pa[jv] = 0.; pb[jv] = 0.; }
   double rrhong_mr = 0.;  // RRHONG of the hard call (graupel produced at once)
   R ka = 0, dv = 0, ai = 0, cj = 0, lnt = 0, esi = 0, esw = 0;
+  R dep = 0;  // ssi / (rho ai): deposition on snow and graupel, Bergeron-Findeisen
   double esi_tab = 0., colf = 1., acrf = 1.;  // OCND2: tabulated ZESI, ZCOLF, ZACRF
   if (!soft) {
     double rvheni, rrhong, rimltc;
-    nucleation<R, OCND2>(true, zv[ITH], pres, rhodref, exn, lsfact, zt, zv[IRV], cit, rvheni, x);
+    nucleation<R, OCND2>(true, zv[ITH], pres, rhodref, tt_exn, lsfact, zt, zv[IRV], cit, rvheni, x);
     zv[ITH] = zv[ITH] + rvheni * lsfact;
     zt = zv[ITH] * exn;
     zv[IRV] = zv[IRV] - rvheni;
     zv[IRI] = zv[IRI] + rvheni;
     // RRHONG (micro/mode_ice4_rrhong.F90:65-75)
     if (zt < P.XTT - 35.0 && zv[IRR] > P.XRTMIN[3])
-      rrhong = dmin(zv[IRR], dmax(0., ((P.XTT - 35.) / exn - zv[ITH]) / (lsfact - lvfact)));
+      rrhong = dmin(zv[IRR], dmax(0., ((P.XTT - 35.) / by(exn) - zv[ITH]) / by(lsfact - lvfact)));
     else
       rrhong = 0.;
     if (br && rrhong > 0.) *br |= 1u << ICE3_BR_RRHONG;
@@ -596,7 +628,7 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
     rrhong_mr = rrhong;
     // RIMLTC (micro/mode_ice4_rimltc.F90:64-74)
     if (zv[IRI] > 0. && zt > P.XTT)
-      rimltc = dmin(zv[IRI], dmax(0., (zv[ITH] - P.XTT / exn) / (lsfact - lvfact)));
+      rimltc = dmin(zv[IRI], dmax(0., (zv[ITH] - tt_exn) / by(lsfact - lvfact)));
     else
       rimltc = 0.;
     if (br && rimltc > 0.) *br |= 1u << ICE3_BR_RIMLTC;
@@ -616,36 +648,37 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
     // derived fields (:312-320)
     const R t = (R)zt;
     lnt = rlog<R>(t);
-    esi = rexp<R>((R)P.XALPI - (R)P.XBETAI / t - (R)P.XGAMI * lnt);
-    esw = rexp<R>((R)P.XALPW - (R)P.XBETAW / t - (R)P.XGAMW * lnt);
+    esi = rexp<R>((R)P.XALPI - (R)P.XBETAI / by(t) - (R)P.XGAMI * lnt);
+    esw = rexp<R>((R)P.XALPW - (R)P.XBETAW / by(t) - (R)P.XGAMW * lnt);
     if constexpr (OCND2) {
       esi_tab = tiwmx_at(x->tiwmx, ICE3_TW_ESI, zt);
-      S.ssi = (R)(zv[IRV] * (pres - esi_tab) / (P.XEPSILO * esi_tab) - 1.0);
+      S.ssi = (R)(zv[IRV] * (pres - esi_tab) / by(P.XEPSILO * esi_tab) - 1.0);
       ka = (R)2.38E-2 + (R)0.0071E-2 * (t - (R)P.XTT);
-      dv = (R)0.211E-4 * powl_<R>(lnt - (R)P.LN_XTT, (R)1.94) * ((R)P.XP00 / (R)pres);
+      dv = (R)0.211E-4 * powl_<R>(lnt - (R)P.LN_XTT, (R)1.94) * ((R)P.XP00 / by((R)pres));
       ai = (R)(tiwmx_at(x->tiwmx, ICE3_TW_A2, zt) + tiwmx_at(x->tiwmx, ICE3_TW_BB3, zt) * pres);
     } else {
       const R zzw = esi;
-      S.ssi = (R)zv[IRV] * ((R)pres - zzw) / ((R)P.XEPSILO * zzw) - (R)1.0;
+      S.ssi = (R)zv[IRV] * ((R)pres - zzw) / by((R)P.XEPSILO * zzw) - (R)1.0;
       ka = (R)2.38E-2 + (R)0.0071E-2 * (t - (R)P.XTT);
-      dv = (R)0.211E-4 * powl_<R>(lnt - (R)P.LN_XTT, (R)1.94) * ((R)P.XP00 / (R)pres);
-      ai = sq((R)P.XLSTT + (R)(P.XCPV - P.XCI) * (t - (R)P.XTT)) / (ka * (R)P.XRV * sq(t)) +
-           ((R)P.XRV * t) / (dv * zzw);
+      dv = (R)0.211E-4 * powl_<R>(lnt - (R)P.LN_XTT, (R)1.94) * ((R)P.XP00 / by((R)pres));
+      ai = sq((R)P.XLSTT + (R)(P.XCPV - P.XCI) * (t - (R)P.XTT)) / by(ka * (R)P.XRV * sq(t)) +
+           ((R)P.XRV * t) / by(dv * zzw);
     }
-    cj = (R)P.XSCFAC * pc.rho03 / sqrt((R)1.718E-5 + (R)0.0049E-5 * (t - (R)P.XTT));
+    dep = S.ssi / by((R)rhodref * ai);
+    cj = (R)P.XSCFAC * pc.rho03 / by(sqrt((R)1.718E-5 + (R)0.0049E-5 * (t - (R)P.XTT)));
     if constexpr (OCND2) {  // collision factors, PCONC = XCONC_LAND (:321-345)
       colf = 0.00001;
       acrf = 0.00001;
       if (zv[IRC] > 1.0E-10) {
         const double conc = P.XCONC_LAND * 0.000001;
-        const double rcw = 0.1 * rpow<double>(0.75 * zv[IRC] * rhodref / (P.XPI * conc), 0.333);
+        const double rcw = 0.1 * rpow<double>(0.75 * zv[IRC] * rhodref / by(P.XPI * conc), 0.333);
         double vt = rcw < 0.0065 ? 1.19E6 * sq(rcw) : 8000. * rcw;
         vt = dmin(10., vt);
-        const double st = dmax(0.01, 2. * (100. - vt) * vt / (P.XG * 10.));
+        const double st = dmax(0.01, 2. * (100. - vt) * vt / by(P.XG * 10.));
         if (st > 0.1) colf = dmax(0.01, dmin(1., 0.939 * rpow<double>(st, 2.657)));
         if (zv[IRR] > 1.0E-10 && rcw > 1.0E-5) {
           const double r20 = exp_f64(rcw * 2000.);
-          acrf = (r20 - 1.) / (r20 + 1.);
+          acrf = (r20 - 1.) / by(r20 + 1.);
         }
       }
     }
@@ -658,12 +691,12 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
   // ICE4_COMPUTE_PDF (micro/mode_ice4_compute_pdf.F90:88-390): rc 'PDF'+'SIGM', ri 'NONE'
   R hlc_hcf, hlc_hrc, hli_hcf, hli_hri, criauti;
   {
-    const double rcrautc = P.XCRIAUTC / rhodref, zrc = zv[IRC];
+    const double rcrautc = P.XCRIAUTC / by(rhodref), zrc = zv[IRC];
     if (zrc > rcrautc + sigma_rc) {
       hlc_hcf = 1.; hlc_hrc = (R)zrc;
     } else if (zrc > (rcrautc - sigma_rc) && zrc <= (rcrautc + sigma_rc)) {
-      hlc_hcf = (R)((zrc + sigma_rc - rcrautc) / (2. * sigma_rc));
-      hlc_hrc = (R)((zrc + sigma_rc - rcrautc) * (zrc + sigma_rc + rcrautc) / (4. * sigma_rc));
+      hlc_hcf = (R)((zrc + sigma_rc - rcrautc) / by(2. * sigma_rc));
+      hlc_hrc = (R)((zrc + sigma_rc - rcrautc) * (zrc + sigma_rc + rcrautc) / by(4. * sigma_rc));
     } else {
       hlc_hcf = 0.; hlc_hrc = 0.;
     }
@@ -677,24 +710,40 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
 
   // slope parameters (:389-433), hard calls only (soft calls reuse rates)
   // ln(lbda) is kept beside each lbda: every power and table index below uses it.
+  // Powers with the same exponent are one power: graupel's and hail's sticking efficiencies,
+  // lbda_s^-1.27 of the aggregation and the riming, lbda_s^-0.9 of the riming and the collections,
+  // lbda_r^-3.8 of the accretion and the freezing by ice; lbda_s^XCXS is lbda_s before its bound,
+  // and the first term of snow's ventilation is constant (k_micro 2.85 -> 2.80 ms at 512x512x90,
+  // with hail 4.84 -> 4.67).
+  static_assert(P.XCXS == 1. && P.XEX0DEPS == 0. && P.XEXIAGGS == P.XEXCRIMSS &&
+                    P.XCXS - P.XBS == P.XEXSRIMCG && P.XEXCACCR == P.XEXICFRR &&
+                    P.XCOLEXIG == P.XCOLEXSG && P.XCOLEXIG == P.XCOLEXIH &&
+                    P.XCOLEXIG == P.XCOLEXSH && P.XCOLEXIG == P.XCOLEXGH,
+                "exponents of the pinned configuration");
   R lbdar = 0, lbdas = 0, lbdag = 0, llr = 0, lls = 0, llg = 0;
+  R lbs_cxs = 0, lbs_cxs_bs = 0, lbs_agg = 0, vent_s = 0, vent_g = 0, lbg_cxg = 0, lbr_acc = 0;
   if (!soft) {
     if (rr > (R)0.) {
       llr = (R)P.LN_XLBR + (R)P.XLBEXR * rlog<R>(rho * dmax(rr, (R)P.XRTMIN[3]));
       lbdar = rexp<R>(llr);
+      lbr_acc = powl_<R>(llr, (R)P.XEXCACCR);
     }
     if (rs > (R)0.) {
       lls = (R)P.LN_XLBS + (R)P.XLBEXS * rlog<R>(rho * dmax(rs, (R)P.XRTMIN[5]));
-      if (lls < (R)P.LN_XLBDAS_MAX) {
-        lbdas = rexp<R>(lls);
-      } else {
-        lbdas = (R)P.XLBDAS_MAX;
-        lls = (R)P.LN_XLBDAS_MAX;
-      }
+      const bool bounded = !(lls < (R)P.LN_XLBDAS_MAX);
+      if (bounded) lls = (R)P.LN_XLBDAS_MAX;
+      lbs_cxs = rexp<R>(lls);
+      lbdas = bounded ? (R)P.XLBDAS_MAX : lbs_cxs;
+      // (1 + 0 lls: a non-finite slope stays so)
+      vent_s = (R)P.X0DEPS * ((R)1. + (R)P.XEX0DEPS * lls) + (R)P.X1DEPS * cj * powl_<R>(lls, (R)P.XEX1DEPS);
+      lbs_cxs_bs = powl_<R>(lls, (R)(P.XCXS - P.XBS));
+      lbs_agg = powl_<R>(lls, (R)P.XEXIAGGS);
     }
     if (rg > (R)0.) {
       llg = (R)P.LN_XLBG + (R)P.XLBEXG * rlog<R>(rho * dmax(rg, (R)P.XRTMIN[6]));
       lbdag = rexp<R>(llg);
+      vent_g = (R)P.X0DEPG * powl_<R>(llg, (R)P.XEX0DEPG) + (R)P.X1DEPG * cj * powl_<R>(llg, (R)P.XEX1DEPG);
+      lbg_cxg = powl_<R>(llg, (R)P.XCXG);
     }
   }
   R lbdah = 0, llh = 0, vent_h = 0;
@@ -705,18 +754,7 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
     }
   }
   const R rhomcexvt = soft ? (R)0 : pc.rhomcexvt;
-  // powers of the snow and graupel slopes used by several processes of the hard call
-  // (vapour deposition, freezing budget, melting; accretion and dry growth)
-  R vent_s = 0, vent_g = 0, lbs_cxs_bs = 0, lbg_cxg = 0;
   if (!soft) {
-    if (rs > (R)0.) {
-      vent_s = (R)P.X0DEPS * powl_<R>(lls, (R)P.XEX0DEPS) + (R)P.X1DEPS * cj * powl_<R>(lls, (R)P.XEX1DEPS);
-      lbs_cxs_bs = powl_<R>(lls, (R)(P.XCXS - P.XBS));
-    }
-    if (rg > (R)0.) {
-      vent_g = (R)P.X0DEPG * powl_<R>(llg, (R)P.XEX0DEPG) + (R)P.X1DEPG * cj * powl_<R>(llg, (R)P.XEX1DEPG);
-      lbg_cxg = powl_<R>(llg, (R)P.XCXG);
-    }
     if constexpr (HAIL)
       if (zv[IRH] > 0.)
         vent_h = (R)P.X0DEPH * powl_<R>(llh, (R)P.XEX0DEPH) + (R)P.X1DEPH * cj * powl_<R>(llh, (R)P.XEX1DEPH);
@@ -732,12 +770,12 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
   } else S.rchoni = 0;
   if (rv_ok && rs_ok) {
     if (!soft) {
-      S.rvdeps = (ssi / (rho * ai)) * vent_s;
+      S.rvdeps = dep * vent_s;
       if constexpr (OCND2) S.rvdeps = S.rvdeps * (R)P.XFRMIN[40];
     }
   } else S.rvdeps = 0;
   if (ri_ok && rs_ok) {
-    if (!soft) S.riaggs = (R)P.XFIAGGS * rexp<R>((R)P.XCOLEXIS * (t - (R)P.XTT)) * ri * powl_<R>(lls, (R)P.XEXIAGGS) * rhomcexvt;
+    if (!soft) S.riaggs = (R)P.XFIAGGS * rexp<R>((R)P.XCOLEXIS * (t - (R)P.XTT)) * ri * lbs_agg * rhomcexvt;
   } else S.riaggs = 0;
   if (hli_hri > (R)P.XRTMIN[4]) {
     if (!soft) {
@@ -746,7 +784,7 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
   } else S.riauts = 0;
   if (rv_ok && rg_ok) {
     if (!soft) {
-      S.rvdepg = (ssi / (rho * ai)) * vent_g;
+      S.rvdepg = dep * vent_g;
       if constexpr (OCND2) S.rvdepg = S.rvdepg * (R)P.XFRMIN[39];
     }
   } else S.rvdepg = 0;
@@ -754,39 +792,49 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
   double zdepg_s = 0., znodepg_s = 1.;
   if constexpr (OCND2) {
     if (P.XFRMIN[5] > 1.0E-12 && P.XFRMIN[6] > 0.01) {
-      zdepg_s = dmax(0., dmin(1., (P.XFRMIN[5] - zv[IRG] / P.XFRMIN[5]))) *
-                dmax(0., dmin(1., ((double)ssi / P.XFRMIN[6])));
+      zdepg_s = dmax(0., dmin(1., (P.XFRMIN[5] - zv[IRG] / by(P.XFRMIN[5])))) *
+                dmax(0., dmin(1., ((double)ssi / by(P.XFRMIN[6]))));
       znodepg_s = 1. - zdepg_s;
     }
   }
 
   // ICE4_WARM (micro/mode_ice4_warm.F90:100-197)
   if (hlc_hrc > (R)P.XRTMIN[2] && hlc_hcf > (R)0.) {
-    if (!soft) S.rcautr = (R)P.XTIMAUTC * dmax(hlc_hrc - hlc_hcf * (R)P.XCRIAUTC / rho, (R)0.0);
+    if (!soft) S.rcautr = (R)P.XTIMAUTC * dmax(hlc_hrc - hlc_hcf * (R)P.XCRIAUTC / by(rho), (R)0.0);
   } else S.rcautr = 0;
   if (rc_ok && rr_ok) {
-    if (!soft) S.rcaccr = (R)P.XFCACCR * rc * (R)acrf * powl_<R>(llr, (R)P.XEXCACCR) * rhomcexvt;
+    if (!soft) S.rcaccr = (R)P.XFCACCR * rc * (R)acrf * lbr_acc * rhomcexvt;
   } else S.rcaccr = 0;
   if (rr_ok && !rc_ok) {
     if (!soft) {
       const R ev = esw;
-      const R usw = (R)1. - rv * ((R)pres - ev) / ((R)P.XEPSILO * ev);
-      const R x = sq((R)P.XLVTT + (R)(P.XCPV - P.XCL) * (t - (R)P.XTT)) / (ka * (R)P.XRV * sq(t)) + ((R)P.XRV * t) / (dv * ev);
-      S.rrevav = (dmax((R)0., usw) / (rho * x)) * ((R)P.X0EVAR * powl_<R>(llr, (R)P.XEX0EVAR) + (R)P.X1EVAR * cj * powl_<R>(llr, (R)P.XEX1EVAR));
+      const R usw = (R)1. - rv * ((R)pres - ev) / by((R)P.XEPSILO * ev);
+      const R x = sq((R)P.XLVTT + (R)(P.XCPV - P.XCL) * (t - (R)P.XTT)) / by(ka * (R)P.XRV * sq(t)) + ((R)P.XRV * t) / by(dv * ev);
+      S.rrevav = (dmax((R)0., usw) / by(rho * x)) * ((R)P.X0EVAR * powl_<R>(llr, (R)P.XEX0EVAR) + (R)P.X1EVAR * cj * powl_<R>(llr, (R)P.XEX1EVAR));
     }
   } else S.rrevav = 0;
+
+  // heat budget of a collecting or melting particle, per unit ventilation, with the vapour
+  // pressure capped by saturation over ice (freezing) or water (melting), and the freezing
+  // efficiency: the same for snow, graupel and hail
+  R heat_i = 0, heat_w = 0, freez_eff = 0;
+  By<R> freez_den{};
+  if (!soft && (rs_ok || rg_ok || (HAIL && zv[NV - 1] > P.XRTMIN[7]))) {
+    const R ev = rv * (R)pres / by((R)P.XEPSILO + rv);
+    const By<R> rvt = by((R)P.XRV * t);
+    const R dvl = dv * ((R)P.XLVTT + (R)(P.XCPV - P.XCL) * (t - (R)P.XTT));
+    heat_i = ka * ((R)P.XTT - t) + (dvl * ((R)P.XESTT - dmin(ev, esi)) / rvt);
+    if (warm) heat_w = ka * ((R)P.XTT - t) + (dvl * ((R)P.XESTT - dmin(ev, esw)) / rvt);
+    freez_den = by(rho * ((R)P.XLMTT - (R)P.XCL * ((R)P.XTT - t)));
+    freez_eff = (rho * ((R)P.XLMTT + (R)(P.XCI - P.XCL) * ((R)P.XTT - t))) / freez_den;
+  }
 
   // ICE4_FAST_RS (micro/mode_ice4_fast_rs.F90:109-441)
   R freez;
   if (rs_ok) {
     if (!soft) {
-      R f1 = rv * (R)pres / ((R)P.XEPSILO + rv);
-      f1 = dmin(f1, esi);
-      f1 = ka * ((R)P.XTT - t) + (dv * ((R)P.XLVTT + (R)(P.XCPV - P.XCL) * (t - (R)P.XTT)) * ((R)P.XESTT - f1) / ((R)P.XRV * t));
-      f1 = f1 * vent_s /
-           (rho * ((R)P.XLMTT - (R)P.XCL * ((R)P.XTT - t)));
-      S.rs_freez1 = f1;
-      S.rs_freez2 = (rho * ((R)P.XLMTT + (R)(P.XCI - P.XCL) * ((R)P.XTT - t))) / (rho * ((R)P.XLMTT - (R)P.XCL * ((R)P.XTT - t)));
+      S.rs_freez1 = heat_i * vent_s / freez_den;
+      S.rs_freez2 = freez_eff;
     }
     freez = dmax((R)0., dmax((R)0., S.rs_freez1 + S.rs_freez2 * S.riaggs) - S.riaggs);
   } else {
@@ -798,18 +846,17 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
     const R zzw1 = interp1d<R>(lls, P.NGAMINC, (R)P.XRIMINTP1, (R)P.XRIMINTP2, tab + ICE3_T_RIM1);
     const R zzw2 = interp1d<R>(lls, P.NGAMINC, (R)P.XRIMINTP1, (R)P.XRIMINTP2, tab + ICE3_T_RIM2);
     const R zzw3 = interp1d<R>(lls, P.NGAMINC, (R)P.XRIMINTP1, (R)P.XRIMINTP2, tab + ICE3_T_RIM4);
-    const R lexc = powl_<R>(lls, (R)P.XEXCRIMSS);
-    S.rs_rcrimss = (R)P.XCRIMSS * zzw1 * rc * (R)colf * lexc * rhomcexvt;
-    S.rs_rcrims = (R)P.XCRIMSG * rc * (R)colf * lexc * rhomcexvt;
+    S.rs_rcrimss = (R)P.XCRIMSS * zzw1 * rc * (R)colf * lbs_agg * rhomcexvt;
+    S.rs_rcrims = (R)P.XCRIMSG * rc * (R)colf * lbs_agg * rhomcexvt;
     const R zzw = S.rs_rcrims - S.rs_rcrimss;
-    const R x = (R)P.XSRIMCG * powl_<R>(lls, (R)P.XEXSRIMCG) * ((R)1.0 - zzw2);
-    S.rs_rsrimcg = zzw * x / dmax((R)1.E-20, (R)P.XSRIMCG3 * (R)P.XSRIMCG2 * powl_<R>(lls, (R)P.XEXSRIMCG2) * ((R)1. - zzw3) - (R)P.XSRIMCG3 * x);
+    const R x = (R)P.XSRIMCG * lbs_cxs_bs * ((R)1.0 - zzw2);
+    S.rs_rsrimcg = zzw * x / by(dmax((R)1.E-20, (R)P.XSRIMCG3 * (R)P.XSRIMCG2 * powl_<R>(lls, (R)P.XEXSRIMCG2) * ((R)1. - zzw3) - (R)P.XSRIMCG3 * x));
   }
   R rcrimss = 0, rcrimsg = 0, rsrimcg = 0;
   if (grim && cold) {
     rcrimss = dmin(freez, S.rs_rcrimss);
     freez = dmax((R)0., freez - rcrimss);
-    const R zzw0d = dmin((R)1., freez / dmax((R)1.E-20, S.rs_rcrims - rcrimss));
+    const R zzw0d = dmin((R)1., freez / by(dmax((R)1.E-20, S.rs_rcrims - rcrimss)));
     rcrimsg = zzw0d * dmax((R)0., S.rs_rcrims - rcrimss);
     freez = dmax((R)0., freez - rcrimsg);
     rsrimcg = zzw0d * S.rs_rsrimcg;
@@ -828,21 +875,21 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
       const R zzw3 = interp2d_t<R>(ix, P.NACCLBDAR, tab + ICE3_T_SACCRG);
       const R rhom = pc.rhom;
       const R lr2 = lbdar * lbdar;
-      const R zzw = (R)P.XFRACCSS * (powl_<R>(lls, (R)P.XCXS)) * rhom *
-                    ((R)P.XLBRACCS1 / (sq(lbdas)) + (R)P.XLBRACCS2 / (lbdas * lbdar) + (R)P.XLBRACCS3 / (lr2)) / (lr2 * lr2);
+      const R zzw = (R)P.XFRACCSS * lbs_cxs * rhom *
+                    ((R)P.XLBRACCS1 / by(sq(lbdas)) + (R)P.XLBRACCS2 / by(lbdas * lbdar) + (R)P.XLBRACCS3 / by(lr2)) / by(lr2 * lr2);
       S.rs_rraccss = zzw1 * zzw;
       if constexpr (OCND2) S.rs_rraccss = S.rs_rraccss * (R)P.XFRMIN[7];
       S.rs_rraccs = zzw2 * zzw;
       if (!OCND2 || zv[IRS] > P.XFRMIN[1])
         S.rs_rsaccrg = (R)P.XFSACCRG * zzw3 * lbs_cxs_bs * rhom *
-                       ((R)P.XLBSACCR1 / (lr2) + (R)P.XLBSACCR2 / (lbdar * lbdas) + (R)P.XLBSACCR3 / (sq(lbdas))) / lbdar;
+                       ((R)P.XLBSACCR1 / by(lr2) + (R)P.XLBSACCR2 / by(lbdar * lbdas) + (R)P.XLBSACCR3 / by(sq(lbdas))) / by(lbdar);
     }
   }
   R rraccss = 0, rraccsg = 0, rsaccrg = 0;
   if (gacc && cold) {
     rraccss = dmin(freez, S.rs_rraccss);
     freez = dmax((R)0., freez - rraccss);
-    const R zzw = dmin((R)1., freez / dmax((R)1.E-20, S.rs_rraccs - rraccss));
+    const R zzw = dmin((R)1., freez / by(dmax((R)1.E-20, S.rs_rraccs - rraccss)));
     rraccsg = zzw * dmax((R)0., S.rs_rraccs - rraccss);
     freez = dmax((R)0., freez - rraccsg);
     rsaccrg = zzw * S.rs_rsaccrg;
@@ -851,11 +898,8 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
   }
   if (rs_ok && warm) {
     if (!soft) {
-      R m = rv * (R)pres / ((R)P.XEPSILO + rv);
-      m = dmin(m, esw);
-      m = ka * ((R)P.XTT - t) + (dv * ((R)P.XLVTT + (R)(P.XCPV - P.XCL) * (t - (R)P.XTT)) * ((R)P.XESTT - m) / ((R)P.XRV * t));
-      S.rsmltg = (R)P.XFSCVMG * dmax((R)0., (-m * vent_s -
-                                              (S.rs_rcrims + S.rs_rraccs) * (rho * (R)P.XCL * ((R)P.XTT - t))) / (rho * (R)P.XLMTT));
+      S.rsmltg = (R)P.XFSCVMG * dmax((R)0., (-heat_w * vent_s -
+                                              (S.rs_rcrims + S.rs_rraccs) * (rho * (R)P.XCL * ((R)P.XTT - t))) / by(rho * (R)P.XLMTT));
       S.rcmltsr = S.rs_rcrims;
     }
   } else {
@@ -865,9 +909,9 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
   // ICE4_FAST_RG (micro/mode_ice4_fast_rg.F90:121-410)
   if (ri_ok && rr_ok) {
     if (!soft) {
-      R icf = (R)P.XICFRR * ri * powl_<R>(llr, (R)P.XEXICFRR) * rhomcexvt;
+      R icf = (R)P.XICFRR * ri * lbr_acc * rhomcexvt;
       R rcf = (R)P.XRCFRI * (R)cit * powl_<R>(llr, (R)P.XEXRCFRI) * pc.rhom;
-      const R zzw0d = dmax((R)0., dmin((R)1., (icf * (R)P.XCI + rcf * (R)P.XCL) * ((R)P.XTT - t) / dmax((R)1.E-20, (R)P.XLVTT * rcf)));
+      const R zzw0d = dmax((R)0., dmin((R)1., (icf * (R)P.XCI + rcf * (R)P.XCL) * ((R)P.XTT - t) / by(dmax((R)1.E-20, (R)P.XLVTT * rcf))));
       S.rrcfrig = zzw0d * rcf;
       S.ricfrr = ((R)1. - zzw0d) * icf;
       S.ricfrrg = zzw0d * icf;
@@ -875,15 +919,16 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
   } else {
     S.ricfrrg = 0; S.rrcfrig = 0; S.ricfrr = 0;
   }
+  R stick = 0;  // exp(XCOLEX (t - XTT)): ice and snow sticking to graupel (or hail)
+  if (!soft && (rg_ok || (HAIL && zv[NV - 1] > P.XRTMIN[7]))) stick = rexp<R>((R)P.XCOLEXIG * (t - (R)P.XTT));
   const R lgx = (!soft && rg_ok) ? powl_<R>(llg, (R)(P.XCXG - P.XDG - 2.)) * rhomcexvt : (R)0;
   if (rg_ok && rc_ok) {
     if (!soft) S.rg_rcdryg = (R)P.XFCDRYG * rc * lgx;
   } else S.rg_rcdryg = 0;
   if (rg_ok && ri_ok) {
     if (!soft) {
-      const R e = rexp<R>((R)P.XCOLEXIG * (t - (R)P.XTT));
-      S.rg_ridryg = (R)P.XFIDRYG * e * ri * lgx;
-      S.rg_riwetg = S.rg_ridryg / ((R)P.XCOLIG * e);
+      S.rg_ridryg = (R)P.XFIDRYG * stick * ri * lgx;
+      S.rg_riwetg = S.rg_ridryg / by((R)P.XCOLIG * stick);
     }
   } else {
     S.rg_ridryg = 0; S.rg_riwetg = 0;
@@ -895,9 +940,9 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
     const Idx2<R> ix = interp2d_idx<R>(llg, lls, P.NDRYLBDAG, P.NDRYLBDAS, (R)P.XDRYINTP1G,
                                        (R)P.XDRYINTP2G, (R)P.XDRYINTP1S, (R)P.XDRYINTP2S);
     const R zzw = interp2d<R>(ix, P.NDRYLBDAG, tab + ICE3_T_SDRYG);
-    S.rg_rswetg = (R)P.XFSDRYG * zzw / (R)P.XCOLSG * lbs_cxs_bs * lbg_cxg * rhom1 *
-                  ((R)P.XLBSDRYG1 / (sq(lbdag)) + (R)P.XLBSDRYG2 / (lbdag * lbdas) + (R)P.XLBSDRYG3 / (sq(lbdas)));
-    S.rg_rsdryg = S.rg_rswetg * (R)P.XCOLSG * rexp<R>((R)P.XCOLEXSG * (t - (R)P.XTT));
+    S.rg_rswetg = (R)P.XFSDRYG * zzw / by((R)P.XCOLSG) * lbs_cxs_bs * lbg_cxg * rhom1 *
+                  ((R)P.XLBSDRYG1 / by(sq(lbdag)) + (R)P.XLBSDRYG2 / by(lbdag * lbdas) + (R)P.XLBSDRYG3 / by(sq(lbdas)));
+    S.rg_rsdryg = S.rg_rswetg * (R)P.XCOLSG * stick;
   }
   const bool gdryr = rr_ok && rg_ok;
   if (!gdryr) S.rg_rrdryg = 0;
@@ -906,21 +951,16 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
                                        (R)P.XDRYINTP2G, (R)P.XDRYINTP1R, (R)P.XDRYINTP2R);
     const R zzw = interp2d<R>(ix, P.NDRYLBDAG, tab + ICE3_T_RDRYG);
     const R lr2 = lbdar * lbdar;
-    S.rg_rrdryg = (R)P.XFRDRYG * zzw * ((R)1.0 / (lr2 * lr2)) * lbg_cxg * rhom1 *
-                  ((R)P.XLBRDRYG1 / (sq(lbdag)) + (R)P.XLBRDRYG2 / (lbdag * lbdar) + (R)P.XLBRDRYG3 / (lr2));
+    S.rg_rrdryg = (R)P.XFRDRYG * zzw * ((R)1.0 / by(lr2 * lr2)) * lbg_cxg * rhom1 *
+                  ((R)P.XLBRDRYG1 / by(sq(lbdag)) + (R)P.XLBRDRYG2 / by(lbdag * lbdar) + (R)P.XLBRDRYG3 / by(lr2));
   }
   const R rdryg_init = S.rg_rcdryg + S.rg_ridryg + S.rg_rsdryg + S.rg_rrdryg;
   R rwetg_init = 0;
   bool ldwetg = false, lldryg = false;
   if (rg_ok) {
     if (!soft) {
-      R f1 = rv * (R)pres / ((R)P.XEPSILO + rv);
-      f1 = dmin(f1, esi);
-      f1 = ka * ((R)P.XTT - t) + (dv * ((R)P.XLVTT + (R)(P.XCPV - P.XCL) * (t - (R)P.XTT)) * ((R)P.XESTT - f1) / ((R)P.XRV * t));
-      f1 = f1 * vent_g /
-           (rho * ((R)P.XLMTT - (R)P.XCL * ((R)P.XTT - t)));
-      S.rg_freez1 = f1;
-      S.rg_freez2 = (rho * ((R)P.XLMTT + (R)(P.XCI - P.XCL) * ((R)P.XTT - t))) / (rho * ((R)P.XLMTT - (R)P.XCL * ((R)P.XTT - t)));
+      S.rg_freez1 = heat_i * vent_g / freez_den;
+      S.rg_freez2 = freez_eff;
     }
     rwetg_init = dmax(S.rg_riwetg + S.rg_rswetg, dmax((R)0., S.rg_freez1 + S.rg_freez2 * (S.rg_riwetg + S.rg_rswetg)));
     const R wet = dmax((R)0., rwetg_init - S.rg_riwetg - S.rg_rswetg);
@@ -938,8 +978,8 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
       const R rgsi = S.rvdepg + S.rsmltg + rraccsg + rsaccrg + rcrimsg + rsrimcg;
       const R rgsi_mr = (R)rrhong_mr;
       rwetgh = (dmax((R)0., rgsi + S.ricfrrg + S.rrcfrig) + rwetg_init) * rdryg_init /
-               (rwetg_init + rdryg_init);
-      rwetgh_mr = dmax((R)0., rgsi_mr) * rdryg_init / (rwetg_init + rdryg_init);
+               by(rwetg_init + rdryg_init);
+      rwetgh_mr = dmax((R)0., rgsi_mr) * rdryg_init / by(rwetg_init + rdryg_init);
     }
   }
   R rrwetg = 0, rcwetg = 0, riwetg = 0, rswetg = 0, rcdryg = 0, rrdryg = 0, ridryg = 0, rsdryg = 0;
@@ -952,11 +992,8 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
   }
   if (rg_ok && warm) {
     if (!soft) {
-      R m = rv * (R)pres / ((R)P.XEPSILO + rv);
-      m = dmin(m, esw);
-      m = ka * ((R)P.XTT - t) + dv * ((R)P.XLVTT + (R)(P.XCPV - P.XCL) * (t - (R)P.XTT)) * ((R)P.XESTT - m) / ((R)P.XRV * t);
-      S.rgmltr = dmax((R)0., (-m * vent_g -
-                              (S.rg_rcdryg + S.rg_rrdryg) * (rho * (R)P.XCL * ((R)P.XTT - t))) / (rho * (R)P.XLMTT));
+      S.rgmltr = dmax((R)0., (-heat_w * vent_g -
+                              (S.rg_rcdryg + S.rg_rrdryg) * (rho * (R)P.XCL * ((R)P.XTT - t))) / by(rho * (R)P.XLMTT));
     }
   } else S.rgmltr = 0;
 
@@ -975,7 +1012,7 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
     if (rh_ok && ri_ok) {
       if (!soft) {
         S.rh_riweth = (R)P.XFWETH * ri * lhx;
-        S.rh_ridryh = S.rh_riweth * ((R)P.XCOLIH * rexp<R>((R)P.XCOLEXIH * (t - (R)P.XTT)));
+        S.rh_ridryh = S.rh_riweth * ((R)P.XCOLIH * stick);
       }
     } else {
       S.rh_riweth = 0; S.rh_ridryh = 0;
@@ -986,8 +1023,8 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
                                          (R)P.XWETINTP2H, (R)P.XWETINTP1S, (R)P.XWETINTP2S);
       const R zzw = interp2d<R>(ix, P.NWETLBDAH, htab + (ICE3_T_SWETH - ICE3_T_ICE3));
       S.rh_rsweth = (R)P.XFSWETH * zzw * lbs_cxs_bs * lbh_cxh * pc.rhom *
-                    ((R)P.XLBSWETH1 / (sq(lbdah)) + (R)P.XLBSWETH2 / (lbdah * lbdas) + (R)P.XLBSWETH3 / (sq(lbdas)));
-      S.rh_rsdryh = S.rh_rsweth * ((R)P.XCOLSH * rexp<R>((R)P.XCOLEXSH * (t - (R)P.XTT)));
+                    ((R)P.XLBSWETH1 / by(sq(lbdah)) + (R)P.XLBSWETH2 / by(lbdah * lbdas) + (R)P.XLBSWETH3 / by(sq(lbdas)));
+      S.rh_rsdryh = S.rh_rsweth * ((R)P.XCOLSH * stick);
     }
     if (!(rh_ok && rg_ok)) { S.rh_rgweth = 0; S.rh_rgdryh = 0; }
     if (!soft && rh_ok && rg_ok) {
@@ -995,10 +1032,10 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
                                          (R)P.XWETINTP2H, (R)P.XWETINTP1G, (R)P.XWETINTP2G);
       const R zzw = interp2d<R>(ix, P.NWETLBDAH, htab + (ICE3_T_GWETH - ICE3_T_ICE3));
       S.rh_rgweth = (R)P.XFGWETH * zzw * powl_<R>(llg, (R)(P.XCXG - P.XBG)) * lbh_cxh * pc.rhom *
-                    ((R)P.XLBGWETH1 / (sq(lbdah)) + (R)P.XLBGWETH2 / (lbdah * lbdag) + (R)P.XLBGWETH3 / (sq(lbdag)));
+                    ((R)P.XLBGWETH1 / by(sq(lbdah)) + (R)P.XLBGWETH2 / by(lbdah * lbdag) + (R)P.XLBGWETH3 / by(sq(lbdag)));
       S.rh_rgdryh = S.rh_rgweth;
       // wet graupel keeps its collection efficiency (:221-223)
-      if (!ldwetg) S.rh_rgdryh = S.rh_rgdryh * ((R)P.XCOLGH * rexp<R>((R)P.XCOLEXGH * (t - (R)P.XTT)));
+      if (!ldwetg) S.rh_rgdryh = S.rh_rgdryh * ((R)P.XCOLGH * stick);
     }
     if (!(rh_ok && rr_ok)) S.rh_rrweth = 0;
     if (!soft && rh_ok && rr_ok) {
@@ -1006,20 +1043,16 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
                                          (R)P.XWETINTP2H, (R)P.XWETINTP1R, (R)P.XWETINTP2R);
       const R zzw = interp2d<R>(ix, P.NWETLBDAH, htab + (ICE3_T_RWETH - ICE3_T_ICE3));
       const R lr2 = lbdar * lbdar;
-      S.rh_rrweth = (R)P.XFRWETH * zzw * ((R)1.0 / (lr2 * lr2)) * lbh_cxh * pc.rhom *
-                    ((R)P.XLBRWETH1 / (sq(lbdah)) + (R)P.XLBRWETH2 / (lbdah * lbdar) + (R)P.XLBRWETH3 / (lr2));
+      S.rh_rrweth = (R)P.XFRWETH * zzw * ((R)1.0 / by(lr2 * lr2)) * lbh_cxh * pc.rhom *
+                    ((R)P.XLBRWETH1 / by(sq(lbdah)) + (R)P.XLBRWETH2 / by(lbdah * lbdar) + (R)P.XLBRWETH3 / by(lr2));
     }
     const R rdryh_init = S.rh_rcweth + S.rh_ridryh + S.rh_rsdryh + S.rh_rrweth + S.rh_rgdryh;
     R rweth_init = 0;
     bool llweth = false, lldryh = false;
     if (rh_ok) {
       if (!soft) {
-        R f1 = rv * (R)pres / ((R)P.XEPSILO + rv);
-        f1 = dmin(f1, esi);
-        f1 = ka * ((R)P.XTT - t) + (dv * ((R)P.XLVTT + (R)(P.XCPV - P.XCL) * (t - (R)P.XTT)) * ((R)P.XESTT - f1) / ((R)P.XRV * t));
-        f1 = f1 * vent_h / (rho * ((R)P.XLMTT - (R)P.XCL * ((R)P.XTT - t)));
-        S.rh_freez1 = f1;
-        S.rh_freez2 = (rho * ((R)P.XLMTT + (R)(P.XCI - P.XCL) * ((R)P.XTT - t))) / (rho * ((R)P.XLMTT - (R)P.XCL * ((R)P.XTT - t)));
+        S.rh_freez1 = heat_i * vent_h / freez_den;
+        S.rh_freez2 = freez_eff;
       }
       const R isg = S.rh_riweth + S.rh_rsweth + S.rh_rgweth;
       rweth_init = dmax(isg, dmax((R)0., S.rh_freez1 + S.rh_freez2 * isg));
@@ -1039,18 +1072,15 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
     if (lldryh) {
       rcdryh = S.rh_rcweth; ridryh = S.rh_ridryh; rsdryh = S.rh_rsdryh; rrdryh = S.rh_rrweth;
       rgdryh = S.rh_rgdryh;
-      rdryhg = rdryh_init * rweth_init / (rdryh_init + rweth_init);
+      rdryhg = rdryh_init * rweth_init / by(rdryh_init + rweth_init);
     }
     if (br)
       *br |= (llweth ? 1u << ICE3_BR_WETH : 0u) | (lldryh ? 1u << ICE3_BR_DRYH : 0u) |
              (rdryhg > (R)0 ? 1u << ICE3_BR_DRYHG : 0u);
     if (rh_ok && warm) {
       if (!soft) {
-        R m = rv * (R)pres / ((R)P.XEPSILO + rv);
-        m = dmin(m, esw);
-        m = ka * ((R)P.XTT - t) + dv * ((R)P.XLVTT + (R)(P.XCPV - P.XCL) * (t - (R)P.XTT)) * ((R)P.XESTT - m) / ((R)P.XRV * t);
-        S.rhmltr = dmax((R)0., (-m * vent_h - (S.rh_rcweth + S.rh_rrweth) * (rho * (R)P.XCL * ((R)P.XTT - t))) /
-                                   (rho * (R)P.XLMTT));
+        S.rhmltr = dmax((R)0., (-heat_w * vent_h - (S.rh_rcweth + S.rh_rrweth) * (rho * (R)P.XCL * ((R)P.XTT - t))) /
+                                   by(rho * (R)P.XLMTT));
       }
     } else S.rhmltr = 0;
   }
@@ -1060,7 +1090,7 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
     S.rcberi = 0;
   } else if (ssi > (R)0. && rc_ok && ri_ok && cit > 1.E-20) {
     if (!soft) {
-      R lli = (R)P.LN_XLBI + (R)P.XLBEXI * rlog<R>(rho * ri / (R)cit);
+      R lli = (R)P.LN_XLBI + (R)P.XLBEXI * rlog<R>(rho * ri / by((R)cit));
       R l;
       if (lli < (R)P.LN_1E8) {
         l = rexp<R>(lli);
@@ -1068,7 +1098,7 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
         l = (R)1.E8;
         lli = (R)P.LN_1E8;
       }
-      S.rcberi = (ssi / (rho * ai)) * (R)cit * ((R)P.X0DEPI / l + (R)P.X2DEPI * cj * cj / powl_<R>(lli, (R)(P.XDI + 2.0)));
+      S.rcberi = dep * (R)cit * ((R)P.X0DEPI / by(l) + (R)P.X2DEPI * cj * cj / by(powl_<R>(lli, (R)(P.XDI + 2.0))));
     }
   } else S.rcberi = 0;
 
@@ -1080,17 +1110,17 @@ __device__ __forceinline__ void tendencies(bool soft, double exn, double rhodref
     if (!soft) {
       const double ztimesc = P.XFRMIN[14], zdicrit = P.XFRMIN[15], zwcitred = 0.1;
       const double ri_d = zv[IRI], ssi_d = (double)ssi, ai_d = (double)ai;
-      if (ri_d > 0.0 && ssi_d > 0.001) rilars = dmin(ri_d, ri_d / (87.5 * sq(zdicrit) * ai_d / ssi_d));
+      if (ri_d > 0.0 && ssi_d > 0.001) rilars = dmin(ri_d, ri_d / by(87.5 * sq(zdicrit) * ai_d / by(ssi_d)));
       if ((pres * 0.5 - esi_tab) > 0. && cit > 0.) {
-        const double zw2d = 1. / (x->ifr * x->icldfr + 1. - x->icldfr);
+        const double zw2d = 1. / by(x->ifr * x->icldfr + 1. - x->icldfr);
         const double ztc = dmax(-18., dmin(-1., zt - P.XTT));
         const double zhu = dmin(0.15, dmax(0., ssi_d));
         const double zcrysha = 1.1 + 3. * zhu * (1. + sin(0.64 * ztc - 1.3));
-        const double zqimax = 366.5 * (zdicrit * zdicrit * zdicrit) * cit * zwcitred / rhodref;
+        const double zqimax = 366.5 * (zdicrit * zdicrit * zdicrit) * cit * zwcitred / by(rhodref);
         double zci2s = 0.;
         if (ri_d > 1.0e-12 && ztimesc > 0.)
-          zci2s = ri_d * (1. - dmin(1., 0.5 * zqimax / ri_d)) * (1. - x->icldfr) * zw2d / (ztimesc * 0.5);
-        const double zzwc = zcrysha * 0.878 / ai_d * rpow<double>(cit / rhodref, 0.667) *
+          zci2s = ri_d * (1. - dmin(1., 0.5 * zqimax / by(ri_d))) * (1. - x->icldfr) * zw2d / by(ztimesc * 0.5);
+        const double zzwc = zcrysha * 0.878 / by(ai_d) * rpow<double>(cit / by(rhodref), 0.667) *
                             rpow<double>(dmax(P.XRTMIN[4], ri_d) * zw2d, 0.333);
         if (x->ssio > 0. && x->icldfr > 0.02)
           rvdepi = rvdepi + zzwc * rpow<double>(x->ifr, 0.333) * x->ssio * x->icldfr;
@@ -1259,7 +1289,7 @@ template <int NV>
 __device__ __forceinline__ void step_point(double dt, double exn, double rhodref, double pres,
                                            double cf, double sigs, const double *s,
                                            const double *vart, StepPointN<NV> &p) {
-  const double zinv = 1. / dt;
+  const double zinv = 1. / by(dt);
   p.exn = exn; p.rhodref = rhodref; p.pres = pres; p.cf = cf; p.sigma_rc = sigs * 2.;
 #pragma unroll
   for (int jv = 0; jv < NV; ++jv) p.extpk[jv] = s[jv] - vart[jv] * zinv;
@@ -1296,24 +1326,24 @@ __device__ __forceinline__ int step_call(double dt, const StepPointN<NV> &p, con
   const double zdevide =
       (P.XCPD + P.XCPV * vart[IRV] + P.XCL * (vart[IRC] + vart[IRR]) + P.XCI * sum2) * exn;
   const double zzt = vart[ITH] * exn;
-  const double lsfact = (P.XLSTT + (P.XCPV - P.XCI) * (zzt - P.XTT)) / zdevide;
-  const double lvfact = (P.XLVTT + (P.XCPV - P.XCL) * (zzt - P.XTT)) / zdevide;
-  tendencies<R, OCND2, HAIL>(SOFT, exn, p.rhodref, lvfact, lsfact, p.pres, p.cf, p.sigma_rc, cit,
+  const double lsfact = (P.XLSTT + (P.XCPV - P.XCI) * (zzt - P.XTT)) / by(zdevide);
+  const double lvfact = (P.XLVTT + (P.XCPV - P.XCL) * (zzt - P.XTT)) / by(zdevide);
+  const double zx = P.XTT / by(exn);
+  tendencies<R, OCND2, HAIL>(SOFT, exn, zx, p.rhodref, lvfact, lsfact, p.pres, p.cf, p.sigma_rc, cit,
                              zzt, vart, S, pc, tab, za, zb, x, htab, br);
 #pragma unroll
   for (int jv = 0; jv < NV; ++jv) za[jv] = za[jv] + p.extpk[jv];
   const double time = time_;
   double maxtime = dt - time;
-  const double zx = P.XTT / exn;
   if ((vart[ITH] - zx) * (vart[ITH] + zb[ITH] - zx) < 0.) maxtime = 0.;
   if (fabs(za[ITH]) > 1.E-20) {
-    const double tth = (zx - zb[ITH] - vart[ITH]) / za[ITH];
+    const double tth = (zx - zb[ITH] - vart[ITH]) / by(za[ITH]);
     if (tth > 0.) maxtime = dmin(maxtime, tth);
   }
 #pragma unroll
   for (int jv = 1; jv < NV; ++jv)
     if (za[jv] < -1.E-20 && vart[jv] > P.XRTMIN[jv]) {
-      maxtime = dmin(maxtime, -(zb[jv] + vart[jv]) / za[jv]);
+      maxtime = dmin(maxtime, -(zb[jv] + vart[jv]) / by(za[jv]));
       maxtime = dmax(maxtime, P.XMNH_TINY);
     }
   const bool done = time + maxtime >= dt;
@@ -1400,7 +1430,7 @@ __device__ __forceinline__ void sediment_through(const FallLaw<R> &law, double d
   double cur = f1;
   if (qp > law.thr) {
     const double w2 = (double)fall_speed_above<R>(law, qp, lnrho, rhoc);
-    if (w2 != 0.) cur = f1 + dmax(0., 1. - dz / (dt * w2)) * flux;
+    if (w2 != 0.) cur = f1 + dmax(0., 1. - dz / by(dt * w2)) * flux;
   }
   rs = rs + tsorhodz * (flux - cur) * zinv;
   flux = cur;
@@ -1413,11 +1443,11 @@ template <class R>
 __device__ __forceinline__ void sediment_species(int jrr, double dt, double rho, R lnrho, double dz,
                                                  double &rs, double &flux) {
   const FallLaw<R> law = fall_law<R>(jrr);
-  const double zinv = 1. / dt;
+  const double zinv = 1. / by(dt);
   const double rx = rs * dt;
   const R rhoc = law.ice ? fall_rhoc<R>(lnrho) : (R)0;
   const double w1 = rx > law.thr ? (double)fall_speed_above<R>(law, rx, lnrho, rhoc) : 0.;
-  sediment_through<R>(law, dt, zinv, lnrho, rhoc, dz, dt / (rho * dz),
+  sediment_through<R>(law, dt, zinv, lnrho, rhoc, dz, dt / by(rho * dz),
                       sediment_own(zinv, rho, dz, rx, w1), rs, flux);
 }
 

@@ -49,7 +49,7 @@ __global__ void __launch_bounds__(128 * (HAIL ? 5 : 4)) k_sedim(SedimArgs a) {
                          : sp == 2 ? fall_law<R>(5)
                          : sp == 3 ? fall_law<R>(6)
                                    : fall_law<R>(7);
-  const double dt = a.dt, zinv = 1. / dt;
+  const double dt = a.dt, zinv = 1. / by(dt);
   const int top = a.nlev - 1, ng = (a.nlev + SG - 1) / SG;
   // levels below the ground are read as level 0 and not used
   auto at = [&](int k) { return (size_t)(k > 0 ? k : 0) * a.ld + i; };
@@ -68,7 +68,7 @@ __global__ void __launch_bounds__(128 * (HAIL ? 5 : 4)) k_sedim(SedimArgs a) {
     sDz[b][w][lane] = dz;
     sLn[b][w][lane] = ln;
     sRhoc[b][w][lane] = fall_rhoc<R>(ln);
-    sTs[b][w][lane] = dt / (rho * dz);
+    sTs[b][w][lane] = dt / by(rho * dz);
   };
   if (ZZZ && w == 3) sZz[lane] = 0.;  // read by this wavefront only
   load_src(0);
@@ -134,7 +134,7 @@ __global__ void __launch_bounds__(128 * (HAIL ? 5 : 4)) k_sedim(SedimArgs a) {
     __syncthreads();
     b = bn;
   }
-  const double rate = flux / P.XRHOLW;
+  const double rate = flux / by(P.XRHOLW);
   if (!own && sp == 1) sFi[lane] = rate;
   __syncthreads();
   if (!in || own) return;

@@ -155,11 +155,11 @@ __device__ __forceinline__ void sedim_column(const SedimArgs &a, int i) {
     }
   }
   a.inprc[i] = 0.;
-  a.inprr[i] = fr / P.XRHOLW;
-  a.inpri[i] = fi / P.XRHOLW;
-  a.inprs[i] = fs / P.XRHOLW + fi / P.XRHOLW;
-  a.inprg[i] = fg / P.XRHOLW;
-  if constexpr (HAIL) a.inprh[i] = fh / P.XRHOLW;
+  a.inprr[i] = fr / by(P.XRHOLW);
+  a.inpri[i] = fi / by(P.XRHOLW);
+  a.inprs[i] = fs / by(P.XRHOLW) + fi / by(P.XRHOLW);
+  a.inprg[i] = fg / by(P.XRHOLW);
+  if constexpr (HAIL) a.inprh[i] = fh / by(P.XRHOLW);
 }
 
 // ICE_ADJUST and the sedimentation of column i in one top-down walk (the FP64 fused step):
@@ -189,11 +189,11 @@ __device__ __forceinline__ void adjust_sedim_column(const AdjustArgs &aa, const 
     }
   }
   a.inprc[i] = 0.;
-  a.inprr[i] = fr / P.XRHOLW;
-  a.inpri[i] = fi / P.XRHOLW;
-  a.inprs[i] = fs / P.XRHOLW + fi / P.XRHOLW;
-  a.inprg[i] = fg / P.XRHOLW;
-  if constexpr (HAIL) a.inprh[i] = fh / P.XRHOLW;
+  a.inprr[i] = fr / by(P.XRHOLW);
+  a.inpri[i] = fi / by(P.XRHOLW);
+  a.inprs[i] = fs / by(P.XRHOLW) + fi / by(P.XRHOLW);
+  a.inprg[i] = fg / by(P.XRHOLW);
+  if constexpr (HAIL) a.inprh[i] = fh / by(P.XRHOLW);
 }
 
 // Microphysics stage arguments.  The t-state of species v is t[v][j] * tscale
@@ -240,7 +240,7 @@ __device__ __forceinline__ void correct_negativities(double &ths, double &rvs, d
   if constexpr (HAIL) {
     zw = *rhs - dmax(*rhs, 0.); rvs = rvs + zw; ths = ths - zw * lsfact; *rhs = *rhs - zw;
   }
-  zw = dmin(1., dmax(P.XRTMIN[1] - rvs, 0.) / dmax(rcs + ris, 1.E-20));
+  zw = dmin(1., dmax(P.XRTMIN[1] - rvs, 0.) / by(dmax(rcs + ris, 1.E-20)));
   ths = ths - zw * (rcs * lvfact + ris * lsfact);
   rvs = rvs + zw * (rcs + ris);
   rcs = (1. - zw) * rcs;
@@ -276,8 +276,8 @@ __device__ __forceinline__ void rain_ice_factors(const double *t, double exn, do
   if constexpr (HAIL) zrice = zrice + t[IRH];
   const double zdevide = P.XCPD + P.XCPV * t[IRV] + P.XCL * (t[IRC] + t[IRR]) + P.XCI * zrice;
   const double zt = t[ITH] * exn;
-  lsfact = (P.XLSTT + (P.XCPV - P.XCI) * (zt - P.XTT)) / zdevide;
-  lvfact = (P.XLVTT + (P.XCPV - P.XCL) * (zt - P.XTT)) / zdevide;
+  lsfact = (P.XLSTT + (P.XCPV - P.XCI) * (zt - P.XTT)) / by(zdevide);
+  lvfact = (P.XLVTT + (P.XCPV - P.XCL) * (zt - P.XTT)) / by(zdevide);
 }
 
 // RAIN_ICE's microphysics mask (micro/rain_ice.F90:365-381): a hydrometeor above XRTMIN;
@@ -311,7 +311,7 @@ __device__ __forceinline__ void micro_nucleation(const MicroArgs &a, size_t j, c
   cit = 0.;
   MicroOcnd2 x;
   if constexpr (OCND2) x = ocnd2_point(a, j);
-  nucleation<R, OCND2>(true, t[ITH], a.pabs[j], a.rhodref[j], exn, lsfact / exn, t[ITH] * exn,
+  nucleation<R, OCND2>(true, t[ITH], a.pabs[j], a.rhodref[j], P.XTT / by(exn), lsfact / by(exn), t[ITH] * exn,
                        t[IRV], cit, rvheni, &x);
 }
 
@@ -324,16 +324,16 @@ template <bool HAIL = false>
 __device__ __forceinline__ void micro_finish(const MicroArgs &a, size_t j, const double *wr,
                                              double cit, double evap3d, double rvheni, int calls) {
   constexpr int NV = HAIL ? 8 : 7;
-  const double dt = a.dt, zinv = 1. / dt;
+  const double dt = a.dt, zinv = 1. / by(dt);
   double t[NV], s[NV];
   micro_load<NV>(a, j, t, s);
   double lsfact, lvfact;
   rain_ice_factors<HAIL>(t, a.exn[j], lsfact, lvfact);
-  rvheni = dmin(s[IRV], rvheni / dt);
+  rvheni = dmin(s[IRV], rvheni / by(dt));
   // 8.1 total tendencies
   const double exnref = a.exn_ref[j];
-  lsfact = lsfact / exnref;
-  lvfact = lvfact / exnref;
+  lsfact = lsfact / by(exnref);
+  lvfact = lvfact / by(exnref);
   const double wrv = (wr[IRV] - t[IRV]) * zinv, wrc = (wr[IRC] - t[IRC]) * zinv;
   const double wrr = (wr[IRR] - t[IRR]) * zinv, wri = (wr[IRI] - t[IRI]) * zinv;
   const double wrs = (wr[IRS] - t[IRS]) * zinv, wrg = (wr[IRG] - t[IRG]) * zinv;
@@ -417,8 +417,8 @@ __device__ __forceinline__ void latent_factors(const MicroArgs &a, size_t j, dou
   double t[7], s[7];
   micro_load(a, j, t, s);
   rain_ice_factors(t, a.exn[j], lsfact, lvfact);
-  lsfact = lsfact / a.exn_ref[j];
-  lvfact = lvfact / a.exn_ref[j];
+  lsfact = lsfact / by(a.exn_ref[j]);
+  lvfact = lvfact / by(a.exn_ref[j]);
 }
 
 // ---------------------------------------------------------------- argument set-up
