@@ -447,7 +447,7 @@ def hail_step(lib, ctx, dev, g, cin, sp, stream, args, outputs, stage_times_of, 
     return {"columns_per_s": ncol / (ms * 1e-3), "ms_per_step": ms, "speedup_vs_stat_krr6": ms_stat / ms,
             "stages_ms": stages, "water_budget_max_rel_err": budget,
             "note": "fused step with KRR=7: k_adjust_sedim_hail (column walk), then the hail "
-                    "microphysics k_micro<double, false, HAIL> (persistent, one wavefront per SIMD)"}
+                    "microphysics k_micro<double, false, HAIL> (persistent, two wavefronts per SIMD)"}
 
 
 def timed_steps(fn, stream, steps, warmup):

@@ -13,7 +13,7 @@
 //                  precipitation, a wavefront per 64 columns and species;
 //   k_micro<R>     persistent, one workgroup per compute unit, lookup tables in LDS:
 //                  the ICE4 time-split microphysics, total tendencies and negativity
-//                  correction per point, with the points still being time-stepped
+//                  correction per point, with the points of long time splittings
 //                  compacted into full wavefronts (ballot, LDS parking);
 //   k_sg_features, k_mlp_infer, k_sg_decode
 //                  the learned surrogate of k_micro: features and range check per point;
@@ -491,21 +491,25 @@ __global__ void __launch_bounds__(64 * SPLIT_COLS)
 // Every point makes one hard tendency call, and 42 % of them (on the 512x512x90 synthetic
 // workload) then make soft calls, most of them one, a few up to five.  Run one point per
 // lane to the end and a wavefront makes as many soft passes as its slowest lane needs,
-// nearly all with few lanes active.  Here a wavefront takes 64-point chunks in turn; after
-// the chunk's hard call, the lanes whose time step goes on are joined by points parked in
-// LDS by earlier chunks, and a soft pass runs over a full wavefront (64 points) whenever
-// that many are at hand, or over more than MicroPark::CAP points when the park would
-// otherwise overflow; unfinished points are parked again (ballot + prefix count give
-// each its slot).  The per-point arithmetic is that of micro_at, only the order in which
-// points are advanced differs, so the results are those of one thread per point.
-// Eight wavefronts per workgroup, two per SIMD: the register budget of 256 per wavefront
-// costs a few spills (FP64), but the second wavefront hides the memory latency the first
-// one waits on.  The workgroup's wavefronts share the lookup tables, staged once into LDS.
-// Wavefronts per workgroup.  The mixed path (183 VGPRs at two wavefronts per SIMD) measured
-// slower with three (168 VGPRs, spills, 49-slot parks: +22 %) or four (+120 %) per SIMD.
-// The hail state needs about 306 registers: one wavefront per SIMD (at two, 55 registers
-// spill and the kernel is slower than one thread per point), with 49-slot parks.
-template <class R, bool HAIL = false> constexpr int micro_waves() { return HAIL ? 4 : 8; }
+// nearly all with few lanes active.  Here a wavefront takes 64-point chunks in turn: the hard
+// call of all of them, one soft pass over those whose time step goes on, and the stores of
+// every point that is then complete (94 %), while the chunk's state is in registers and its
+// lines are in the caches.  The few left over are parked in LDS; a soft pass over parked
+// points runs when 64 are at hand, or when the park (MicroPark::CAP) would otherwise overflow
+// (ballot + prefix count give each its slot).  The per-point arithmetic is that of micro_at,
+// only the order in which points are advanced differs, so the results are those of one thread
+// per point.
+//
+// What bounds it: the latency that the wavefronts of a SIMD cannot cover for each other; the
+// FP64 VALU issues about two thirds of the cycles.  Parking every unfinished point after its
+// hard call, so that soft passes were full, read every input line and wrote every output line
+// twice (10 GB at 512x512x90 against 5.3 algorithmic), as their lines had left the L2 by then:
+// 2.79 ms in FP64, 2.40 mixed, 3.57 with OCND2, against 2.72, 1.88 and 3.37 now.
+//
+// Wavefronts per workgroup (one workgroup a compute unit).  FP64: two per SIMD, 231 of 256
+// VGPRs.  Mixed: three per SIMD (163 of 168 VGPRs; two per SIMD: 2.17 ms).  Hail: two per SIMD
+// (256 VGPRs and a few spills: 3.33 ms; one per SIMD: 4.74).
+template <class R, bool HAIL = false> constexpr int micro_waves() { return sizeof(R) == 4 ? 12 : 8; }
 // Lookup tables staged in LDS: the ICE3 block; the hail kernel reads the wet-growth kernels
 // of hail, which follow it, from device memory.
 template <class R, bool HAIL = false> constexpr size_t micro_tab_bytes() {
@@ -517,7 +521,7 @@ template <class R, bool HAIL> constexpr int micro_ns() {
   return (int)(sizeof(typename StepStateFor<R, HAIL>::type) / sizeof(R));
 }
 // Park slots per wavefront: what the LDS holds beside the tables, at most 63 (31 in FP64,
-// 63 in the mixed path, 49 with hail).
+// 49 in the mixed path, 24 with hail).
 template <class R, bool HAIL = false> constexpr int micro_park_cap() {
   const size_t slot = (micro_nv<HAIL>() + 2) * sizeof(double) + micro_ns<R, HAIL>() * sizeof(R) +
                       2 * sizeof(int);
@@ -542,8 +546,9 @@ static_assert(sizeof(StepStateHail<double>) == 43 * sizeof(double), "StepStateHa
 template <class R, bool HAIL = false> constexpr size_t micro_lds_bytes() {
   return micro_tab_bytes<R, HAIL>() + micro_waves<R, HAIL>() * sizeof(MicroPark<R, HAIL>);
 }
-static_assert(MicroPark<double>::CAP == 31 && MicroPark<float>::CAP == 63 &&
-              MicroPark<double, true>::CAP == 49, "park capacity");
+static_assert(MicroPark<double>::CAP == 31 && MicroPark<float>::CAP == 49 &&
+              MicroPark<double, true>::CAP == 24, "park capacity");
+static_assert(ICE3_T_ICE3 % 2 == 0, "k_micro stages the tables by pairs");
 static_assert(micro_lds_bytes<double>() <= 160 * 1024, "k_micro<double> LDS");
 static_assert(micro_lds_bytes<float>() <= 160 * 1024, "k_micro<float> LDS");
 static_assert(micro_lds_bytes<double, true>() <= 160 * 1024, "k_micro<double, false, true> LDS");
@@ -584,11 +589,31 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
   extern __shared__ __align__(16) unsigned char micro_lds[];
   constexpr int NV = micro_nv<HAIL>();
   R *tab = reinterpret_cast<R *>(micro_lds);
-  for (int e = threadIdx.x; e < ICE3_T_ICE3; e += blockDim.x) tab[e] = (R)a.tab[e];
+  // the tables, every load issued before the first store (a load and a store at a time take 8 us
+  // longer, a fifth of the call on 1,024 columns)
+  {
+    constexpr int NT = 64 * micro_waves<R, HAIL>(), N2 = ICE3_T_ICE3 / 2, NL = (N2 + NT - 1) / NT;
+    typedef double f64x2 __attribute__((ext_vector_type(2)));
+    const f64x2 *src = (const f64x2 *)a.tab;
+    f64x2 v[NL];
+#pragma unroll
+    for (int b = 0; b < NL; ++b) {
+      const int e = threadIdx.x + b * NT;
+      v[b] = src[e < N2 ? e : 0];
+    }
+#pragma unroll
+    for (int b = 0; b < NL; ++b) {
+      const int e = threadIdx.x + b * NT;
+      if (e < N2) {
+        tab[2 * e] = (R)v[b][0];
+        tab[2 * e + 1] = (R)v[b][1];
+      }
+    }
+  }
   __syncthreads();
   // hail: the wet-growth kernels of hail from device memory
   const double *htab = HAIL ? a.tab + ICE3_T_ICE3 : nullptr;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   MicroPark<R, HAIL> &pk =
       reinterpret_cast<MicroPark<R, HAIL> *>(micro_lds + micro_tab_bytes<R, HAIL>())[wid];
   const unsigned long long below = (1ull << lane) - 1ull;  // lanes under this one
@@ -605,7 +630,15 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
   typename StepStateFor<R, HAIL>::type S;
   int calls = 0;
   unsigned long long ncalls = 0, ncap = 0, nmicro = 0;
-  for (int c = blockIdx.x * micro_waves<R, HAIL>() + wid;; c += gridDim.x * micro_waves<R, HAIL>()) {
+  bool done = false;              // this lane holds a point's end state, to be stored
+  double evap3d = 0., rvheni = 0.;
+  // Few chunks go one to a compute unit before a second to any (1,024 columns: 27.7 us, 35.0 with
+  // eight in a row to each); many go in rows of a workgroup's wavefronts, whose chunks are then
+  // neighbours (mixed path at 512x512x90: 1.88 ms, 1.93 the other way; FP64 the same).
+  const int cstep = gridDim.x * micro_waves<R, HAIL>();
+  const int c0 = nchunk < 4 * cstep ? wid * (int)gridDim.x + (int)blockIdx.x
+                                    : (int)blockIdx.x * micro_waves<R, HAIL>() + wid;
+  for (int c = c0;; c += cstep) {
     const bool more = c < nchunk;  // wave-uniform
     if (more) {
       const int k = c / cpl, i = (c - k * cpl) * 64 + lane;
@@ -615,7 +648,8 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
         double t[NV], s[NV];
         micro_load<NV>(a, j, t, s);
         cit = a.src_ci[j];
-        double rvheni = 0., evap3d = 0.;
+        rvheni = 0.;
+        evap3d = 0.;
         int st = 0;
         calls = 0;
         if (micro_mask<OCND2, HAIL>(t, a, j)) {
@@ -635,44 +669,52 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
 #pragma unroll
           for (int f = 0; f < NV; ++f) vart[f] = t[f];
         }
-        if (st > 0) {
-          active = true;
-        } else {
-          ncalls += calls;
-          ncap += st < 0;
-          micro_finish<HAIL>(a, j, vart, cit, evap3d, rvheni, st < 0 ? -calls : calls);
-        }
+        active = st > 0;
+        done = !active;
+        ncap += st < 0;
+        if (st < 0) calls = -calls;
       }
     }
-    // soft passes: over a full wavefront while 64 points are at hand, over all of them
-    // while they would not fit the park, and over all of them once the chunks are done
-    for (;;) {
+    // After the chunk's hard call (own): a soft pass over its own unfinished lanes, then the
+    // stores of every finished one.  Then soft passes joined by parked points: over a full
+    // wavefront while 64 points are at hand, over all of them while they would not fit the park,
+    // and over all of them once the chunks are done.
+#pragma clang loop unroll(disable)
+    for (bool own = more;; own = false) {
       const unsigned long long am = __ballot(active);
       const int nact = __popcll(am), need = 64 - nact;
-      if (more ? parked < need && nact + parked <= MicroPark<R, HAIL>::CAP : nact + parked == 0) break;
-      if (!active) {
-        const int r = __popcll(~am & below);  // rank among the idle lanes
-        if (r < parked) {
-          q = park_load(pk, parked - 1 - r, vart, cit, time, S, calls);
-          const unsigned int k = q / (unsigned int)a.ncol;
-          j = (size_t)k * a.ld + (q - k * (unsigned int)a.ncol);
-          double t[NV], s[NV];
-          micro_load<NV>(a, j, t, s);
-          step_point(dt, a.exn[j], a.rhodref[j], a.pabs[j], a.cldfr[j], a.sigs[j], s, t, p);
-          active = true;
+      const bool pass = own ? nact != 0
+                            : (more ? parked >= need || nact + parked > MicroPark<R, HAIL>::CAP : nact + parked != 0);
+      if (!own && !pass) break;
+      if (!own) {
+        if (!active) {
+          const int r = __popcll(~am & below);  // rank among the idle lanes
+          if (r < parked) {
+            q = park_load(pk, parked - 1 - r, vart, cit, time, S, calls);
+            const unsigned int k = q / (unsigned int)a.ncol;
+            j = (size_t)k * a.ld + (q - k * (unsigned int)a.ncol);
+            double t[NV], s[NV];
+            micro_load<NV>(a, j, t, s);
+            step_point(dt, a.exn[j], a.rhodref[j], a.pabs[j], a.cldfr[j], a.sigs[j], s, t, p);
+            active = true;
+            rvheni = 0.;
+          }
         }
+        parked -= need < parked ? need : parked;
       }
-      parked -= need < parked ? need : parked;
-      if (active) {
+      if (pass && active) {
         const int st = step_call<R, true, OCND2, HAIL>(dt, p, pc_soft, vart, cit, time, S, calls,
                                                        DEFAULT_MAX_CALLS, tab, nullptr, htab);
-        if (st <= 0) {
-          ncalls += calls;
-          ncap += st < 0;
-          micro_finish<HAIL>(a, j, vart, cit, st == 0 ? (double)S.rrevav : 0., 0.,
-                             st < 0 ? -calls : calls);
-          active = false;
-        }
+        active = st > 0;
+        done = !active;
+        evap3d = st == 0 ? (double)S.rrevav : 0.;
+        ncap += st < 0;
+        if (st < 0) calls = -calls;
+      }
+      if (done) {
+        ncalls += calls < 0 ? -calls : calls;
+        micro_finish<HAIL>(a, j, vart, cit, evap3d, rvheni, calls);
+        done = false;
       }
     }
     if (!more) break;
@@ -1333,8 +1375,8 @@ extern "C" int ice3_ice_adjust_rows(ice3_ctx *ctx, int ncol, int nlev, double dt
   return ICE3_OK;
 }
 
-// Launch k_micro: one workgroup of eight wavefronts per compute unit (its LDS holds the
-// tables and the parked points, so one workgroup fits a CU).
+// Launch k_micro: one workgroup per compute unit (its LDS holds the tables and the parked
+// points, so one workgroup fits a CU).
 static hipError_t launch_micro(const ice3_ctx *ctx, int prec, const MicroArgs &m, hipStream_t s) {
   if (m.max_calls != DEFAULT_MAX_CALLS) {  // a context-set cap: the point kernel reads it
     const unsigned int npts = (unsigned int)m.nlev * (unsigned int)m.ncol;
