@@ -7,14 +7,17 @@
 //   k_mlp_backward  one tile per workgroup: dW = H^T dZ and dH = dZ W^T on the matrix
 //                   cores, SiLU derivative, bias gradients; one fp32 partial gradient per
 //                   workgroup (no atomics: the reduction is deterministic).
-//   k_mlp_reduce    sum of the partial gradients.
+//   k_mlp_gradient  both in one kernel, nothing saved between them (the training step).
+//   k_mlp_reduce    sum of the partial gradients (and losses).
 //   k_mlp_adam      Adam on the fp32 master parameters; rewrites the bf16 row-major and
 //                   packed-fragment copies the matrix cores read.
 //   k_mlp_infer     inference over all points of the surrogate step: persistent grid,
 //                   weights resident in LDS (launched by mlp_infer_launch).
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
 #include <cstring>
+#include <type_traits>
 
 #include "../../include/ice3.h"
 #include "ice3_mlp.hpp"
@@ -254,12 +257,297 @@ __global__ void __launch_bounds__(256) k_mlp_backward(MlpBwdArgs a) {
 
 constexpr size_t MLP_BWD_LDS = (size_t)4 * BW_TILE * 2;
 
-__global__ void __launch_bounds__(256) k_mlp_reduce(const float *gpart, int nblk, float *grad) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= MLP_NP) return;
+// ---- Forward and backward in one kernel, nothing saved to memory between them.
+// A workgroup takes a tile of 128 points, a wavefront 16 of them through every layer, activations
+// in registers as in k_mlp_infer, the pre-activations of the four hidden layers beside them
+// (fp32, 128 of 256 registers; the sigmoid is computed a second time rather than kept).  For
+// dW = H^T dZ the points are the contraction, so H and dZ of a layer go through LDS transposed;
+// dH = W dZ takes dZ from registers.  The backward tiles lie where the forward weights were, the
+// weights of a layer one layer ahead of their use.
+// 32,768 points (a tile for each compute unit), with the reduction: 54 us, against 208 us of
+// k_mlp_forward (34, with 100 MB of pre-activations and activations saved), k_mlp_backward (112)
+// and a serial sum of the partials (62).  Bound by the latency of its ten phases between
+// barriers at two wavefronts a SIMD, and the 59 MB of partials written and read.
+struct MlpGradArgs {
+  int npts;
+  const bf16x8 *wpk;      // packed bf16 weights
+  const __bf16 *wrm;      // row-major bf16 weights
+  const float *params;    // fp32 master parameters (biases at MLP_NW)
+  const __bf16 *x;        // [npts][MLP_IN]
+  const float *target;    // [npts][MLP_NTARG]
+  float *gpart;           // [gridDim.x][MLP_NP]
+  float *loss_part;       // [gridDim.x]
+  float inv_count;        // 1 / (npts * MLP_NTARG)
+};
+
+constexpr int GRAD_WAVES = MLP_TILE / 16, GRAD_THREADS = 64 * GRAD_WAVES;
+
+// v: bf16 units u0 .. u0+3 of point col (one point a lane, neighbouring lanes neighbouring points)
+// into the transposed tile s[unit][BW_S]; an even lane writes the pairs of the first two units,
+// an odd one those of the last two, every bank once.
+__device__ __forceinline__ void put_transposed(__bf16 *s, int u0, int col, const u32x2 &v) {
+  const bool odd = col & 1;
+  const unsigned int own = odd ? v[1] : v[0], send = odd ? v[0] : v[1];
+  const unsigned int got = __builtin_amdgcn_update_dpp(0u, send, 0xB1, 0xF, 0xF, true);  // lane ^ 1
+  const unsigned int lo = odd ? got : own, hi = odd ? own : got;
+  __bf16 *d = s + (u0 + (odd ? 2 : 0)) * BW_S + (col & ~1);
+  *(unsigned int *)d = (lo & 0xFFFFu) | (hi << 16);
+  *(unsigned int *)(d + BW_S) = (lo >> 16) | (hi & 0xFFFF0000u);
+}
+
+// W_L (row-major) to registers, and from there into its padded tile.
+template <int L> struct StagedW {
+  static constexpr int N = mlp_n(L), NQ = MLP_H * (N / 8) / GRAD_THREADS;
+  bf16x8 v[NQ];
+  __device__ __forceinline__ void load(const __bf16 *wrm) {
+#pragma unroll
+    for (int b = 0; b < NQ; ++b)
+      v[b] = *(const bf16x8 *)(wrm + mlp_woff(L) + (threadIdx.x + b * GRAD_THREADS) * 8);
+  }
+  __device__ __forceinline__ void store(__bf16 *sW) const {
+#pragma unroll
+    for (int b = 0; b < NQ; ++b) {
+      const int q = threadIdx.x + b * GRAD_THREADS;
+      *(bf16x8 *)(sW + (q / (N / 8)) * BW_S + (q % (N / 8)) * 8) = v[b];
+    }
+  }
+};
+
+// dW_L = H^T dZ and the bias gradient of a tile, to its partial: wavefront w's NT x KT output
+// tiles of 16 units of layer L by 16 of its input, from the transposed tiles.
+template <int L, int NT, int KT>
+__device__ __forceinline__ void grad_weights(float *gp, const __bf16 *sDZT, const __bf16 *sHT,
+                                             int n0, int k0, bool bias, int lane) {
+  constexpr int N = mlp_n(L);
+  const int pt = lane % 16, g = lane / 16;
+  f32x4 acc[NT][KT], sum[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    sum[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < KT; ++k) acc[n][k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  bf16x8 ones;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.f;
+#pragma unroll
+  for (int kk = 0; kk < MLP_TILE / 32; ++kk) {
+    bf16x8 dz[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      dz[n] = *(const bf16x8 *)(sDZT + (n0 + n * 16 + pt) * BW_S + kk * 32 + 8 * g);
+      if (bias) sum[n] = mfma_bf16(dz[n], ones, sum[n]);
+    }
+#pragma unroll
+    for (int k = 0; k < KT; ++k) {
+      const bf16x8 h = *(const bf16x8 *)(sHT + (k0 + k * 16 + pt) * BW_S + kk * 32 + 8 * g);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) acc[n][k] = mfma_bf16(dz[n], h, acc[n][k]);
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+#pragma unroll
+    for (int k = 0; k < KT; ++k)
+      *(f32x4 *)(gp + mlp_woff(L) + (k0 + k * 16 + pt) * N + n0 + n * 16 + 4 * g) = acc[n][k];
+    if (bias && pt == 0) *(f32x4 *)(gp + mlp_boff(L) + n0 + n * 16 + 4 * g) = sum[n];
+  }
+}
+
+__global__ void __launch_bounds__(GRAD_THREADS) k_mlp_gradient(MlpGradArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  bf16x8 *sWF = (bf16x8 *)smem;                   // forward: every layer's packed weights
+  __bf16 *sHT = (__bf16 *)smem;                   // backward, in their place: H^T,
+  __bf16 *sW0 = sHT + BW_TILE, *sW1 = sW0 + BW_TILE;  // and the weights of two layers
+  float *sB = (float *)(smem + MLP_NW * 2);       // biases
+  __bf16 *sDZT = (__bf16 *)(sB + MLP_NB);         // dZ^T
+  __shared__ float sLoss[GRAD_WAVES];
+  const int lane = threadIdx.x % 64, w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int pt = lane % 16, g = lane / 16;
+  const int col = w * 16 + pt, p = blockIdx.x * MLP_TILE + col;  // this lane's point
+  const bool live = p < a.npts;
+  float *gp = a.gpart + (size_t)blockIdx.x * MLP_NP;
+  bf16x8 x0[1][1];
+  if (live) x0[0][0] = *(const bf16x8 *)(a.x + (size_t)p * MLP_IN + 8 * g);
+  else x0[0][0] = bf16x8{};
+  float t[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    t[i] = live && 4 * g < MLP_NTARG ? a.target[(size_t)p * MLP_NTARG + 4 * g + i] : 0.f;
+  block_copy16(sWF, a.wpk, MLP_NW * 2);
+  for (int q = threadIdx.x; q < MLP_NB; q += blockDim.x) sB[q] = a.params[MLP_NW + q];
+  __syncthreads();
+
+  // forward
+  f32x4 z[4][MLP_H / 16];
+  u32x2 dz[MLP_H / 16];   // dZ of a layer, bf16, units 16 nn + 4 g .. +3
+  {
+    bf16x8 h[1][MLP_H / 32];
+    f32x4 acc[1][MLP_H / 16];
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+      if (l == 0) mlp_product<MLP_IN, MLP_H, MLP_H / 16, 1>(sWF, x0, acc, lane);
+      else mlp_product<MLP_H, MLP_H, MLP_H / 16, 1>(sWF + mlp_woff(l) / 8, h, acc, lane);
+      u32x2 v[MLP_H / 16];
+#pragma unroll
+      for (int nn = 0; nn < MLP_H / 16; ++nn) {
+        z[l][nn] = acc[0][nn] + *(const f32x4 *)(sB + l * MLP_H + nn * 16 + 4 * g);
+        v[nn] = pack4(silu(z[l][nn][0]), silu(z[l][nn][1]), silu(z[l][nn][2]), silu(z[l][nn][3]));
+        // opaque to the compiler, which would keep this sigmoid for the backward part (128 registers)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) asm("" : "+v"(z[l][nn][i]));
+      }
+#pragma unroll
+      for (int kk = 0; kk < MLP_H / 32; ++kk) h[0][kk] = operand_of(v[2 * kk], v[2 * kk + 1]);
+    }
+    f32x4 out[1][1];  // the first 16 of the padded outputs
+    mlp_product<MLP_H, 16, MLP_OUT / 16, 1>(sWF + mlp_woff(4) / 8, h, out, lane);
+    const f32x4 b = *(const f32x4 *)(sB + 4 * MLP_H + 4 * g);
+    float loss = 0.f, dy[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float d = out[0][0][i] + b[i] - t[i];
+      const bool used = live && 4 * g < MLP_NTARG;
+      loss += used ? d * d : 0.f;
+      dy[i] = used ? 2.f * d * a.inv_count : 0.f;
+    }
+    dz[0] = pack4(dy[0], dy[1], dy[2], dy[3]);
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) loss += __shfl_xor(loss, m, 64);
+    if (lane == 0) sLoss[w] = loss;
+  }
+
+  // backward: from the layer above's dZ (registers) and its weights, dZ of layer l
+  auto dz_below = [&](auto LC, const __bf16 *sW) {
+    constexpr int L = decltype(LC)::value, N = mlp_n(L);  // through W_L to layer L - 1
+    bf16x8 d[N / 32];
+#pragma unroll
+    for (int kk = 0; kk < N / 32; ++kk)
+      d[kk] = operand_of(dz[2 * kk], L == MLP_LAYERS - 1 ? u32x2{0u, 0u} : dz[2 * kk + 1]);
+    f32x4 acc[MLP_H / 16];
+#pragma unroll
+    for (int nn = 0; nn < MLP_H / 16; ++nn) acc[nn] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < N / 32; ++kk)
+#pragma unroll
+      for (int nn = 0; nn < MLP_H / 16; ++nn)
+        acc[nn] = mfma_bf16(*(const bf16x8 *)(sW + (nn * 16 + pt) * BW_S + kk * 32 + 8 * g), d[kk], acc[nn]);
+#pragma unroll
+    for (int nn = 0; nn < MLP_H / 16; ++nn) {
+      f32x4 v;  // z[L - 1] holds silu'(z) by now
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = live ? acc[nn][i] * z[L - 1][nn][i] : 0.f;
+      dz[nn] = pack4(v[0], v[1], v[2], v[3]);
+    }
+  };
+  auto put_dz = [&] {
+#pragma unroll
+    for (int nn = 0; nn < MLP_H / 16; ++nn) put_transposed(sDZT, nn * 16 + 4 * g, col, dz[nn]);
+  };
+  auto put_h = [&](f32x4 (&zl)[MLP_H / 16]) {  // H^T of a layer; its z becomes silu'(z)
+#pragma unroll
+    for (int nn = 0; nn < MLP_H / 16; ++nn) {
+      f32x4 h;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = zl[nn][i], s = sigmoid_fast(v);
+        h[i] = live ? v * s : 0.f;
+        zl[nn][i] = s * (1.f + v * (1.f - s));
+      }
+      put_transposed(sHT, nn * 16 + 4 * g, col, pack4(h[0], h[1], h[2], h[3]));
+    }
+  };
+  const int n2 = (w % 4) * 32, k4 = (w / 4) * 64;  // this wavefront's 2 x 4 tiles of a hidden layer
+  StagedW<4> w4;
+  StagedW<3> w3;
+  w4.load(a.wrm);
+  w3.load(a.wrm);
+  __syncthreads();  // the forward weights are read
+  if (threadIdx.x == 0) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < GRAD_WAVES; ++i) s += sLoss[i];
+    a.loss_part[blockIdx.x] = s;
+  }
+  w4.store(sW0);
+  w3.store(sW1);
+  put_h(z[3]);
+  put_transposed(sDZT, 4 * g, col, dz[0]);
+  __syncthreads();
+  // the outputs: 16 of 32 columns, the others' gradients are zero
+  grad_weights<4, 1, 1>(gp, sDZT, sHT, 0, w * 16, w == 0, lane);
+  *(f32x4 *)(gp + mlp_woff(4) + (w * 16 + pt) * MLP_OUT + 16 + 4 * g) = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (threadIdx.x < 16) gp[mlp_boff(4) + 16 + threadIdx.x] = 0.f;
+  StagedW<2> w2;
+  w2.load(a.wrm);
+  dz_below(std::integral_constant<int, 4>{}, sW0);
+  __syncthreads();
+  put_dz();
+  put_h(z[2]);
+  w2.store(sW0);
+  __syncthreads();
+  grad_weights<3, 2, 4>(gp, sDZT, sHT, n2, k4, k4 == 0, lane);
+  StagedW<1> w1;
+  w1.load(a.wrm);
+  dz_below(std::integral_constant<int, 3>{}, sW1);
+  __syncthreads();
+  put_dz();
+  put_h(z[1]);
+  w1.store(sW1);
+  __syncthreads();
+  grad_weights<2, 2, 4>(gp, sDZT, sHT, n2, k4, k4 == 0, lane);
+  dz_below(std::integral_constant<int, 2>{}, sW0);
+  __syncthreads();
+  put_dz();
+  put_h(z[0]);
+  __syncthreads();
+  grad_weights<1, 2, 4>(gp, sDZT, sHT, n2, k4, k4 == 0, lane);
+  dz_below(std::integral_constant<int, 1>{}, sW1);
+  __syncthreads();
+  put_dz();
+  const u32x4 xf = __builtin_bit_cast(u32x4, x0[0][0]);
+  put_transposed(sHT, 8 * g, col, u32x2{xf[0], xf[1]});
+  put_transposed(sHT, 8 * g + 4, col, u32x2{xf[2], xf[3]});
+  __syncthreads();
+  grad_weights<0, 1, 2>(gp, sDZT, sHT, w * 16, 0, true, lane);
+}
+
+constexpr size_t MLP_GRAD_LDS = (size_t)MLP_NW * 2 + MLP_NB * 4 + BW_TILE * 2;
+static_assert(3 * BW_TILE * 2 <= MLP_NW * 2, "the backward tiles take the forward weights' place");
+static_assert(MLP_GRAD_LDS + GRAD_WAVES * 4 <= 160 * 1024, "k_mlp_gradient LDS");
+
+constexpr int RED_WAVES = 16;
+
+// grad = sum of the tiles' partials; a last block (loss given) sums the tiles' losses.  A workgroup
+// sums 64 parameters, each wavefront every RED_WAVES-th tile, in an order that depends on
+// the number of tiles alone.  256 tiles: 9.6 us, 6.2 TB/s; 62 us with one thread a parameter, a
+// chain of 256 loads.
+__global__ void __launch_bounds__(64 * RED_WAVES) k_mlp_reduce(const float *__restrict__ gpart, int nblk,
+                                                             float *__restrict__ grad,
+                                                             const float *__restrict__ loss_part,
+                                                             float *__restrict__ loss) {
+  __shared__ float part[RED_WAVES][64];
+  const int lane = threadIdx.x % 64, w = threadIdx.x / 64, e = blockIdx.x * 64 + lane;
+  const bool last = blockIdx.x * 64 >= MLP_NP;  // uniform
   float s = 0.f;
-  for (int b = 0; b < nblk; ++b) s += gpart[(size_t)b * MLP_NP + e];
-  grad[e] = s;
+  if (last) {
+    for (int b = threadIdx.x; b < nblk; b += 64 * RED_WAVES) s += loss_part[b];
+  } else if (e < MLP_NP) {
+#pragma unroll 8
+    for (int b = w; b < nblk; b += RED_WAVES) s += gpart[(size_t)b * MLP_NP + e];
+  }
+  part[w][lane] = s;
+  __syncthreads();
+  if (w) return;
+#pragma unroll
+  for (int i = 1; i < RED_WAVES; ++i) s += part[i][lane];
+  if (last) {
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
+    if (lane == 0) *loss = s;
+  } else if (e < MLP_NP) {
+    grad[e] = s;
+  }
 }
 
 // Layer, row and column of weight element e (row-major per layer).
@@ -417,8 +705,28 @@ extern "C" int ice3_mlp_backward(int npts, const void *wrm, const void *x, const
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(k_mlp_backward, dim3(nblk), dim3(256), MLP_BWD_LDS, s, a);
   HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((MLP_NP + 255) / 256), dim3(256), 0, s,
-                     (const float *)gpart, nblk, grad);
+  hipLaunchKernelGGL(k_mlp_reduce, dim3((MLP_NP + 63) / 64), dim3(64 * RED_WAVES), 0, s,
+                     (const float *)gpart, nblk, grad, (const float *)nullptr, (float *)nullptr);
+  HIPCHK(hipGetLastError());
+  return ICE3_OK;
+}
+
+extern "C" int ice3_mlp_gradient(int npts, const void *wpk, const void *wrm, const float *params,
+                                 const void *x, const float *target, float *gpart,
+                                 float *loss_part, float *grad, float *loss, void *stream) {
+  if (npts <= 0 || !wpk || !wrm || !params || !x || !target || !gpart || !loss_part || !grad || !loss)
+    return ICE3_EINVAL;
+  if ((uintptr_t)gpart % 16 != 0) return ICE3_EINVAL;  // stored by 16 bytes
+  MlpGradArgs a;
+  a.npts = npts; a.wpk = (const bf16x8 *)wpk; a.wrm = (const __bf16 *)wrm; a.params = params;
+  a.x = (const __bf16 *)x; a.target = target; a.gpart = gpart; a.loss_part = loss_part;
+  a.inv_count = 1.f / ((float)npts * MLP_NTARG);
+  const int nblk = (npts - 1) / MLP_TILE + 1;
+  hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(k_mlp_gradient, dim3(nblk), dim3(GRAD_THREADS), MLP_GRAD_LDS, s, a);
+  HIPCHK(hipGetLastError());
+  hipLaunchKernelGGL(k_mlp_reduce, dim3((MLP_NP + 63) / 64 + 1), dim3(64 * RED_WAVES), 0, s,
+                     (const float *)gpart, nblk, grad, (const float *)loss_part, loss);
   HIPCHK(hipGetLastError());
   return ICE3_OK;
 }

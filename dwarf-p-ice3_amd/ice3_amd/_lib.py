@@ -89,6 +89,7 @@ EXPORTS = ("ice3_ctx_create", "ice3_ctx_destroy", "ice3_strerror", "ice3_dump_co
            "ice3_stage_times", "ice3_adjust_rain_ice_stages", "ice3_adjust_rain_ice_surrogate",
            "ice3_adjust_rain_ice_surrogate_noalloc",
            "ice3_surrogate_features", "ice3_surrogate_work_bytes", "ice3_mlp_sizes", "ice3_mlp_forward", "ice3_mlp_backward",
+           "ice3_mlp_gradient",
            "ice3_mlp_adam", "ice3_count_nonfinite")
 
 _lib = None
@@ -166,6 +167,7 @@ def load():
         lib.ice3_mlp_sizes.argtypes = [ctypes.POINTER(ctypes.c_int)] * 5
         lib.ice3_mlp_forward.argtypes = [ctypes.c_int] + [_P] * 10
         lib.ice3_mlp_backward.argtypes = [ctypes.c_int] + [_P] * 8
+        lib.ice3_mlp_gradient.argtypes = [ctypes.c_int] + [_P] * 10
         lib.ice3_mlp_adam.argtypes = [ctypes.c_int] + [ctypes.c_float] * 4 + [_P] * 7
         lib.ice3_count_nonfinite.argtypes = [ctypes.c_int, ctypes.POINTER(_P), ctypes.POINTER(ctypes.c_int),
                                              ctypes.c_int, ctypes.c_int, _P, _P]

@@ -2,7 +2,7 @@
 
 The surrogate is a per-point MLP (18 features -> 4 x 128 SiLU -> 8 outputs) whose
 weights run in bf16 on the matrix cores with fp32 accumulation.  It is trained here,
-on the GPU, by the library's own kernels (``ice3_mlp_forward`` / ``ice3_mlp_backward``
+on the GPU, by the library's own kernels (``ice3_mlp_forward`` / ``ice3_mlp_gradient``
 / ``ice3_mlp_adam``), on state -> tendency pairs that the FP64 kernels produce
 (``make_pairs``): the input of the microphysics stage of the fused step
 (``ice3_surrogate_features``) and the change that stage makes to each source.
@@ -195,9 +195,6 @@ class MLP:
     def _buffers(self, n):
         if getattr(self, "_bn", 0) != n:
             tiles = (n + 127) // 128
-            self.zsave = torch.empty((4, n, 128), dtype=torch.float32, device=self.dev)
-            self.hsave = torch.empty((4, n, 128), dtype=torch.bfloat16, device=self.dev)
-            self.dy = torch.empty((n, 32), dtype=torch.float32, device=self.dev)
             self.loss_part = torch.empty(tiles, dtype=torch.float32, device=self.dev)
             self.gpart = torch.empty((tiles, self.n_params), dtype=torch.float32, device=self.dev)
             self._bn = n
@@ -206,14 +203,11 @@ class MLP:
         """Sum of squared errors and the gradient of the mean over the batch (into self.grad)."""
         n = x.shape[0]
         self._buffers(n)
-        sp = _sp(self.dev)
-        _lib.check(self.lib.ice3_mlp_forward(n, ptr(self.wpk), ptr(self.params), ptr(x), ptr(t), None,
-                                             ptr(self.zsave), ptr(self.hsave), ptr(self.dy), ptr(self.loss_part),
-                                             sp), "ice3_mlp_forward")
-        _lib.check(self.lib.ice3_mlp_backward(n, ptr(self.wrm), ptr(x), ptr(self.zsave), ptr(self.hsave),
-                                              ptr(self.dy), ptr(self.gpart), ptr(self.grad), sp),
-                   "ice3_mlp_backward")
-        return self.loss_part.sum()
+        loss = torch.empty((), dtype=torch.float32, device=self.dev)
+        _lib.check(self.lib.ice3_mlp_gradient(n, ptr(self.wpk), ptr(self.wrm), ptr(self.params), ptr(x), ptr(t),
+                                              ptr(self.gpart), ptr(self.loss_part), ptr(self.grad), ptr(loss),
+                                              _sp(self.dev)), "ice3_mlp_gradient")
+        return loss
 
     def adam(self, lr: float, b1: float = 0.9, b2: float = 0.999, eps: float = 1e-8):
         self.step += 1

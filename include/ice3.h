@@ -424,6 +424,8 @@ int ice3_surrogate_features(ice3_ctx *ctx, int ncol, int nlev, int ld, double dt
  * NULL); for training also zsave [4][npts][128] fp32, hsave [4][npts][128] bf16,
  * dy [npts][32] fp32 and loss_part [ceil(npts/128)] (sum of squared errors per tile).
  * ice3_mlp_backward: gpart [ceil(npts/128)][n_params] scratch, grad [n_params].
+ * ice3_mlp_gradient: both in one kernel, with nothing saved between them: gpart (16-byte
+ * aligned) and loss_part as above, scratch; grad [n_params] and loss[0], the sum of squared errors.
  * ice3_mlp_adam: one Adam step (grad NULL: only rewrite the bf16 copies wrm, wpk). */
 int ice3_mlp_sizes(int *n_params, int *n_weights, int *tile, int *in_width, int *out_width);
 int ice3_mlp_forward(int npts, const void *wpk, const float *params, const void *x,
@@ -432,6 +434,9 @@ int ice3_mlp_forward(int npts, const void *wpk, const float *params, const void 
 int ice3_mlp_backward(int npts, const void *wrm, const void *x, const float *zsave,
                       const void *hsave, const float *dy, float *gpart, float *grad,
                       void *stream);
+int ice3_mlp_gradient(int npts, const void *wpk, const void *wrm, const float *params,
+                      const void *x, const float *target, float *gpart, float *loss_part,
+                      float *grad, float *loss, void *stream);
 int ice3_mlp_adam(int step, float lr, float beta1, float beta2, float eps, float *params,
                   float *m, float *v, const float *grad, void *wrm, void *wpk, void *stream);
 
