@@ -135,5 +135,22 @@ def ptr(t) -> ctypes.c_void_p:
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(None)
 
 
+def addresses(tensors) -> list:
+    """The device addresses of tensors (None: 0) as integers, which a struct of pointers takes as
+    they are (without an object for each)."""
+    return [t.data_ptr() if t is not None else 0 for t in tensors]
+
+
+def new_fields(names, shape, device) -> dict:
+    """Uninitialised float64 fields of one shape, each with memory of its own (a torch.empty_like
+    takes 1.2 us, a torch.empty 1.7)."""
+    names = iter(names)
+    first = torch.empty(shape, dtype=torch.float64, device=device)
+    out = {next(names): first}
+    for k in names:
+        out[k] = torch.empty_like(first)
+    return out
+
+
 def stream_ptr(device) -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)

@@ -20,7 +20,8 @@ import ctypes
 import torch
 
 from . import _lib
-from ._fields import as_columns, as_rows, check_layout, from_columns, in_rows, ptr, resolve_layout, stream_ptr
+from ._fields import (addresses, as_columns, as_rows, check_layout, columns_of, from_columns, in_rows,
+                      new_fields, ptr, resolve_layout, stream_ptr)
 
 _PREC = {"fp64": _lib.PREC_FP64, "mixed": _lib.PREC_MIXED}
 _OUT_ORDER = ("t", "rv_out", "rc_out", "ri_out", "cldfr", "hlc_hrc", "hlc_hcf", "hli_hri",
@@ -120,12 +121,12 @@ class IceAdjust:
             f = {k: as_rows(v, k) for k, v in args.items()}
             ncol, nlev = f["th"].shape
         else:
-            f = {k: as_columns(v, layout, device=self.device, name=k) for k, v in args.items()}
+            f, _ = columns_of(args, layout, device=self.device)
             nlev, ncol = f["th"].shape
+        want = (ncol, nlev) if rows else (nlev, ncol)
         for k, v in f.items():
-            have = tuple(v.shape[::-1]) if rows else tuple(v.shape)
-            if have != (nlev, ncol):
-                raise ValueError(f"{k}: shape {have} != {(nlev, ncol)}")
+            if v.shape != want:
+                raise ValueError(f"{k}: shape {tuple(v.shape[::-1]) if rows else tuple(v.shape)} != {(nlev, ncol)}")
         sq = self._per_column(sigqsat, "sigqsat", ncol, layout)
         return f, sq, nlev, ncol, rows
 
@@ -134,11 +135,13 @@ class IceAdjust:
         _lib.require_finite({**{k: v.view(nlev, ncol) for k, v in f.items()}, **per_column}, self.device)
 
     def _results(self, out, names, layout, rows, shape):
+        if layout == "columns":
+            return tuple([out[k] for k in names])
         return tuple(out[k].reshape(shape) if rows else from_columns(out[k], layout, shape) for k in names)
 
     def _outputs(self, names, nlev, ncol, rows):
         shape = (ncol, nlev) if rows else (nlev, ncol)
-        return {k: torch.empty(shape, dtype=torch.float64, device=self.device) for k in names}
+        return new_fields(names, shape, self.device)
 
     def _per_column(self, x, name, ncol, layout):
         t = torch.as_tensor(x, dtype=torch.float64, device=self.device)
@@ -162,8 +165,8 @@ class IceAdjust:
             self._check_finite(f, {"sigqsat": sq}, nlev, ncol)
         names = _OUT_ORDER + (("srcs",) if return_srcs else ())
         out = self._outputs(names, nlev, ncol, rows)
-        cin = _lib.AdjustIn(*[ptr(f[k]) for k in _lib.ADJ_IN_FIELDS[:-1]], ptr(sq))
-        cout = _lib.AdjustOut(*[ptr(out[k]) for k in _lib.ADJ_OUT_FIELDS[:-1]], ptr(out.get("srcs")))
+        cin = _lib.AdjustIn(*addresses([f[k] for k in _lib.ADJ_IN_FIELDS[:-1]]), sq.data_ptr())
+        cout = _lib.AdjustOut(*addresses([out.get(k) for k in _lib.ADJ_OUT_FIELDS]))
         with torch.cuda.device(self.device):
             prec = _PREC[precision]
             if rows:
@@ -210,9 +213,9 @@ class IceAdjustOCND2(IceAdjust):
             self._check_finite(f, {"sigqsat": sq, "ice_cld_wgt": wgt}, nlev, ncol)
         names = _OUT_ORDER + _lib.OCND2_OUT_FIELDS + (("srcs",) if return_srcs else ())
         out = self._outputs(names, nlev, ncol, rows)
-        cin = _lib.AdjustIn(*[ptr(f[k]) for k in _lib.ADJ_IN_FIELDS[:-1]], ptr(sq))
+        cin = _lib.AdjustIn(*addresses([f[k] for k in _lib.ADJ_IN_FIELDS[:-1]]), sq.data_ptr())
         cin2 = _lib.Ocnd2In(ptr(f["zz"]), ptr(wgt))
-        cout = _lib.AdjustOut(*[ptr(out[k]) for k in _lib.ADJ_OUT_FIELDS[:-1]], ptr(out.get("srcs")))
+        cout = _lib.AdjustOut(*addresses([out.get(k) for k in _lib.ADJ_OUT_FIELDS]))
         cout2 = _lib.Ocnd2Out(*[ptr(out[k]) for k in _lib.OCND2_OUT_FIELDS])
         with torch.cuda.device(self.device):
             if rows:
@@ -249,8 +252,8 @@ class IceAdjustHail(IceAdjust):
             self._check_finite(f, {"sigqsat": sq}, nlev, ncol)
         names = _OUT_ORDER + (("srcs",) if return_srcs else ())
         out = self._outputs(names, nlev, ncol, rows)
-        cin = _lib.AdjustIn(*[ptr(f[k]) for k in _lib.ADJ_IN_FIELDS[:-1]], ptr(sq))
-        cout = _lib.AdjustOut(*[ptr(out[k]) for k in _lib.ADJ_OUT_FIELDS[:-1]], ptr(out.get("srcs")))
+        cin = _lib.AdjustIn(*addresses([f[k] for k in _lib.ADJ_IN_FIELDS[:-1]]), sq.data_ptr())
+        cout = _lib.AdjustOut(*addresses([out.get(k) for k in _lib.ADJ_OUT_FIELDS]))
         with torch.cuda.device(self.device):
             if rows:
                 rc_ = self._lib.ice3_ice_adjust_rows(self._ctx, ncol, nlev, float(timestep), ctypes.byref(cin),

@@ -43,8 +43,8 @@ import ctypes
 import torch
 
 from . import _lib
-from ._fields import (as_columns, check_layout, column_shape, columns_of, from_columns, ptr, resolve_layout,
-                      stream_ptr)
+from ._fields import (addresses, as_columns, check_layout, column_shape, columns_of, from_columns, new_fields, ptr,
+                      resolve_layout, stream_ptr)
 from .ice_adjust import check_configuration, sedimentation_of
 
 _PREC = {"fp64": _lib.PREC_FP64, "mixed": _lib.PREC_MIXED}
@@ -147,7 +147,7 @@ class RainIce(_Base):
             if v in state and k not in f and column_shape(state[v], layout, v) != (nlev, ncol):
                 raise ValueError(f"{k}: shape {column_shape(state[v], layout, v)} != {(nlev, ncol)}")
         for k, v in f.items():
-            if tuple(v.shape) != (nlev, ncol):
+            if v.shape != (nlev, ncol):
                 raise ValueError(f"{k}: shape {tuple(v.shape)} != {(nlev, ncol)}")
         extra = {k: f.pop(k) for k in self._EXTRA}
         f.setdefault("exn_ref", f["exn"])
@@ -159,18 +159,17 @@ class RainIce(_Base):
         src = {k: f[k] for k in _lib.RAIN_IO_FIELDS}
         # the sources and ci are updated in the copies made above, or apart from the caller's arrays
         io = {k: v if k in fresh else torch.empty_like(v) for k, v in src.items()}
-        out = {k: torch.empty((nlev, ncol), dtype=torch.float64, device=self.device) for k in ("evap3d", "rainfr")}
-        out.update({k: torch.empty(ncol, dtype=torch.float64, device=self.device)
-                    for k in ("inprc", "inprr", "inpri", "inprs", "inprg")})
+        out = {**new_fields(("evap3d", "rainfr"), (nlev, ncol), self.device),
+               **new_fields(("inprc", "inprr", "inpri", "inprs", "inprg"), (ncol,), self.device)}
         if check_inputs:
             _lib.require_finite(f, self.device)
             _lib.require_finite(extra, self.device)
         extra = self._extra_arrays(extra, fresh, nlev, ncol)
         counters, calls, st = self._stats(nlev * ncol, return_calls)
-        cin = _lib.RainIn(*[ptr(inp[k]) for k in _lib.RAIN_IN_FIELDS])
-        csrc = _lib.RainSrc(*[ptr(src[k]) for k in _lib.RAIN_IO_FIELDS], ptr(extra.get("rhs")))
-        cio = _lib.RainIO(*[ptr(io[k]) for k in _lib.RAIN_IO_FIELDS])
-        cout = _lib.RainOut(*[ptr(out[k]) for k in _lib.RAIN_OUT_FIELDS])
+        cin = _lib.RainIn(*addresses([inp[k] for k in _lib.RAIN_IN_FIELDS]))
+        csrc = _lib.RainSrc(*addresses([src[k] for k in _lib.RAIN_IO_FIELDS] + [extra.get("rhs")]))
+        cio = _lib.RainIO(*addresses([io[k] for k in _lib.RAIN_IO_FIELDS]))
+        cout = _lib.RainOut(*addresses([out[k] for k in _lib.RAIN_OUT_FIELDS]))
         with torch.cuda.device(self.device), self._scheme():
             rc = self._launch(precision, ncol, nlev, dt, cin, csrc, extra, cio, cout, st)
         _lib.check(rc, self._ENTRY)
@@ -214,26 +213,23 @@ class AdjustRainIce(_Base):
             wgt = self._per_column(f["ice_cld_wgt"], "ice_cld_wgt", ncol, layout)
             if nlev < 2:
                 raise ValueError("the OCND2 branch needs at least two levels")
-        for k, v in {**{k: tuple(v.shape) for k, v in g.items()},
+        for k, v in {**{k: v.shape for k, v in g.items()},
                      "rhodj": column_shape(f["rhodj"], layout, "rhodj")}.items():
             if v != (nlev, ncol):
-                raise ValueError(f"{k}: shape {v} != {(nlev, ncol)}")
+                raise ValueError(f"{k}: shape {tuple(v)} != {(nlev, ncol)}")
         g.setdefault("rhodj", g["rhodref"])
         extra = {k: g.pop(k) for k in more}
         if check_inputs:
             _lib.require_finite({**g, **extra, "sigqsat": sq, **({"ice_cld_wgt": wgt} if ocnd2 else {})},
                                 self.device)
-        out = {k: torch.empty((nlev, ncol), dtype=torch.float64, device=self.device)
-               for k in _lib.PIPE_OUT_FIELDS[:15]}
-        out.update({k: torch.empty(ncol, dtype=torch.float64, device=self.device)
-                    for k in _lib.PIPE_OUT_FIELDS[15:]})
+        out = {**new_fields(_lib.PIPE_OUT_FIELDS[:15], (nlev, ncol), self.device),
+               **new_fields(_lib.PIPE_OUT_FIELDS[15:], (ncol,), self.device)}
         counters, calls, st = self._stats(nlev * ncol, return_calls)
-        cin = _lib.PipeIn(*[ptr(g[k]) for k in _lib.PIPE_IN_FIELDS[:-1]], ptr(sq))
-        cout = _lib.PipeOut(*[ptr(out[k]) for k in _lib.PIPE_OUT_FIELDS])
+        cin = _lib.PipeIn(*addresses([g[k] for k in _lib.PIPE_IN_FIELDS[:-1]]), sq.data_ptr())
+        cout = _lib.PipeOut(*addresses([out[k] for k in _lib.PIPE_OUT_FIELDS]))
         with torch.cuda.device(self.device), self._scheme():
             if ocnd2:
-                x = {k: torch.empty((nlev, ncol), dtype=torch.float64, device=self.device)
-                     for k in _lib.OCND2_OUT_FIELDS}
+                x = new_fields(_lib.OCND2_OUT_FIELDS, (nlev, ncol), self.device)
                 cin2 = _lib.Ocnd2In(ptr(extra["zz"]), ptr(wgt))
                 cout2 = _lib.Ocnd2Out(*[ptr(x[k]) for k in _lib.OCND2_OUT_FIELDS])
                 rc = self._lib.ice3_adjust_rain_ice_ocnd2(self._ctx, ncol, nlev, ncol, float(dt),
@@ -255,7 +251,7 @@ class AdjustRainIce(_Base):
         _lib.check(rc, "ice3_adjust_rain_ice_ocnd2" if ocnd2 else
                    ("ice3_adjust_rain_ice_hail" if hail else "ice3_adjust_rain_ice"))
         self._finish_counters(counters)
-        res = {k: from_columns(v, layout, shape) for k, v in out.items()}
+        res = out if layout == "columns" else {k: from_columns(v, layout, shape) for k, v in out.items()}
         if return_calls:
             res["calls"] = from_columns(calls.view(nlev, ncol), layout, shape)
         return res

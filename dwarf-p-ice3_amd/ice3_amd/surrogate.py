@@ -26,7 +26,7 @@ import numpy as np
 import torch
 
 from . import _lib, synthetic
-from ._fields import ptr
+from ._fields import addresses, new_fields, ptr
 
 NFEAT, NTARG = _lib.NFEAT, _lib.NTARG
 FEATURES = ("T", "ln_p", "rhodref", "ln_rv", "ln_rc", "ln_rr", "ln_ri", "ln_rs", "ln_rg", "ln_1p_ci",
@@ -326,15 +326,15 @@ class AdjustRainIceSurrogate:
         g = {k: base_col(f[k], self.dev) for k in _lib.PIPE_IN_FIELDS if k != "sigqsat"}
         nlev, ncol = g["th"].shape
         sq = torch.as_tensor(f["sigqsat"], dtype=torch.float64, device=self.dev).reshape(-1)[:ncol].contiguous()
-        out = {k: torch.empty((nlev, ncol), dtype=torch.float64, device=self.dev) for k in _lib.PIPE_OUT_FIELDS[:15]}
-        out.update({k: torch.empty(ncol, dtype=torch.float64, device=self.dev) for k in _lib.PIPE_OUT_FIELDS[15:]})
+        out = {**new_fields(_lib.PIPE_OUT_FIELDS[:15], (nlev, ncol), self.dev),
+               **new_fields(_lib.PIPE_OUT_FIELDS[15:], (ncol,), self.dev)}
         work = torch.empty(self.lib.ice3_surrogate_work_bytes(ncol, nlev), dtype=torch.uint8, device=self.dev)
         sgc = torch.zeros(5, dtype=torch.int64, device=self.dev)
         counters = torch.zeros(3, dtype=torch.int64, device=self.dev)
         calls = torch.zeros(nlev * ncol, dtype=torch.int32, device=self.dev) if return_calls else None
         st = _lib.Stats(ptr(calls), ptr(counters))
-        cin = _lib.PipeIn(*[ptr(g[k]) for k in _lib.PIPE_IN_FIELDS[:-1]], ptr(sq))
-        cout = _lib.PipeOut(*[ptr(out[k]) for k in _lib.PIPE_OUT_FIELDS])
+        cin = _lib.PipeIn(*addresses([g[k] for k in _lib.PIPE_IN_FIELDS[:-1]]), sq.data_ptr())
+        cout = _lib.PipeOut(*addresses([out[k] for k in _lib.PIPE_OUT_FIELDS]))
         h = self.sg.handle()
         with torch.cuda.device(self.dev):
             rc = self.lib.ice3_adjust_rain_ice_surrogate(self.ctx, ncol, nlev, ncol, float(dt), ctypes.byref(cin),
