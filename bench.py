@@ -481,7 +481,7 @@ MLP_FLOP_EXECUTED = 2.0 * (32 * 128 + 3 * 128 * 128 + 128 * 32)   # 114,688 per 
 MLP_ACTIVATIONS = 4 * 128                                         # SiLU evaluations per point
 # Full-rate FP32 VALU lane operations per second: 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz.
 VALU_LANE_OPS = 256 * 4 * 16 * 2.4e9
-# VALU issue slots per activation in k_mlp_infer's epilogue as compiled: v_exp_f32 and
+# VALU issue slots per activation in k_sg_network's epilogue as compiled: v_exp_f32 and
 # v_rcp_f32 (quarter rate, 4 slots each), 2 v_add_f32, 2 v_mul_f32, a bf16 convert and an
 # accumulator read; with a single quarter-rate operation and the bias add, multiply and
 # convert, 7.
@@ -601,8 +601,8 @@ def surrogate_variant(lib, ctx, dev, g, args, reps: int = 4):
              "fp64_step_ms": ms_plain,
              "basis": "matrix-core time at the dense bf16 peak; SiLU epilogue at the full-rate FP32 VALU "
                       "issue rate (quarter-rate exp/rcp = 4 slots); step floor = the column walk and the "
-                      "FP64 fallback as measured, plus the network at its floor, with features and decode "
-                      "fused away"}
+                      "FP64 fallback as measured, plus the network at its floor (the measured network "
+                      "stage has features and decode in it)"}
     return {"columns": ncol, "levels": nlev, "weights": os.path.relpath(S.DEFAULT_WEIGHTS, ROOT),
             "train_pairs": int(sg.meta.get("pairs", 0)), "budget_tol": sg.budget_tol, "neg_tol": sg.neg_tol,
             "fp64_ms_per_step": ms_plain, "fp64_columns_per_s": ncol / (ms_plain * 1e-3),
@@ -612,7 +612,7 @@ def surrogate_variant(lib, ctx, dev, g, args, reps: int = 4):
                                                                  "water_residual": c[3], "no_hydrometeor": c[4]},
             "network_fraction": c[0] / npts, "water_budget_max_rel_err": budget, "error_vs_fp64": err,
             "floor": floor,
-            "roofline": {"bound": "mfma", "kernel": "k_mlp_infer", "achieved": tflops,
+            "roofline": {"bound": "mfma", "kernel": "k_sg_network", "achieved": tflops,
                          "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": tflops / MFMA_BF16_PEAK_TFLOPS,
                          "flop_per_point": MLP_FLOP_PER_POINT, "ms_per_launch": stages["network"]}}
 

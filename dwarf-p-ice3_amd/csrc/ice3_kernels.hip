@@ -15,11 +15,10 @@
 //                  the ICE4 time-split microphysics, total tendencies and negativity
 //                  correction per point, with the points of long time splittings
 //                  compacted into full wavefronts (ballot, LDS parking);
-//   k_sg_features, k_mlp_infer, k_sg_decode
-//                  the learned surrogate of k_micro: features and range check per point;
-//                  the MLP on the bf16 matrix cores (k_mlp_infer, in ice3_mlp.hip);
-//                  decode, water and sign checks per point.  Points it rejects are
-//                  queued for k_micro_segments, the plain FP64 microphysics over the queue.
+//   k_sg_network   (ice3_surrogate.hip) the learned surrogate of k_micro: features and range
+//                  check per point, the MLP on the bf16 matrix cores, decode, water and sign
+//                  checks per point.  Points it rejects are queued for k_micro_segments, the
+//                  plain FP64 microphysics over the queue.
 // rain_ice is k_sedim then k_micro on one stream; the fused time step is
 // k_ice_adjust, k_sedim, k_micro, or k_adjust_sedim, k_micro.  R is the arithmetic of the process rates
 // and lookups (double, or float for the mixed path).
@@ -36,6 +35,7 @@
 #include "ice3_stages.hpp"
 #include "ice3_mlp.hpp"
 #include "ice3_sedim.hpp"
+#include "ice3_surrogate.hpp"
 
 namespace ice3 {
 
@@ -794,163 +794,30 @@ __global__ void __launch_bounds__(256) k_micro_branches(MicroArgs a) {
   a.branches[j] = br;
 }
 
-struct SurrogateArgs {
-  MicroArgs m;
-  unsigned int npts;                 // nlev * ncol; point q = k * ncol + i
-  const ice3_surrogate_norm *norm;
-  float budget_tol, neg_tol;
-  __bf16 *x;                         // [npts][MLP_IN] network inputs
-  float *y;                          // [npts][MLP_NTARG] network outputs
-  unsigned char *flag;               // [npts] SG_* reason, SG_OK = ask the network
-  unsigned int *queue;               // [0] count, [1 + q] point offsets
-  unsigned long long *counters;      // 5 entries, see include/ice3.h
-};
-
-// Reasons a point is not taken from the network.
-enum { SG_OK = 0, SG_RANGE = 1, SG_NEG = 2, SG_BUDGET = 3, SG_NOMICRO = 4 };
-
-__device__ __forceinline__ size_t point_offset(const MicroArgs &m, unsigned int q) {
-  return (size_t)(q / m.ncol) * m.ld + q % m.ncol;
-}
-
-// Stage 1 of the surrogate: features, range check, network inputs (one thread per point).
-__global__ void __launch_bounds__(256) k_sg_features(SurrogateArgs a) {
-  const unsigned int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= a.npts) return;
-  const ice3_surrogate_norm &nm = *a.norm;
-  float f[MLP_NFEAT];
-  int flag = SG_NOMICRO;
-  if (surrogate_features(a.m, point_offset(a.m, q), f)) {
-    flag = SG_OK;
-#pragma unroll
-    for (int c = 0; c < MLP_NFEAT; ++c)
-      if (!(f[c] >= nm.feat_lo[c] && f[c] <= nm.feat_hi[c])) flag = SG_RANGE;
-  }
-  a.flag[q] = (unsigned char)flag;
-  bf16x8 v[MLP_IN / 8];
-#pragma unroll
-  for (int c = 0; c < MLP_IN; ++c)
-    v[c / 8][c % 8] = (__bf16)(flag == SG_OK && c < MLP_NFEAT ? (f[c] - nm.feat_mean[c]) * nm.feat_scale[c] : 0.f);
-  bf16x8 *xr = (bf16x8 *)(a.x + (size_t)q * MLP_IN);
-#pragma unroll
-  for (int c = 0; c < MLP_IN / 8; ++c) xr[c] = v[c];
-}
-
-// Stage 2: the network over all points, k_mlp_infer (ice3_mlp.hip, launched by
-// mlp_infer_launch).
-
-
-// Stage 3: decode, physical checks, results or fallback queue.  Persistent grid: block b
-// decodes the 256-point chunks b, b + gridDim.x, ... (spread over all levels, so every
-// block meets the same mix of cheap and costly fallback points) and appends its rejected
-// points to its own queue segment queue[1 + b*seg ...], counting them in qcount[b]; no
-// global atomics but the 5 counters.
-// Decode blocks: a fixed count (8 per CU on a 256-CU MI355X), so that the scratch size
-// depends on the problem size only.  Block b's queue segment holds seg =
-// ceil(chunks / SG_DEC_BLOCKS) * 256 entries; all segments fit in npts + 256 * (SG_DEC_BLOCKS + 1).
-constexpr unsigned int SG_DEC_BLOCKS = 2048;
-
-__device__ __forceinline__ int sg_decode_point(const SurrogateArgs &a, unsigned int q, size_t j) {
-  const MicroArgs &m = a.m;
-  const ice3_surrogate_norm &nm = *a.norm;
-  int flag = a.flag[q];
-  if (flag != SG_OK) return flag;
-  double out[7], y[7], rsum = 0., rmag = 0.;
-  const float *yq = a.y + (size_t)q * MLP_NTARG;
-#pragma unroll
-  for (int v = 0; v < 7; ++v) {
-    y[v] = (double)(nm.targ_unit[v] * sinhf(nm.targ_mean[v] + nm.targ_std[v] * yq[v]));
-    out[v] = m.src[v][j] + y[v];
-    if (v >= 1) { rsum += y[v]; rmag += fabs(y[v]); }
-  }
-  // water residual against the predicted changes, with a floor of budget_tol times the
-  // smallest typical change (median |change| of the training targets)
-  double umin = nm.targ_unit[IRV];
-#pragma unroll
-  for (int v = IRC; v <= IRG; ++v) umin = fmin(umin, (double)nm.targ_unit[v]);
-  if (!(fabs(rsum) <= (double)a.budget_tol * (rmag + umin))) return SG_BUDGET;
-  out[IRV] -= rsum;  // move the water residual into vapour
-  // a source may go negative by neg_tol of (its value + its change + the typical change)
-#pragma unroll
-  for (int v = IRC; v <= IRG; ++v)
-    if (!(out[v] >= -(double)a.neg_tol * (fabs(m.src[v][j]) + fabs(y[v]) + (double)nm.targ_unit[v])))
-      return SG_NEG;
-  double lvfact, lsfact;
-  latent_factors(m, j, lvfact, lsfact);
-  correct_negativities(out[ITH], out[IRV], out[IRC], out[IRR], out[IRI], out[IRS], out[IRG],
-                       lvfact, lsfact);
-  if (!(out[IRV] >= 0.)) return SG_NEG;
-  const double cinew =
-      fmax(0., m.src_ci[j] + (double)(nm.targ_unit[7] * sinhf(nm.targ_mean[7] + nm.targ_std[7] * yq[7])));
-#pragma unroll
-  for (int v = 0; v < 7; ++v) m.dst[v][j] = out[v];
-  m.ci[j] = cinew;
-  m.evap3d[j] = 0.;
-  m.rainfr[j] = 1.;
-  if (m.calls) m.calls[j] = 0;
-  return SG_OK;
-}
-
-__global__ void __launch_bounds__(256) k_sg_decode(SurrogateArgs a, unsigned int seg,
-                                                   unsigned int *qcount) {
-  __shared__ unsigned int sWave[MLP_WAVES];
-  const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
-  const unsigned int q0 = blockIdx.x * seg;   // this block's queue segment
-  unsigned int nq = 0;                 // rejected points of this block so far (uniform)
-  unsigned int cnt[5] = {0, 0, 0, 0, 0};
-  for (unsigned int base = blockIdx.x * blockDim.x; base < a.npts; base += gridDim.x * blockDim.x) {
-    const unsigned int q = base + threadIdx.x;
-    int flag = -1;
-    size_t j = 0;
-    if (q < a.npts) {
-      j = point_offset(a.m, q);
-      flag = sg_decode_point(a, q, j);
-      ++cnt[flag];
-    }
-    const bool rej = flag > SG_OK;
-    const unsigned long long mask = __ballot(rej);
-    if (lane == 0) sWave[w] = (unsigned int)__popcll(mask);
-    __syncthreads();
-    unsigned int off = nq;
-    for (int v = 0; v < w; ++v) off += sWave[v];
-    if (rej) a.queue[1 + q0 + off + __popcll(mask & ((1ull << lane) - 1ull))] = (unsigned int)j;
-    for (int v = 0; v < MLP_WAVES; ++v) nq += sWave[v];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) qcount[blockIdx.x] = nq;
-#pragma unroll
-  for (int c = 0; c < 5; ++c) {
-    unsigned long long v = cnt[c];
-#pragma unroll
-    for (int mm = 32; mm >= 1; mm >>= 1) v += __shfl_xor(v, mm, 64);
-    if (lane == 0 && v) atomicAdd(&a.counters[c], v);
-  }
-}
-
 // Plain microphysics over the surrogate's rejected points: block b runs the qcount[b]
-// points that decode block b queued.
+// points that wavefront b of the network stage queued.
 template <class R>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) k_micro_segments(MicroArgs a, const unsigned int *queue,
                                                        const unsigned int *qcount, unsigned int seg) {
   const unsigned int n = qcount[blockIdx.x];
-  const unsigned int *list = queue + 1 + (size_t)blockIdx.x * seg;
+  const unsigned int *list = queue + (size_t)blockIdx.x * seg;
   for (unsigned int e = threadIdx.x; e < n; e += blockDim.x)
     if (micro_at<R>(a, (size_t)list[e], a.tab) < 0 && a.capped) atomicAdd(a.capped, 1ull);
 }
 
-// Scratch layout of the surrogate step (bytes, 256-aligned blocks).
+// Scratch layout of the surrogate step (bytes, 256-aligned blocks).  total is more than the queue
+// takes: it is what the interface asks of a work area and measures the allocation-free entry's
+// limit by (room for a network input, an output and a reason per point as well; 64 (SG_WAVES +
+// 1) words and SG_WAVES counts are fewer than its 256 x 2049 words beside the points').
 struct SgWork {
-  size_t x, y, flag, queue, qcount, total;
+  size_t queue, qcount, total;
 };
 static SgWork sg_work_layout(size_t npts) {
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
   SgWork w;
-  w.x = 0;
-  w.y = w.x + al(npts * MLP_IN * 2);
-  w.flag = w.y + al(npts * MLP_NTARG * 4);
-  w.queue = w.flag + al(npts);
-  w.qcount = w.queue + al((npts + 1 + 256 * ((size_t)SG_DEC_BLOCKS + 1)) * 4);
-  w.total = w.qcount + al((size_t)SG_DEC_BLOCKS * 4);
+  w.queue = 0;
+  w.qcount = al((npts + 64 * ((size_t)SG_WAVES + 1)) * 4);
+  w.total = al(npts * 64) + al(npts * 32) + al(npts) + al((npts + 1 + 256 * 2049) * 4) + 8192;
   return w;
 }
 
@@ -1826,14 +1693,6 @@ extern "C" int ice3_adjust_rain_ice_hail(ice3_ctx *ctx, int ncol, int nlev, int 
   return ICE3_OK;
 }
 
-static int n_cus(int device) {
-  int n = 0;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
-      n <= 0)
-    n = 256;
-  return n;
-}
-
 extern "C" size_t ice3_surrogate_work_bytes(int ncol, int nlev) {
   if (ncol <= 0 || nlev <= 0) return 0;
   return sg_work_layout((size_t)ncol * nlev).total;
@@ -1883,34 +1742,22 @@ static int surrogate_step(ice3_ctx *ctx, int ncol, int nlev, int ld, double dt,
   g.norm = sg->norm;
   g.budget_tol = sg->budget_tol;
   g.neg_tol = sg->neg_tol;
-  g.x = (__bf16 *)(wb + wl.x);
-  g.y = (float *)(wb + wl.y);
-  g.flag = wb + wl.flag;
+  g.wpk = sg->weights_packed;
+  g.params = sg->params;
   g.queue = (unsigned int *)(wb + wl.queue);
   g.counters = sg_counters;
-  const int ncu = n_cus(ctx->device);
-  const unsigned int ntiles = (npts + MLP_TILE - 1) / MLP_TILE;
-  const unsigned int nblk = ntiles < (unsigned int)ncu ? ntiles : (unsigned int)ncu;
+  g.qcount = (unsigned int *)(wb + wl.qcount);
+  unsigned int nseg = 0;
   MARK(0);
   HIPCHK(launch_adjust_sedim(ctx, aa, sa, s));
   MARK(1);
   MARK(2);
-  hipLaunchKernelGGL(k_sg_features, dim3((npts + 255) / 256), dim3(256), 0, s, g);
-  HIPCHK(hipGetLastError());
   MARK(3);
-  HIPCHK(mlp_infer_launch(sg->weights_packed, sg->params, g.x, g.y, npts, nblk, s));
+  HIPCHK(surrogate_network_launch(g, ctx->ncu, &nseg, s));
   MARK(4);
-  // decode: a persistent grid of SG_DEC_BLOCKS blocks; block b decodes chunks
-  // b, b + ndec, ... of 256 points and owns a queue segment of seg entries
-  unsigned int *qcount = (unsigned int *)(wb + wl.qcount);
-  const unsigned int nchunks = (npts + 255) / 256;
-  const unsigned int ndec = nchunks < SG_DEC_BLOCKS ? nchunks : SG_DEC_BLOCKS;
-  const unsigned int seg = ((nchunks + ndec - 1) / ndec) * 256;
-  hipLaunchKernelGGL(k_sg_decode, dim3(ndec), dim3(256), 0, s, g, seg, qcount);
-  HIPCHK(hipGetLastError());
   MARK(5);
-  hipLaunchKernelGGL(k_micro_segments<double>, dim3(ndec), dim3(64), 0, s, m,
-                     (const unsigned int *)g.queue, (const unsigned int *)qcount, seg);
+  hipLaunchKernelGGL(k_micro_segments<double>, dim3(nseg), dim3(64), 0, s, m,
+                     (const unsigned int *)g.queue, (const unsigned int *)g.qcount, g.seg);
   HIPCHK(hipGetLastError());
   MARK(6);
   return ICE3_OK;

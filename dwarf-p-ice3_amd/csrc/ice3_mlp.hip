@@ -1,5 +1,5 @@
 // ice3_mlp.hip -- kernels of the rain_ice surrogate MLP (bf16 matrix cores, fp32
-// accumulation): training, with its C ABI (declared in include/ice3.h), and inference.
+// accumulation): training, with its C ABI (declared in include/ice3.h).
 //
 //   k_mlp_forward   one 128-point tile per workgroup: 5 layers on v_mfma_f32_16x16x32_bf16
 //                   with every weight resident in LDS; saves pre-activations (fp32) and
@@ -11,8 +11,6 @@
 //   k_mlp_reduce    sum of the partial gradients (and losses).
 //   k_mlp_adam      Adam on the fp32 master parameters; rewrites the bf16 row-major and
 //                   packed-fragment copies the matrix cores read.
-//   k_mlp_infer     inference over all points of the surrogate step: persistent grid,
-//                   weights resident in LDS (launched by mlp_infer_launch).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -259,7 +257,7 @@ constexpr size_t MLP_BWD_LDS = (size_t)4 * BW_TILE * 2;
 
 // ---- Forward and backward in one kernel, nothing saved to memory between them.
 // A workgroup takes a tile of 128 points, a wavefront 16 of them through every layer, activations
-// in registers as in k_mlp_infer, the pre-activations of the four hidden layers beside them
+// in registers as in k_sg_network, the pre-activations of the four hidden layers beside them
 // (fp32, 128 of 256 registers; the sigmoid is computed a second time rather than kept).  For
 // dW = H^T dZ the points are the contraction, so H and dZ of a layer go through LDS transposed;
 // dH = W dZ takes dZ from registers.  The backward tiles lie where the forward weights were, the
@@ -585,88 +583,6 @@ __global__ void __launch_bounds__(256) k_mlp_adam(int step, float lr, float b1, 
     wrm[e] = b;
     wpk[mlp_pack_index(l, k, n)] = b;
   }
-}
-
-// Inference over all points (the surrogate step's network stage).  Persistent grid, one
-// workgroup a compute unit, all weights resident in LDS; every wavefront takes 32-point tiles of
-// its own, activations in registers, no barrier after the weights are in.
-// Bound by the VALU: a SiLU takes two quarter-rate transcendentals, four other operations and half
-// a conversion, 50 of the 56 cycles a wavefront of activations takes (512 x 512 x 90 points: 4.27
-// ms, 574 TFLOP/s; 6.41 ms with four wavefronts and the activations through LDS).  Two wavefronts a
-// SIMD, so that one's matrix products run beside the other's SiLUs; four a SIMD at 16 points
-// each, the weights read twice as often, take 4.69 ms.
-constexpr int INFER_WAVES = 8, INFER_MT = 2, INFER_PTS = 16 * INFER_MT;
-
-__global__ void __launch_bounds__(64 * INFER_WAVES) k_mlp_infer(const bf16x8 *__restrict__ wpk,
-                                                                const float *__restrict__ params,
-                                                                const __bf16 *__restrict__ x,
-                                                                float *__restrict__ y, unsigned int npts) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  bf16x8 *sW = (bf16x8 *)smem;
-  float *sB = (float *)(smem + MLP_NW * 2);
-  const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
-  const int pt = lane % 16, g = lane / 16;  // this lane's point of a tile, and its quarter of the units
-  block_copy16(sW, wpk, MLP_NW * 2);
-  for (int q = threadIdx.x; q < MLP_NB; q += blockDim.x) sB[q] = params[MLP_NW + q];
-  __syncthreads();
-  const unsigned int ntiles = (npts + INFER_PTS - 1) / INFER_PTS, step = gridDim.x * INFER_WAVES;
-  auto load_x = [&](unsigned int tile, bf16x8 (&x0)[INFER_MT][1]) {
-#pragma unroll
-    for (int mt = 0; mt < INFER_MT; ++mt) {
-      const unsigned int p = tile * INFER_PTS + mt * 16 + pt;
-      if (p < npts) x0[mt][0] = *(const bf16x8 *)(x + (size_t)p * MLP_IN + 8 * g);
-      else x0[mt][0] = bf16x8{};
-    }
-  };
-  bf16x8 x0[INFER_MT][1];
-  unsigned int tile = blockIdx.x * INFER_WAVES + w;
-  if (tile < ntiles) load_x(tile, x0);
-  for (; tile < ntiles; tile += step) {
-    f32x4 acc[INFER_MT][MLP_H / 16];
-    bf16x8 h[INFER_MT][MLP_H / 32];
-    auto epilogue = [&](int l) {  // bias, SiLU, and the next layer's operands
-#pragma unroll
-      for (int kk = 0; kk < MLP_H / 32; ++kk) {
-        const f32x4 b0 = *(const f32x4 *)(sB + l * MLP_H + kk * 32 + 4 * g);
-        const f32x4 b1 = *(const f32x4 *)(sB + l * MLP_H + kk * 32 + 16 + 4 * g);
-#pragma unroll
-        for (int mt = 0; mt < INFER_MT; ++mt) {
-          float v0[4], v1[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            v0[i] = silu(acc[mt][2 * kk][i] + b0[i]);
-            v1[i] = silu(acc[mt][2 * kk + 1][i] + b1[i]);
-          }
-          h[mt][kk] = operand_of(pack4(v0[0], v0[1], v0[2], v0[3]), pack4(v1[0], v1[1], v1[2], v1[3]));
-        }
-      }
-    };
-    mlp_product<MLP_IN, MLP_H, MLP_H / 16, INFER_MT>(sW + mlp_woff(0) / 8, x0, acc, lane);
-    if (tile + step < ntiles) load_x(tile + step, x0);  // prefetch the next tile
-    epilogue(0);
-#pragma unroll 1
-    for (int l = 1; l <= 3; ++l) {
-      mlp_product<MLP_H, MLP_H, MLP_H / 16, INFER_MT>(sW + mlp_woff(l) / 8, h, acc, lane);
-      epilogue(l);
-    }
-    f32x4 out[INFER_MT][1];  // the first 16 of the padded outputs
-    mlp_product<MLP_H, 16, MLP_OUT / 16, INFER_MT>(sW + mlp_woff(4) / 8, h, out, lane);
-    const f32x4 b = *(const f32x4 *)(sB + 4 * MLP_H + 4 * g);
-#pragma unroll
-    for (int mt = 0; mt < INFER_MT; ++mt) {
-      const unsigned int p = tile * INFER_PTS + mt * 16 + pt;
-      if (4 * g < MLP_NTARG && p < npts) *(f32x4 *)(y + (size_t)p * MLP_NTARG + 4 * g) = out[mt][0] + b;
-    }
-  }
-}
-
-constexpr size_t INFER_LDS = (size_t)MLP_NW * 2 + MLP_NB * 4;
-
-hipError_t mlp_infer_launch(const void *wpk, const float *params, const void *x, float *y,
-                            unsigned int npts, unsigned int nblk, hipStream_t s) {
-  hipLaunchKernelGGL(k_mlp_infer, dim3(nblk), dim3(64 * INFER_WAVES), INFER_LDS, s, (const bf16x8 *)wpk,
-                     params, (const __bf16 *)x, y, npts);
-  return hipGetLastError();
 }
 
 }  // namespace ice3

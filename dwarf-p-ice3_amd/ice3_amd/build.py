@@ -11,7 +11,7 @@ CSRC = os.path.join(PKG, "csrc")
 OUT = os.path.join(HERE, "_lib", "libice3_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ("ice3_kernels.hip", "ice3_sedim.hip", "ice3_mlp.hip", "ice3_params.cpp")
+SOURCES = ("ice3_kernels.hip", "ice3_sedim.hip", "ice3_surrogate.hip", "ice3_mlp.hip", "ice3_params.cpp")
 # -ffp-contract=off keeps FP64 a*b+c as two roundings, the sequence of the CPU reference.
 # Packed FP32 instructions (v_pk_*_f32) are disabled for the device code: some of their
 # forms have given wrong results on this hardware without any error.
@@ -30,8 +30,8 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
 # allocator has failed on it).
 # The iterative ILP scheduler for the physics kernels: they run at a fixed two (k_micro) or four
 # (k_adjust_sedim) wavefronts per SIMD and hide latency mostly within a wavefront (k_micro
-# -7 %; results bit for bit the same).  k_mlp_infer, bound by the VALU, is faster with the
-# default one (4.27 against 4.46 ms at 512x512x90).
+# -7 %; results bit for bit the same), and for the surrogate's network kernel (k_sg_network 5.79
+# ms at 512x512x90, 5.94 with the default one, 6.23 with max-ilp).
 # -fapprox-func for the physics kernels' device code: divisions become a reciprocal and
 # Newton steps (FP64: two steps and a residual correction, within 1 ulp and in practice
 # correctly rounded; FP32: the hardware reciprocal, 1 ulp) instead of the scaled IEEE
@@ -42,6 +42,7 @@ ILP = ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]
 SOURCE_FLAGS = {"ice3_kernels.hip": ["-mllvm", "-disable-machine-licm", "-Xarch_device", "-fapprox-func",
                                      *ILP],
                 "ice3_sedim.hip": ["-Xarch_device", "-fapprox-func"],
+                "ice3_surrogate.hip": ["-Xarch_device", "-fapprox-func", *ILP],
                 "ice3_mlp.hip": []}
 
 

@@ -380,8 +380,7 @@ typedef struct {
 } ice3_surrogate;
 
 /* Fused step with the surrogate microphysics.  work: device scratch of
- * ice3_surrogate_work_bytes(ncol, nlev) bytes, 256-byte aligned (network inputs and
- * outputs, reasons, fallback queue).  sg_counters (device, 5 entries, accumulated):
+ * ice3_surrogate_work_bytes(ncol, nlev) bytes, 256-byte aligned (the fallback queue).  sg_counters (device, 5 entries, accumulated):
  * [0] points taken from the network, [1] out of range, [2] negative source,
  * [3] water residual, [4] no hydrometeor.  stats as for ice3_adjust_rain_ice (fallback
  * points only; network points report 0 calls). */
@@ -447,8 +446,8 @@ int ice3_mlp_adam(int step, float lr, float beta1, float beta2, float eps, float
  * ms[0] ICE_ADJUST, ms[1] sedimentation, ms[2] microphysics (in the FP64 fused step and
  * the surrogate step the first two stages run as one kernel: ms[0] covers both and ms[1]
  * is about 0); for the surrogate step
- * ms[2] is the feature kernel and ms[3] the network, ms[4] the decode and ms[5] the
- * fallback microphysics (0 for a stage the call did not run).  Off by default; a
+ * ms[3] is the network kernel, features and decode included (ms[2] and ms[4] are about 0),
+ * and ms[5] the fallback microphysics (0 for a stage the call did not run).  Off by default; a
  * context's events serve one call at a time. */
 int ice3_stage_timing(ice3_ctx *ctx, int enable);
 int ice3_stage_times(ice3_ctx *ctx, float ms[6]);
