@@ -504,11 +504,11 @@ __global__ void __launch_bounds__(64 * SPLIT_COLS)
 // FP64 VALU issues about two thirds of the cycles.  Parking every unfinished point after its
 // hard call, so that soft passes were full, read every input line and wrote every output line
 // twice (10 GB at 512x512x90 against 5.3 algorithmic), as their lines had left the L2 by then:
-// 2.79 ms in FP64, 2.40 mixed, 3.57 with OCND2, against 2.72, 1.88 and 3.37 now.
+// 2.79 ms in FP64, 2.40 mixed, 3.57 with OCND2, against 2.56, 1.81 and 3.21 now.
 //
-// Wavefronts per workgroup (one workgroup a compute unit).  FP64: two per SIMD, 231 of 256
-// VGPRs.  Mixed: three per SIMD (163 of 168 VGPRs; two per SIMD: 2.17 ms).  Hail: two per SIMD
-// (256 VGPRs and a few spills: 3.33 ms; one per SIMD: 4.74).
+// Wavefronts per workgroup (one workgroup a compute unit).  FP64: two per SIMD, 233 of 256
+// VGPRs.  Mixed: three per SIMD (165 of 168 VGPRs; two per SIMD: 15 % slower).  Hail: two per SIMD
+// (256 VGPRs and a few spills: 3.30 ms; one per SIMD: 4.74).
 template <class R, bool HAIL = false> constexpr int micro_waves() { return sizeof(R) == 4 ? 12 : 8; }
 // Lookup tables staged in LDS: the ICE3 block; the hail kernel reads the wet-growth kernels
 // of hail, which follow it, from device memory.
@@ -631,10 +631,10 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
   int calls = 0;
   unsigned long long ncalls = 0, ncap = 0, nmicro = 0;
   bool done = false;              // this lane holds a point's end state, to be stored
-  double evap3d = 0., rvheni = 0.;
-  // Few chunks go one to a compute unit before a second to any (1,024 columns: 27.7 us, 35.0 with
-  // eight in a row to each); many go in rows of a workgroup's wavefronts, whose chunks are then
-  // neighbours (mixed path at 512x512x90: 1.88 ms, 1.93 the other way; FP64 the same).
+  double evap3d = 0., rvheni = 0., exnref = 1.;
+  // Few chunks go one to a compute unit before a second to any (1,024 columns: 26.7 us, 7 us more
+  // with eight in a row to each); many go in rows of a workgroup's wavefronts, whose chunks are
+  // then neighbours (mixed path at 512x512x90: 2.6 % faster; FP64 the same).
   const int cstep = gridDim.x * micro_waves<R, HAIL>();
   const int c0 = nchunk < 4 * cstep ? wid * (int)gridDim.x + (int)blockIdx.x
                                     : (int)blockIdx.x * micro_waves<R, HAIL>() + wid;
@@ -648,19 +648,25 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
         double t[NV], s[NV];
         micro_load<NV>(a, j, t, s);
         cit = a.src_ci[j];
+        // Every input is loaded here, not where the mask or the finish first needs it, a wait for
+        // memory later (512x512x90: FP64 2.72 -> 2.56 ms, mixed 1.89 -> 1.81, OCND2 3.37 -> 3.21).
+        // exn_ref stays in registers for the finish; the hail kernel has none left.
+        const double exn = a.exn[j], rhodref = a.rhodref[j], pabs = a.pabs[j], cldfr = a.cldfr[j],
+                     sigs = a.sigs[j];
+        MicroOcnd2 xo;
+        if constexpr (OCND2) xo = ocnd2_point(a, j);
+        if constexpr (!HAIL) exnref = a.exn_ref[j];
         rvheni = 0.;
         evap3d = 0.;
         int st = 0;
         calls = 0;
         if (micro_mask<OCND2, HAIL>(t, a, j)) {
           ++nmicro;
-          step_point(dt, a.exn[j], a.rhodref[j], a.pabs[j], a.cldfr[j], a.sigs[j], s, t, p);
+          step_point(dt, exn, rhodref, pabs, cldfr, sigs, s, t, p);
 #pragma unroll
           for (int f = 0; f < NV; ++f) vart[f] = t[f];
           time = 0.;
           const PointConst<R> pc = point_const<R>(p.rhodref);
-          MicroOcnd2 xo;
-          if constexpr (OCND2) xo = ocnd2_point(a, j);
           st = step_call<R, false, OCND2, HAIL>(dt, p, pc, vart, cit, time, S, calls,
                                                 DEFAULT_MAX_CALLS, tab, &xo, htab);
           if (st == 0) evap3d = (double)S.rrevav;
@@ -696,6 +702,7 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
             double t[NV], s[NV];
             micro_load<NV>(a, j, t, s);
             step_point(dt, a.exn[j], a.rhodref[j], a.pabs[j], a.cldfr[j], a.sigs[j], s, t, p);
+            if constexpr (!HAIL) exnref = a.exn_ref[j];
             active = true;
             rvheni = 0.;
           }
@@ -713,7 +720,8 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
       }
       if (done) {
         ncalls += calls < 0 ? -calls : calls;
-        micro_finish<HAIL>(a, j, vart, cit, evap3d, rvheni, calls);
+        if constexpr (HAIL) exnref = a.exn_ref[j];
+        micro_finish<HAIL>(a, j, vart, cit, evap3d, rvheni, calls, exnref);
         done = false;
       }
     }

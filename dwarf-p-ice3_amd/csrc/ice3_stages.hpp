@@ -322,7 +322,8 @@ __device__ __forceinline__ void micro_nucleation(const MicroArgs &a, size_t j, c
 // wr has hail last, and the hail source takes its tendency and negativity correction.
 template <bool HAIL = false>
 __device__ __forceinline__ void micro_finish(const MicroArgs &a, size_t j, const double *wr,
-                                             double cit, double evap3d, double rvheni, int calls) {
+                                             double cit, double evap3d, double rvheni, int calls,
+                                             double exnref) {
   constexpr int NV = HAIL ? 8 : 7;
   const double dt = a.dt, zinv = 1. / by(dt);
   double t[NV], s[NV];
@@ -331,7 +332,6 @@ __device__ __forceinline__ void micro_finish(const MicroArgs &a, size_t j, const
   rain_ice_factors<HAIL>(t, a.exn[j], lsfact, lvfact);
   rvheni = dmin(s[IRV], rvheni / by(dt));
   // 8.1 total tendencies
-  const double exnref = a.exn_ref[j];
   lsfact = lsfact / by(exnref);
   lvfact = lvfact / by(exnref);
   const double wrv = (wr[IRV] - t[IRV]) * zinv, wrc = (wr[IRC] - t[IRC]) * zinv;
@@ -378,7 +378,7 @@ __device__ __forceinline__ int micro_at(const MicroArgs &a, size_t j, const TB *
   } else {
     micro_nucleation<R, OCND2, HAIL>(a, j, wr, cit, rvheni);
   }
-  micro_finish<HAIL>(a, j, wr, cit, evap3d, rvheni, calls);
+  micro_finish<HAIL>(a, j, wr, cit, evap3d, rvheni, calls, a.exn_ref[j]);
   return calls;
 }
 
