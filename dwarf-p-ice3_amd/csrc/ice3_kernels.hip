@@ -1213,8 +1213,8 @@ extern "C" int ice3_ice_adjust_ocnd2(ice3_ctx *ctx, int ncol, int nlev, int ld, 
 // wavefront takes 6 us a level, so that 1,024 to 65,536 columns of 90 levels all take 0.53 to
 // 0.60 ms, against 0.08 to 0.44 ms for ICE_ADJUST point by point followed by k_sedim.  From
 // SEDIM_WALK_COLS (1.7 wavefronts per SIMD) on the walk saves more traffic than it waits: at
-// 98,304 columns 0.76 against 0.64 ms, at 114,688 0.78 against 0.75 (hail: 0.93 against 0.96),
-// at 131,072 0.81 against 0.85, at 262,144 1.51 against 1.72.
+// 98,304 columns 0.73 against 0.63 ms, at 106,496 0.73 against 0.71, at 114,688 0.743 against 0.741
+// (hail: 0.82 against 0.92), at 131,072 0.78 against 0.85, at 262,144 1.49 against 1.68.
 static hipError_t launch_adjust_sedim(const ice3_ctx *ctx, const AdjustArgs &aa, const SedimArgs &sa,
                                       hipStream_t s) {
   const dim3 gw((aa.ncol + 63) / 64), gp((aa.ncol + 255) / 256, aa.nlev);
