@@ -69,8 +69,7 @@ __global__ void __launch_bounds__(256) k_mlp_forward(MlpFwdArgs a) {
   __shared__ float sLoss[MLP_WAVES];
   const int lane = threadIdx.x % 64, w = threadIdx.x / 64, row0 = w * MLP_ROWS;
   const int p0 = blockIdx.x * MLP_TILE;
-  block_copy16(sW, a.wpk, MLP_NW * 2);
-  for (int q = threadIdx.x; q < MLP_NB; q += blockDim.x) sB[q] = a.params[MLP_NW + q];
+  stage_weights<64 * MLP_WAVES>(sW, sB, a.wpk, a.params);
   // input tile: 4 x 16 bytes per row
   for (int q = threadIdx.x; q < MLP_TILE * 4; q += blockDim.x) {
     const int r = q / 4, c = q % 4, p = p0 + r;
@@ -262,7 +261,7 @@ constexpr size_t MLP_BWD_LDS = (size_t)4 * BW_TILE * 2;
 // dW = H^T dZ the points are the contraction, so H and dZ of a layer go through LDS transposed;
 // dH = W dZ takes dZ from registers.  The backward tiles lie where the forward weights were, the
 // weights of a layer one layer ahead of their use.
-// 32,768 points (a tile for each compute unit), with the reduction: 54 us, against 208 us of
+// 32,768 points (a tile for each compute unit), with the reduction: 51 us, against 208 us of
 // k_mlp_forward (34, with 100 MB of pre-activations and activations saved), k_mlp_backward (112)
 // and a serial sum of the partials (62).  Bound by the latency of its ten phases between
 // barriers at two wavefronts a SIMD, and the 59 MB of partials written and read.
@@ -372,8 +371,7 @@ __global__ void __launch_bounds__(GRAD_THREADS) k_mlp_gradient(MlpGradArgs a) {
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     t[i] = live && 4 * g < MLP_NTARG ? a.target[(size_t)p * MLP_NTARG + 4 * g + i] : 0.f;
-  block_copy16(sWF, a.wpk, MLP_NW * 2);
-  for (int q = threadIdx.x; q < MLP_NB; q += blockDim.x) sB[q] = a.params[MLP_NW + q];
+  stage_weights<GRAD_THREADS>(sWF, sB, a.wpk, a.params);
   __syncthreads();
 
   // forward

@@ -142,11 +142,34 @@ __device__ __forceinline__ void mlp_product(const bf16x8 *sWpk, const bf16x8 (&x
     }
 }
 
-// Copy n elements global -> LDS with the whole workgroup (16-byte granules).
-__device__ __forceinline__ void block_copy16(void *dst, const void *src, int bytes) {
-  const int4 *s = (const int4 *)src;
-  int4 *d = (int4 *)dst;
-  for (int q = threadIdx.x; q < bytes / 16; q += blockDim.x) d[q] = s[q];
+// All packed weights and biases into LDS with a workgroup of NT threads, every load issued before the
+// first store.
+template <int NT>
+__device__ __forceinline__ void stage_weights(bf16x8 *sW, float *sB, const bf16x8 *__restrict__ wpk,
+                                              const float *__restrict__ params) {
+  constexpr int NQ = MLP_NW / 8, NL = (NQ + NT - 1) / NT, NBL = (MLP_NB + NT - 1) / NT;
+  bf16x8 v[NL];
+  float b[NBL];
+#pragma unroll
+  for (int l = 0; l < NL; ++l) {
+    const int q = threadIdx.x + l * NT;
+    v[l] = wpk[q < NQ ? q : 0];
+  }
+#pragma unroll
+  for (int l = 0; l < NBL; ++l) {
+    const int q = threadIdx.x + l * NT;
+    b[l] = params[MLP_NW + (q < MLP_NB ? q : 0)];
+  }
+#pragma unroll
+  for (int l = 0; l < NL; ++l) {
+    const int q = threadIdx.x + l * NT;
+    if (q < NQ) sW[q] = v[l];
+  }
+#pragma unroll
+  for (int l = 0; l < NBL; ++l) {
+    const int q = threadIdx.x + l * NT;
+    if (q < MLP_NB) sB[q] = b[l];
+  }
 }
 
 }  // namespace ice3

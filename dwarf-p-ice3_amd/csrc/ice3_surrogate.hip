@@ -98,8 +98,7 @@ __global__ void __launch_bounds__(64 * SGN_WAVES) k_sg_network(SurrogateArgs a) 
   const int pt = lane % 16, g = lane / 16;  // this lane's point of a tile, and its quarter of the units
   __bf16 *sX = (__bf16 *)(smem + MLP_NW * 2 + MLP_NB * 4 + w * SGN_WAVE_LDS);  // [64][SGN_XROW]
   float *sY = (float *)sX;                                                     // [64][SGN_YROW]
-  block_copy16(sW, a.wpk, MLP_NW * 2);
-  for (int q = threadIdx.x; q < MLP_NB; q += blockDim.x) sB[q] = a.params[MLP_NW + q];
+  stage_weights<64 * SGN_WAVES>(sW, sB, (const bf16x8 *)a.wpk, a.params);
   if (threadIdx.x < sizeof(nm) / 4) ((float *)&nm)[threadIdx.x] = ((const float *)a.norm)[threadIdx.x];
   __syncthreads();
   const unsigned int nchunk = (a.npts + 63) / 64, wid = w * gridDim.x + blockIdx.x;
