@@ -1213,8 +1213,8 @@ extern "C" int ice3_ice_adjust_ocnd2(ice3_ctx *ctx, int ncol, int nlev, int ld, 
 // wavefront takes 6 us a level, so that 1,024 to 65,536 columns of 90 levels all take 0.53 to
 // 0.60 ms, against 0.08 to 0.44 ms for ICE_ADJUST point by point followed by k_sedim.  From
 // SEDIM_WALK_COLS (1.7 wavefronts per SIMD) on the walk saves more traffic than it waits: at
-// 98,304 columns 0.73 against 0.63 ms, at 106,496 0.73 against 0.71, at 114,688 0.743 against 0.741
-// (hail: 0.82 against 0.92), at 131,072 0.78 against 0.85, at 262,144 1.49 against 1.68.
+// 98,304 columns 0.73 against 0.63 ms, at 106,496 0.73 against 0.71, at 114,688 0.74 against 0.74
+// (hail: 0.82 against 0.92), at 131,072 0.78 against 0.85, at 262,144 1.45 against 1.65.
 static hipError_t launch_adjust_sedim(const ice3_ctx *ctx, const AdjustArgs &aa, const SedimArgs &sa,
                                       hipStream_t s) {
   const dim3 gw((aa.ncol + 63) / 64), gp((aa.ncol + 255) / 256, aa.nlev);
@@ -1493,6 +1493,7 @@ extern "C" int ice3_adjust_rain_ice_stages(ice3_ctx *ctx, int prec, int ncol, in
   hipStream_t s = (hipStream_t)stream;
   const dim3 gp((ncol + 255) / 256, nlev);
   const bool split = ctx->sedim == ICE3_SEDIM_SPLI;
+  if ((stages & ICE3_STAGE_ADJUST) && (stages & ICE3_STAGE_SEDIMENTATION)) hand_ris_over(aa, sa);
   MARK(0);
   if (prec == ICE3_PREC_FP64 && !split && (stages & ICE3_STAGE_ADJUST) &&
       (stages & ICE3_STAGE_SEDIMENTATION)) {
@@ -1557,6 +1558,7 @@ extern "C" int ice3_adjust_rain_ice_ocnd2(ice3_ctx *ctx, int ncol, int nlev, int
   if (!sedim_fits(ctx, nlev)) return ICE3_EINVAL;
   const Ocnd2Args x{*in2, *out2, ctx->d_tiwmx};
   hipStream_t s = (hipStream_t)stream;
+  hand_ris_over(aa, sa);
   MARK(0);
   hipLaunchKernelGGL(k_ice_adjust_ocnd2, dim3((ncol + 255) / 256, nlev), dim3(256), 0, s, aa, x);
   HIPCHK(hipGetLastError());
@@ -1697,6 +1699,7 @@ extern "C" int ice3_adjust_rain_ice_hail(ice3_ctx *ctx, int ncol, int nlev, int 
   m.t[IRH] = hail->rhs; m.src[IRH] = hail->rhs_out; m.dst[IRH] = hail->rhs_out;
   if (!sedim_fits(ctx, nlev)) return ICE3_EINVAL;
   hipStream_t s = (hipStream_t)stream;
+  hand_ris_over(aa, sa);
   MARK(0);
   if (ctx->sedim == ICE3_SEDIM_SPLI) {
     hipLaunchKernelGGL(k_ice_adjust_hail, dim3((ncol + 255) / 256, nlev), dim3(256), 0, s, aa);
@@ -1769,6 +1772,7 @@ static int surrogate_step(ice3_ctx *ctx, int ncol, int nlev, int ld, double dt,
   g.counters = sg_counters;
   g.qcount = (unsigned int *)(wb + wl.qcount);
   unsigned int nseg = 0;
+  hand_ris_over(aa, sa);
   MARK(0);
   HIPCHK(launch_adjust_sedim(ctx, aa, sa, s));
   MARK(1);
