@@ -86,12 +86,13 @@ constexpr int SGN_WAVES = 12, SGN_MT = 2, SGN_PTS = 16 * SGN_MT;
 constexpr int SGN_XROW = 24, SGN_YROW = SGN_XROW / 2;
 constexpr size_t SGN_WAVE_LDS = 64 * SGN_XROW * 2;
 constexpr size_t SGN_LDS = (size_t)MLP_NW * 2 + MLP_NB * 4 + SGN_WAVES * SGN_WAVE_LDS;
-static_assert(SGN_LDS + sizeof(ice3_surrogate_norm) <= 160 * 1024, "k_sg_network LDS");
+static_assert(SGN_LDS + sizeof(ice3_surrogate_norm) + SGN_WAVES * 20 + 16 <= 160 * 1024, "k_sg_network LDS");
 static_assert(SG_WAVES % SGN_WAVES == 0 && MLP_NFEAT <= SGN_XROW && MLP_NTARG <= SGN_YROW, "k_sg_network layout");
 
 __global__ void __launch_bounds__(64 * SGN_WAVES) k_sg_network(SurrogateArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ __attribute__((aligned(16))) ice3_surrogate_norm nm;  // read by every point
+  __shared__ unsigned int sCnt[SGN_WAVES][5];
   bf16x8 *sW = (bf16x8 *)smem;
   float *sB = (float *)(smem + MLP_NW * 2);
   const int lane = threadIdx.x % 64, w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -173,11 +174,18 @@ __global__ void __launch_bounds__(64 * SGN_WAVES) k_sg_network(SurrogateArgs a) 
     if (flag > SG_OK) queue[nq + __popcll(rej & ((1ull << lane) - 1ull))] = (unsigned int)j;
     nq += __popcll(rej);
   }
+  // the counts, summed over the workgroup first: additions to one address follow one another
   if (lane == 0) {
     a.qcount[wid] = nq;
 #pragma unroll
-    for (int r = 0; r < 5; ++r)
-      if (cnt[r]) atomicAdd(&a.counters[r], (unsigned long long)cnt[r]);
+    for (int r = 0; r < 5; ++r) sCnt[w][r] = cnt[r];
+  }
+  __syncthreads();
+  if (threadIdx.x < 5) {
+    unsigned int n = 0;
+#pragma unroll
+    for (int i = 0; i < SGN_WAVES; ++i) n += sCnt[i][threadIdx.x];
+    if (n) atomicAdd(&a.counters[threadIdx.x], (unsigned long long)n);
   }
 }
 
