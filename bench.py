@@ -42,7 +42,7 @@ SEED = 20260003
 BYTES_PER_POINT = 320.0   # whole step: 25 inputs + 15 outputs, float64
 BYTES_PER_COLUMN = 48.0   # sigqsat + 5 surface precipitation fields
 # algorithmic bytes of each stage (per point, per column) as launched by the fused step
-STAGE_BYTES = {"ice_adjust": (232.0, 8.0),      # 19 reads + 10 writes; sigqsat
+STAGE_BYTES = {"ice_adjust": (224.0, 8.0),      # 19 reads + 9 writes (ri once); sigqsat
                "sedimentation": (80.0, 40.0),   # 6 reads + 4 writes; 5 precipitation fields
                # one column walk: 23 reads + 13 writes (ri once); sigqsat + precipitation
                "ice_adjust+sedimentation": (288.0, 48.0),

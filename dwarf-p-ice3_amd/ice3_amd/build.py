@@ -33,7 +33,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
 # -7 %; results bit for bit the same), and for the surrogate's network kernel (k_sg_network 5.79
 # ms at 512x512x90, 5.94 with the default one, 6.23 with max-ilp).
 # -fapprox-func for the physics kernels' device code: divisions become a reciprocal and
-# Newton steps (FP64: two steps and a residual correction, within 1 ulp and in practice
+# Newton steps (FP64: by() in ice3_physics.hpp, one step and a residual correction, in practice
 # correctly rounded; FP32: the hardware reciprocal, 1 ulp) instead of the scaled IEEE
 # sequence.  The FP64 outputs of the fused 512x512x90 step are bitwise those of the IEEE
 # build, 6 % faster; the mixed path is 8 % faster.  Every divisor on the path is a positive
