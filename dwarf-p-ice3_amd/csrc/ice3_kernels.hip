@@ -517,7 +517,7 @@ __global__ void __launch_bounds__(64 * SPLIT_COLS)
 // FP64 VALU issues about two thirds of the cycles.  Parking every unfinished point after its
 // hard call, so that soft passes were full, read every input line and wrote every output line
 // twice (10 GB at 512x512x90 against 5.3 algorithmic), as their lines had left the L2 by then:
-// 2.79 ms in FP64, 2.40 mixed, 3.57 with OCND2, against 2.56, 1.81 and 3.21 now.
+// 2.79 ms in FP64, 2.40 mixed, 3.57 with OCND2, against 2.56, 1.68 and 3.21 now.
 //
 // Wavefronts per workgroup (one workgroup a compute unit).  FP64: two per SIMD, 233 of 256
 // VGPRs.  Mixed: three per SIMD (165 of 168 VGPRs; two per SIMD: 15 % slower).  Hail: two per SIMD
@@ -533,12 +533,20 @@ template <bool HAIL> constexpr int micro_nv() { return HAIL ? 8 : 7; }
 template <class R, bool HAIL> constexpr int micro_ns() {
   return (int)(sizeof(typename StepStateFor<R, HAIL>::type) / sizeof(R));
 }
+// Fields of a chunk that its finish reads back from LDS instead of memory: the state at t, the
+// sources of rr, ri, rs, rg, and exn, in the mixed path (three wavefronts a SIMD, whose lines do
+// not all stay in L2 until then: 9.1 GB at 5.0 TB/s).  1.80 -> 1.68 ms at 512x512x90, with 20 park
+// slots instead of 49.  In FP64, bound by latency and with 13 slots left, 2.57 -> 2.59 ms, with
+// OCND2 3.22 -> 3.33.
+template <class R> constexpr int micro_stash() { return sizeof(R) == 4 ? 12 : 0; }
+template <class R> constexpr size_t micro_stash_bytes() { return (size_t)micro_stash<R>() * 64 * sizeof(double); }
 // Park slots per wavefront: what the LDS holds beside the tables, at most 63 (31 in FP64,
-// 49 in the mixed path, 24 with hail).
+// 20 in the mixed path, 24 with hail).
 template <class R, bool HAIL = false> constexpr int micro_park_cap() {
   const size_t slot = (micro_nv<HAIL>() + 2) * sizeof(double) + micro_ns<R, HAIL>() * sizeof(R) +
                       2 * sizeof(int);
-  const size_t n = (160 * 1024 - micro_tab_bytes<R, HAIL>()) / micro_waves<R, HAIL>() / slot;
+  const size_t n = ((160 * 1024 - micro_tab_bytes<R, HAIL>()) / micro_waves<R, HAIL>() -
+                    micro_stash_bytes<R>()) / slot;
   return n < 63 ? (int)n : 63;
 }
 
@@ -557,12 +565,14 @@ static_assert(sizeof(StepState<float>) == 32 * sizeof(float), "StepState layout"
 static_assert(sizeof(StepStateHail<double>) == 43 * sizeof(double), "StepStateHail layout");
 
 template <class R, bool HAIL = false> constexpr size_t micro_lds_bytes() {
-  return micro_tab_bytes<R, HAIL>() + micro_waves<R, HAIL>() * sizeof(MicroPark<R, HAIL>);
+  return micro_tab_bytes<R, HAIL>() +
+         micro_waves<R, HAIL>() * (sizeof(MicroPark<R, HAIL>) + micro_stash_bytes<R>());
 }
-static_assert(MicroPark<double>::CAP == 31 && MicroPark<float>::CAP == 49 &&
+static_assert(MicroPark<double>::CAP == 31 && MicroPark<float>::CAP == 20 &&
               MicroPark<double, true>::CAP == 24, "park capacity");
 static_assert(ICE3_T_ICE3 % 2 == 0, "k_micro stages the tables by pairs");
 static_assert(micro_lds_bytes<double>() <= 160 * 1024, "k_micro<double> LDS");
+static_assert(2 * micro_nv<false>() - 2 <= micro_stash<float>(), "k_micro<float> stash");
 static_assert(micro_lds_bytes<float>() <= 160 * 1024, "k_micro<float> LDS");
 static_assert(micro_lds_bytes<double, true>() <= 160 * 1024, "k_micro<double, false, true> LDS");
 
@@ -629,6 +639,10 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   MicroPark<R, HAIL> &pk =
       reinterpret_cast<MicroPark<R, HAIL> *>(micro_lds + micro_tab_bytes<R, HAIL>())[wid];
+  constexpr int ST = micro_stash<R>();
+  double (*stash)[64] = reinterpret_cast<double (*)[64]>(
+      micro_lds + micro_tab_bytes<R, HAIL>() + micro_waves<R, HAIL>() * sizeof(MicroPark<R, HAIL>) +
+      wid * micro_stash_bytes<R>());
   const unsigned long long below = (1ull << lane) - 1ull;  // lanes under this one
   const int cpl = (a.ncol + 63) >> 6;                       // chunks per level
   const int nchunk = cpl * a.nlev;
@@ -669,6 +683,13 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
         MicroOcnd2 xo;
         if constexpr (OCND2) xo = ocnd2_point(a, j);
         if constexpr (!HAIL) exnref = a.exn_ref[j];
+        if constexpr (ST != 0) {
+#pragma unroll
+          for (int f = 0; f < NV; ++f) stash[f][lane] = t[f];
+#pragma unroll
+          for (int f = 3; f < NV; ++f) stash[NV - 3 + f][lane] = s[f];
+          stash[2 * NV - 3][lane] = exn;
+        }
         rvheni = 0.;
         evap3d = 0.;
         int st = 0;
@@ -734,7 +755,20 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
       if (done) {
         ncalls += calls < 0 ? -calls : calls;
         if constexpr (HAIL) exnref = a.exn_ref[j];
-        micro_finish<HAIL>(a, j, vart, cit, evap3d, rvheni, calls, exnref);
+        double t[NV], s[NV], exn;
+        if (ST != 0 && own) {  // this chunk's points
+#pragma unroll
+          for (int f = 0; f < NV; ++f) t[f] = stash[f][lane];
+#pragma unroll
+          for (int f = 3; f < NV; ++f) s[f] = stash[NV - 3 + f][lane];
+          exn = stash[2 * NV - 3][lane];
+#pragma unroll
+          for (int f = 0; f < 3; ++f) s[f] = a.src[f][j];
+        } else {
+          micro_load<NV>(a, j, t, s);
+          exn = a.exn[j];
+        }
+        micro_finish<HAIL>(a, j, t, s, exn, vart, cit, evap3d, rvheni, calls, exnref);
         done = false;
       }
     }

@@ -344,15 +344,14 @@ __device__ __forceinline__ void micro_nucleation(const MicroArgs &a, size_t j, c
 // written before this point's stores).  rvheni: vapour nucleated outside the mask.  HAIL:
 // wr has hail last, and the hail source takes its tendency and negativity correction.
 template <bool HAIL = false>
-__device__ __forceinline__ void micro_finish(const MicroArgs &a, size_t j, const double *wr,
+__device__ __forceinline__ void micro_finish(const MicroArgs &a, size_t j, const double *t,
+                                             const double *s, double exn, const double *wr,
                                              double cit, double evap3d, double rvheni, int calls,
                                              double exnref) {
   constexpr int NV = HAIL ? 8 : 7;
   const double dt = a.dt, zinv = 1. / by(dt);
-  double t[NV], s[NV];
-  micro_load<NV>(a, j, t, s);
   double lsfact, lvfact;
-  rain_ice_factors<HAIL>(t, a.exn[j], lsfact, lvfact);
+  rain_ice_factors<HAIL>(t, exn, lsfact, lvfact);
   rvheni = dmin(s[IRV], rvheni / by(dt));
   // 8.1 total tendencies
   lsfact = lsfact / by(exnref);
@@ -401,7 +400,9 @@ __device__ __forceinline__ int micro_at(const MicroArgs &a, size_t j, const TB *
   } else {
     micro_nucleation<R, OCND2, HAIL>(a, j, wr, cit, rvheni);
   }
-  micro_finish<HAIL>(a, j, wr, cit, evap3d, rvheni, calls, a.exn_ref[j]);
+  double t[NV];
+  micro_load<NV>(a, j, t, s);
+  micro_finish<HAIL>(a, j, t, s, a.exn[j], wr, cit, evap3d, rvheni, calls, a.exn_ref[j]);
   return calls;
 }
 
