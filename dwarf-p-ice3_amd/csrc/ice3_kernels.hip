@@ -517,11 +517,11 @@ __global__ void __launch_bounds__(64 * SPLIT_COLS)
 // FP64 VALU issues about two thirds of the cycles.  Parking every unfinished point after its
 // hard call, so that soft passes were full, read every input line and wrote every output line
 // twice (10 GB at 512x512x90 against 5.3 algorithmic), as their lines had left the L2 by then:
-// 2.79 ms in FP64, 2.40 mixed, 3.57 with OCND2, against 2.56, 1.68 and 3.21 now.
+// 2.79 ms in FP64, 2.40 mixed, 3.57 with OCND2, against 2.40, 1.54 and 2.92 now.
 //
 // Wavefronts per workgroup (one workgroup a compute unit).  FP64: two per SIMD, 233 of 256
 // VGPRs.  Mixed: three per SIMD (165 of 168 VGPRs; two per SIMD: 15 % slower).  Hail: two per SIMD
-// (256 VGPRs and a few spills: 3.30 ms; one per SIMD: 4.74).
+// (256 VGPRs and a few spills: 3.06 ms; one per SIMD: 4.74 in an earlier form).
 template <class R, bool HAIL = false> constexpr int micro_waves() { return sizeof(R) == 4 ? 12 : 8; }
 // Lookup tables staged in LDS: the ICE3 block; the hail kernel reads the wet-growth kernels
 // of hail, which follow it, from device memory.
@@ -535,7 +535,7 @@ template <class R, bool HAIL> constexpr int micro_ns() {
 }
 // Fields of a chunk that its finish reads back from LDS instead of memory: the state at t, the
 // sources of rr, ri, rs, rg, and exn, in the mixed path (three wavefronts a SIMD, whose lines do
-// not all stay in L2 until then: 9.1 GB at 5.0 TB/s).  1.80 -> 1.68 ms at 512x512x90, with 20 park
+// not all stay in L2 until then: 9.1 GB, now 7.5).  1.80 -> 1.68 ms at 512x512x90, with 20 park
 // slots instead of 49.  In FP64, bound by latency and with 13 slots left, 2.57 -> 2.59 ms, with
 // OCND2 3.22 -> 3.33.
 template <class R> constexpr int micro_stash() { return sizeof(R) == 4 ? 12 : 0; }
@@ -566,7 +566,7 @@ static_assert(sizeof(StepStateHail<double>) == 43 * sizeof(double), "StepStateHa
 
 template <class R, bool HAIL = false> constexpr size_t micro_lds_bytes() {
   return micro_tab_bytes<R, HAIL>() +
-         micro_waves<R, HAIL>() * (sizeof(MicroPark<R, HAIL>) + micro_stash_bytes<R>());
+         micro_waves<R, HAIL>() * (sizeof(MicroPark<R, HAIL>) + micro_stash_bytes<R>()) + 16;
 }
 static_assert(MicroPark<double>::CAP == 31 && MicroPark<float>::CAP == 20 &&
               MicroPark<double, true>::CAP == 24, "park capacity");
@@ -633,6 +633,8 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
       }
     }
   }
+  int *next_chunk = reinterpret_cast<int *>(micro_lds + micro_lds_bytes<R, HAIL>() - 16);
+  if (threadIdx.x == 0) *next_chunk = micro_waves<R, HAIL>();
   __syncthreads();
   // hail: the wet-growth kernels of hail from device memory
   const double *htab = HAIL ? a.tab + ICE3_T_ICE3 : nullptr;
@@ -656,16 +658,21 @@ __global__ void __launch_bounds__((64 * micro_waves<R, HAIL>())) k_micro(MicroAr
   double vart[NV], cit = 0., time = 0.;
   typename StepStateFor<R, HAIL>::type S;
   int calls = 0;
-  unsigned int ncalls = 0, ncap = 0, nmicro = 0;  // of this lane: at most 2^18 points of 2^12 calls
+  unsigned int ncalls = 0, ncap = 0, nmicro = 0;  // of this lane: at most 2^18 points (256 CUs) of 2^12 calls
   bool done = false;              // this lane holds a point's end state, to be stored
   double evap3d = 0., rvheni = 0., exnref = 1.;
-  // Few chunks go one to a compute unit before a second to any (1,024 columns: 26.7 us, 7 us more
-  // with eight in a row to each); many go in rows of a workgroup's wavefronts, whose chunks are
-  // then neighbours (mixed path at 512x512x90: 2.6 % faster; FP64 the same).
-  const int cstep = gridDim.x * micro_waves<R, HAIL>();
-  const int c0 = nchunk < 4 * cstep ? wid * (int)gridDim.x + (int)blockIdx.x
-                                    : (int)blockIdx.x * micro_waves<R, HAIL>() + wid;
-  for (int c = c0;; c += cstep) {
+  // The workgroup's chunks, taken by its wavefronts in turn as they come free (a SIMD favours its
+  // oldest wavefront, and with a fixed share each the others ran on alone at the end: 2.56 ms at
+  // 512x512x90, 2.40 now; mixed 1.69 and 1.54, OCND2 3.22 and 2.92, hail 3.36 and 3.06).  Few chunks go
+  // one to a compute unit before a second to any (1,024 columns: 26.7 us, 7 us more with eight in a
+  // row to each); many go in rows of W to a workgroup, whose wavefronts' chunks are then
+  // neighbours (mixed path at 512x512x90: 2.6 % faster; FP64 the same).
+  constexpr int W = micro_waves<R, HAIL>();
+  const int cstep = gridDim.x * W;
+  const bool spread = nchunk < 4 * cstep;
+  const int c0 = spread ? (int)blockIdx.x : (int)blockIdx.x * W, cw = spread ? (int)gridDim.x : 1;
+  for (int n = wid;; n = __builtin_amdgcn_readfirstlane(lane == 0 ? atomicAdd(next_chunk, 1) : 0)) {
+    const int c = (n / W) * cstep + (n % W) * cw + c0;
     const bool more = c < nchunk;  // wave-uniform
     if (more) {
       const int k = c / cpl, i = (c - k * cpl) * 64 + lane;
@@ -863,21 +870,21 @@ __global__ void __launch_bounds__(256) k_micro_branches(MicroArgs a) {
   a.branches[j] = br;
 }
 
-// Plain microphysics over the surrogate's rejected points: block b runs the qcount[b]
-// points that wavefront b of the network stage queued.
+// Plain microphysics over the surrogate's rejected points: SG_PARTS blocks share the points that
+// a workgroup of the network stage queued.
 template <class R>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) k_micro_segments(MicroArgs a, const unsigned int *queue,
                                                        const unsigned int *qcount, unsigned int seg) {
-  const unsigned int n = qcount[blockIdx.x];
-  const unsigned int *list = queue + (size_t)blockIdx.x * seg;
-  for (unsigned int e = threadIdx.x; e < n; e += blockDim.x)
+  const unsigned int n = qcount[blockIdx.x / SG_PARTS];
+  const unsigned int *list = queue + (size_t)(blockIdx.x / SG_PARTS) * seg;
+  for (unsigned int e = blockIdx.x % SG_PARTS * 64 + threadIdx.x; e < n; e += SG_PARTS * 64)
     if (micro_at<R>(a, (size_t)list[e], a.tab) < 0 && a.capped) atomicAdd(a.capped, 1ull);
 }
 
 // Scratch layout of the surrogate step (bytes, 256-aligned blocks).  total is more than the queue
 // takes: it is what the interface asks of a work area and measures the allocation-free entry's
-// limit by (room for a network input, an output and a reason per point as well; 64 (SG_WAVES +
-// 1) words and SG_WAVES counts are fewer than its 256 x 2049 words beside the points').
+// limit by (room for a network input, an output and a reason per point as well; 64 (SG_BLOCKS +
+// 1) words and SG_BLOCKS counts are fewer than its 256 x 2049 words beside the points').
 struct SgWork {
   size_t queue, qcount, total;
 };
@@ -885,7 +892,7 @@ static SgWork sg_work_layout(size_t npts) {
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
   SgWork w;
   w.queue = 0;
-  w.qcount = al((npts + 64 * ((size_t)SG_WAVES + 1)) * 4);
+  w.qcount = al((npts + 64 * ((size_t)SG_BLOCKS + 1)) * 4);
   w.total = al(npts * 64) + al(npts * 32) + al(npts) + al((npts + 1 + 256 * 2049) * 4) + 8192;
   return w;
 }
@@ -1829,7 +1836,7 @@ static int surrogate_step(ice3_ctx *ctx, int ncol, int nlev, int ld, double dt,
   HIPCHK(surrogate_network_launch(g, ctx->ncu, &nseg, s));
   MARK(4);
   MARK(5);
-  hipLaunchKernelGGL(k_micro_segments<double>, dim3(nseg), dim3(64), 0, s, m,
+  hipLaunchKernelGGL(k_micro_segments<double>, dim3(nseg * SG_PARTS), dim3(64), 0, s, m,
                      (const unsigned int *)g.queue, (const unsigned int *)g.qcount, g.seg);
   HIPCHK(hipGetLastError());
   MARK(6);

@@ -69,30 +69,36 @@ __device__ __forceinline__ int sg_decode_point(const SurrogateArgs &a, const ice
 
 // ---- k_sg_network: features, range check, network, decode and checks of every point, and the
 // queue of those left to the FP64 microphysics.  Persistent grid, one workgroup a compute unit,
-// all weights resident in LDS; every wavefront takes 64-point chunks of its own, a lane a point for
-// features and decode, 32 points at a time through the network with their activations in
+// all weights resident in LDS; the wavefronts of a workgroup take its 64-point chunks in turn as
+// they come free, a lane a point for features and decode, 32 points at a time through the network with their activations in
 // registers, and no barrier after the weights are in.  The network's inputs and outputs (96
 // bytes a point, written and read) never leave LDS.
 // Bound by the VALU: of the 36,000 cycles a chunk issues for, the SiLUs take 25,000 (two
 // quarter-rate transcendentals, four other operations and half a conversion, 50 cycles a
-// wavefront of activations), sinhf of the outputs 3,700 and asinhf of the inputs 2,400; that is
-// 5.4 ms of the 5.79 for 512 x 512 x 90 points.  Three kernels, features 1.01, network 4.24 and decode 1.36
-// ms, the first and last of them at the memory's rate: 6.61.  Three wavefronts a SIMD, so that
-// one's matrix products and loads run beside the others' SiLUs (two: 6.13 ms).  The ranges and
-// scales in LDS: read from memory with a branch a feature, 6.00.
+// wavefront of activations), sinhf of the outputs 3,700 and asinhf of the inputs 2,400.
+// 512 x 512 x 90 points take 5.03 ms; three kernels, features 1.01, network 4.24 and decode 1.36
+// ms, the first and last of them at the memory's rate, 6.61.  Three wavefronts a SIMD, so that one's
+// matrix products and loads run beside the others' SiLUs; a SIMD favours its oldest wavefront, and
+// with a fixed share of the chunks each the others ran on alone at the end: 5.83 ms (two
+// wavefronts a SIMD 6.13; the ranges and scales read from memory with a branch a feature 6.00).
 constexpr int SGN_WAVES = 12, SGN_MT = 2, SGN_PTS = 16 * SGN_MT;
 // A point's row in LDS (48 bytes: no bank conflicts): its inputs, bf16, then in their place its
 // outputs, fp32.
 constexpr int SGN_XROW = 24, SGN_YROW = SGN_XROW / 2;
 constexpr size_t SGN_WAVE_LDS = 64 * SGN_XROW * 2;
 constexpr size_t SGN_LDS = (size_t)MLP_NW * 2 + MLP_NB * 4 + SGN_WAVES * SGN_WAVE_LDS;
-static_assert(SGN_LDS + sizeof(ice3_surrogate_norm) + SGN_WAVES * 20 + 16 <= 160 * 1024, "k_sg_network LDS");
-static_assert(SG_WAVES % SGN_WAVES == 0 && MLP_NFEAT <= SGN_XROW && MLP_NTARG <= SGN_YROW, "k_sg_network layout");
+static_assert(SGN_LDS + sizeof(ice3_surrogate_norm) + SGN_WAVES * 20 + 32 <= 160 * 1024, "k_sg_network LDS");
+static_assert(MLP_NFEAT <= SGN_XROW && MLP_NTARG <= SGN_YROW, "k_sg_network layout");
 
 __global__ void __launch_bounds__(64 * SGN_WAVES) k_sg_network(SurrogateArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ __attribute__((aligned(16))) ice3_surrogate_norm nm;  // read by every point
   __shared__ unsigned int sCnt[SGN_WAVES][5];
+  __shared__ unsigned int sNext, sQueued;  // the next of the workgroup's chunks, points rejected
+  if (threadIdx.x == 0) {
+    sNext = SGN_WAVES;
+    sQueued = 0;
+  }
   bf16x8 *sW = (bf16x8 *)smem;
   float *sB = (float *)(smem + MLP_NW * 2);
   const int lane = threadIdx.x % 64, w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -102,11 +108,12 @@ __global__ void __launch_bounds__(64 * SGN_WAVES) k_sg_network(SurrogateArgs a) 
   stage_weights<64 * SGN_WAVES>(sW, sB, (const bf16x8 *)a.wpk, a.params);
   if (threadIdx.x < sizeof(nm) / 4) ((float *)&nm)[threadIdx.x] = ((const float *)a.norm)[threadIdx.x];
   __syncthreads();
-  const unsigned int nchunk = (a.npts + 63) / 64, wid = w * gridDim.x + blockIdx.x;
-  unsigned int *queue = a.queue + (size_t)wid * a.seg;
-  unsigned int nq = 0;                 // rejected points so far (uniform)
+  const unsigned int nchunk = (a.npts + 63) / 64;
+  unsigned int *queue = a.queue + (size_t)blockIdx.x * a.seg;
   unsigned int cnt[5] = {0, 0, 0, 0, 0};
-  for (unsigned int c = wid; c < nchunk; c += gridDim.x * SGN_WAVES) {
+  for (unsigned int n = w;; n = __builtin_amdgcn_readfirstlane(lane == 0 ? atomicAdd(&sNext, 1u) : 0u)) {
+    const unsigned int c = n * gridDim.x + blockIdx.x;
+    if (c >= nchunk) break;
     const unsigned int q = c * 64 + lane;
     int flag = -1;
     size_t j = 0;
@@ -171,16 +178,18 @@ __global__ void __launch_bounds__(64 * SGN_WAVES) k_sg_network(SurrogateArgs a) 
 #pragma unroll
     for (int r = 0; r < 5; ++r) cnt[r] += __popcll(__ballot(flag == r));
     const unsigned long long rej = __ballot(flag > SG_OK);
-    if (flag > SG_OK) queue[nq + __popcll(rej & ((1ull << lane) - 1ull))] = (unsigned int)j;
-    nq += __popcll(rej);
+    if (rej != 0) {  // uniform
+      const unsigned int at = __builtin_amdgcn_readfirstlane(
+          lane == 0 ? atomicAdd(&sQueued, (unsigned int)__popcll(rej)) : 0u);
+      if (flag > SG_OK) queue[at + __popcll(rej & ((1ull << lane) - 1ull))] = (unsigned int)j;
+    }
   }
   // the counts, summed over the workgroup first: additions to one address follow one another
-  if (lane == 0) {
-    a.qcount[wid] = nq;
+  if (lane == 0)
 #pragma unroll
     for (int r = 0; r < 5; ++r) sCnt[w][r] = cnt[r];
-  }
   __syncthreads();
+  if (threadIdx.x == 64) a.qcount[blockIdx.x] = sQueued;
   if (threadIdx.x < 5) {
     unsigned int n = 0;
 #pragma unroll
@@ -191,11 +200,11 @@ __global__ void __launch_bounds__(64 * SGN_WAVES) k_sg_network(SurrogateArgs a) 
 
 hipError_t surrogate_network_launch(SurrogateArgs &a, int ncu, unsigned int *nseg, hipStream_t s) {
   const unsigned int nchunk = (a.npts + 63) / 64;
-  unsigned int nblk = SG_WAVES / SGN_WAVES;  // one chunk to a compute unit before a second to any
+  unsigned int nblk = SG_BLOCKS;
   if (nblk > (unsigned int)ncu) nblk = ncu;
   if (nblk > nchunk) nblk = nchunk;
-  *nseg = nblk * SGN_WAVES;
-  a.seg = (nchunk + *nseg - 1) / *nseg * 64;
+  *nseg = nblk;
+  a.seg = (nchunk + nblk - 1) / nblk * 64;
   hipLaunchKernelGGL(k_sg_network, dim3(nblk), dim3(64 * SGN_WAVES), SGN_LDS, s, a);
   return hipGetLastError();
 }

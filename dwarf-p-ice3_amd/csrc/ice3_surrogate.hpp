@@ -4,9 +4,9 @@
 
 namespace ice3 {
 
-// Wavefronts of the network stage's grid at most, each with a queue segment of its own: a fixed
-// count (twelve on each of 256 compute units), so that the scratch depends on the problem only.
-constexpr unsigned int SG_WAVES = 3072;
+// Workgroups of the network stage at most, each with a queue segment of its own: a fixed count, so
+// that the scratch depends on the problem only.  SG_PARTS wavefronts of the fallback share a segment.
+constexpr unsigned int SG_BLOCKS = 256, SG_PARTS = 12;
 
 struct SurrogateArgs {
   MicroArgs m;
@@ -15,8 +15,8 @@ struct SurrogateArgs {
   float budget_tol, neg_tol;
   const void *wpk;                   // packed bf16 weights
   const float *params;               // fp32 parameters (biases)
-  unsigned int *queue;               // rejected points' offsets, a segment of seg per wavefront
-  unsigned int *qcount;              // their number per wavefront
+  unsigned int *queue;               // rejected points' offsets, a segment of seg per workgroup
+  unsigned int *qcount;              // their number per workgroup
   unsigned int seg;
   unsigned long long *counters;      // 5 entries, see include/ice3.h
 };
@@ -25,7 +25,7 @@ __device__ __forceinline__ size_t point_offset(const MicroArgs &m, unsigned int 
   return (size_t)(q / m.ncol) * m.ld + q % m.ncol;
 }
 
-// Sets a.seg, launches the stage over ncu compute units and returns its number of wavefronts (queue
+// Sets a.seg, launches the stage over ncu compute units and returns its number of workgroups (queue
 // segments) in nseg.
 hipError_t surrogate_network_launch(SurrogateArgs &a, int ncu, unsigned int *nseg, hipStream_t s);
 
