@@ -78,8 +78,9 @@ __global__ void __launch_bounds__(64) k_adjust_sedim(AdjustArgs aa, SedimArgs a)
 }
 
 // ---- hail (KRR=7), FP64: ICE_ADJUST with the hail heat capacity (one thread per point),
-// and that and the sedimentation with hail in one column walk for the fused step; the microphysics is k_micro<double, false, true> (k_micro_points<double, false,
-// true> when the context sets another sub-step cap).
+// and that and the sedimentation with hail in one column walk for the fused step; the
+// microphysics is k_micro<double, false, true> (k_micro_points<double, false, true> when the
+// context sets another sub-step cap).
 __global__ void __launch_bounds__(256) k_ice_adjust_hail(AdjustArgs a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.ncol) return;
@@ -185,11 +186,12 @@ __global__ void __launch_bounds__(256) k_transpose(TransposeArgs a) {
 // wavefront, and the flux entering level k from above comes from the next lane.  A workgroup
 // of SPLIT_COLS wavefronts takes as many adjacent columns: their inputs are read in rows of
 // SPLIT_COLS doubles, every load issued before the first wait, and handed through LDS to the
-// columns' wavefronts, up to SPLIT_BATCH fields at a time; the outputs go back the same way.  The two workgroups that take the halves of a 16-column row
-// run on the same XCD, so that the row's cache lines are fetched once.  While a wavefront's
+// columns' wavefronts, up to SPLIT_BATCH fields at a time; the outputs go back the same way.  The
+// two workgroups that take the halves of a 16-column row run on the same XCD, so that the row's
+// cache lines are fetched once.  While a wavefront's
 // state fits 128 registers (one slot, or two without hail) two workgroups share a compute
 // unit, one's loads overlapping the other's sub-steps.
-// 65,536 columns of 90 levels: 484 us, the VALU 57 % busy and 2.6 TB/s, 504 with each batch's loads
+// 65,536 columns of 90 levels: 484 us, the VALU 69 % busy and 2.6 TB/s, 504 with each batch's loads
 // waited for before the next batch's were issued (10,007 columns: 81, 88).
 constexpr int SPLIT_COLS = 8, SPLIT_BATCH = 8;
 template <int L, bool HAIL> constexpr int split_wpe() { return L == 1 || (L == 2 && !HAIL) ? 4 : 2; }

@@ -70,9 +70,10 @@ __device__ __forceinline__ int sg_decode_point(const SurrogateArgs &a, const ice
 // ---- k_sg_network: features, range check, network, decode and checks of every point, and the
 // queue of those left to the FP64 microphysics.  Persistent grid, one workgroup a compute unit,
 // all weights resident in LDS; the wavefronts of a workgroup take its 64-point chunks in turn as
-// they come free, a lane a point for features and decode, 32 points at a time through the network with their activations in
-// registers, and no barrier after the weights are in.  The network's inputs and outputs (96
-// bytes a point, written and read) never leave LDS.
+// they come free, a lane a point for features and decode, 32 points at a time through the
+// network with their activations in registers, and no barrier between the weights' arrival and
+// the final counts.  The network's inputs and outputs (96 bytes a point, written and read)
+// never leave LDS.
 // Bound by the VALU: of the 36,000 cycles a chunk issues for, the SiLUs take 25,000 (two
 // quarter-rate transcendentals, four other operations and half a conversion, 50 cycles a
 // wavefront of activations), sinhf of the outputs 3,700 and asinhf of the inputs 2,400.

@@ -30,8 +30,8 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
 # allocator has failed on it).
 # The iterative ILP scheduler for the physics kernels: they run at a fixed two (k_micro) or four
 # (k_adjust_sedim) wavefronts per SIMD and hide latency mostly within a wavefront (k_micro
-# -7 %; results bit for bit the same), and for the surrogate's network kernel (k_sg_network 5.79
-# ms at 512x512x90, 5.94 with the default one, 6.23 with max-ilp).
+# -7 %; results bit for bit the same), and for the surrogate's network kernel (k_sg_network 2 %
+# slower with the default one, 7 % with max-ilp).
 # -fapprox-func for the physics kernels' device code: divisions become a reciprocal and
 # Newton steps (FP64: by() in ice3_physics.hpp, one step and a residual correction, in practice
 # correctly rounded; FP32: the hardware reciprocal, 1 ulp) instead of the scaled IEEE
