@@ -17,6 +17,13 @@
 
 namespace ice3 {
 
+// The wavefront's issue priority on its SIMD (0 to 3); nothing in a CPU build of the stages.
+template <int N> __device__ __forceinline__ void wave_priority() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_s_setprio(N);
+#endif
+}
+
 struct AdjustArgs {
   int ncol, nlev, ld;
   double dt;
@@ -185,16 +192,23 @@ __device__ __forceinline__ void sedim_column(const SedimArgs &a, int i) {
 // adjusted source held in a register.  The sedimentation of a level needs only that level
 // and the flux from above, so the results are those of adjust_at over all points followed
 // by sedim_column.  HAIL: ICE_ADJUST with the hail heat capacity, and hail sediments.
+// A wavefront's priority falls with each quarter of its column, so that those behind catch up: a SIMD
+// favours its oldest, and the last ran on alone (262,144 columns 1.47 -> 1.43 ms, 150,000 0.98 ->
+// 0.91; hail 1.60 -> 1.54, 1.10 -> 1.01).
 // A level's inputs are all named before the first store, which the compiler would not move
-// a load across: 1.45 ms at 262,144 columns of 90 levels (7.0 GB, 4.8 TB/s, the VALU 71 % busy),
+// a load across: 1.43 ms at 262,144 columns of 90 levels (6.8 GB, 4.8 TB/s, the VALU 80 % busy),
 // 0.03 more with the sedimentation's loads after the adjustment's stores.
 template <class R, bool HAIL = false>
 __device__ __forceinline__ void adjust_sedim_column(const AdjustArgs &aa, const SedimArgs &a, int i) {
   const double dt = a.dt;
   double fr = 0., fi = 0., fs = 0., fg = 0., fh = 0.;
   const double sigqsat = aa.in.sigqsat[i];
+  wave_priority<3>();
   for (int k = a.nlev - 1; k >= 0; --k) {
     const size_t j = (size_t)k * a.ld + i;
+    if (k == 3 * a.nlev / 4) wave_priority<2>();
+    if (k == a.nlev / 2) wave_priority<1>();
+    if (k == a.nlev / 4) wave_priority<0>();
     const AdjustPoint p = adjust_load<HAIL>(aa, sigqsat, j);
     const double rho = a.rhodref[j], dz = a.dzz[j];
     double rrs = a.src_rr[j], rss = a.src_rs[j], rgs = a.src_rg[j], rhs = 0.;
