@@ -78,6 +78,12 @@ __global__ void __launch_bounds__(128 * (HAIL ? 5 : 4)) k_sedim(SedimArgs a) {
     load_level(1);
   }
   __syncthreads();
+  // the recurrences, pristine ice's first of all, before the own-content halves that they wait for
+  // least: 1,024 columns 61 -> 58 us (float 39.8 -> 35.4), 1 % at 65,536
+  if (!own) {
+    if (sp == 1) wave_priority<3>();
+    else wave_priority<1>();
+  }
   double flux = 0.;
   for (int t = 0, b = 0, f = 0; t <= ng; ++t, f ^= 1) {
     const int bn = b == 2 ? 0 : b + 1, bp = b == 0 ? 2 : b - 1;  // buffers of groups t + 1, t - 1
