@@ -23,9 +23,9 @@ namespace ice3 {
 // load is issued a step before its use.
 //
 // Few columns: bound by the recurrence (pristine ice's two logarithms and exponential, about
-// 0.7 us a level).  1,024 columns of 90 levels take 62 us (one thread per column, four species
+// 0.7 us a level).  1,024 columns of 90 levels take 59 us (one thread per column, four species
 // after one another: 292 us; four wavefronts without the own-content half split off: 104 us).
-// Many columns: bound by the VALU (76 % busy).  65,536 columns: 190 us (339), 262,144: 714 us
+// Many columns: bound by the VALU (76 % busy).  65,536 columns: 183 us (339), 262,144: 683 us
 // (705).  Groups of three levels keep four workgroups' LDS on a compute unit; four levels took
 // 206 us at 65,536 columns.  The Horner coefficients as scalars, hoisted out of the loop by
 // machine LICM, are worth 9 us at 1,024 columns and 20 us at 65,536 against vector ones.
