@@ -196,7 +196,7 @@ __device__ __forceinline__ void sedim_column(const SedimArgs &a, int i) {
 // favours its oldest, and the last ran on alone (262,144 columns 1.47 -> 1.43 ms, 150,000 0.98 ->
 // 0.91; hail 1.60 -> 1.54, 1.10 -> 1.01).
 // A level's inputs are all named before the first store, which the compiler would not move
-// a load across: 1.43 ms at 262,144 columns of 90 levels (6.8 GB, 4.8 TB/s, the VALU 80 % busy),
+// a load across: 1.43 ms at 262,144 columns of 90 levels (6.8 GB, 4.8 TB/s, the VALU 86 % busy),
 // 0.03 more with the sedimentation's loads after the adjustment's stores.
 template <class R, bool HAIL = false>
 __device__ __forceinline__ void adjust_sedim_column(const AdjustArgs &aa, const SedimArgs &a, int i) {
