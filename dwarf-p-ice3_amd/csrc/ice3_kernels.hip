@@ -1414,8 +1414,8 @@ static int launch_split_keep(ice3_ctx *ctx, int nlev, int ld, const SedimArgs &s
 }
 
 // The rain_ice entry points: checks, the sedimentation, the microphysics.  The sources are read
-// from src and written to io (and hail->rhs); either may be the other's array.  in2 selects
-// OCND2, hail KRR=7.
+// from src and written to io (and hail->rhs), each from its own array or from the one it is
+// written to.  in2 selects OCND2, hail KRR=7.
 static hipError_t launch_micro_hail(const ice3_ctx *ctx, const MicroArgs &m, hipStream_t s);
 
 static int rain_ice_call(ice3_ctx *ctx, int prec, int ncol, int nlev, int ld, double dt,
@@ -1502,6 +1502,27 @@ extern "C" int ice3_rain_ice_hail(ice3_ctx *ctx, int ncol, int nlev, int ld, dou
                        stream);
 }
 
+// Whether an array of src is an output other than the one of the same name.  The sedimentation's
+// wavefronts each write their own species while others still read, and the microphysics writes
+// some points while others wait, so such a source would be overwritten before it is read.
+static bool crossed_sources(const ice3_rain_ice_src *src, const ice3_rain_ice_inout *io,
+                            const ice3_rain_ice_out *out, const ice3_hail *hail) {
+  const double *const s[9] = {src->ths, src->rvs, src->rcs, src->rrs, src->ris,
+                              src->rss, src->rgs, src->ci,  hail ? src->rhs : nullptr};
+  const double *const w[9] = {io->ths, io->rvs, io->rcs, io->rrs, io->ris,
+                              io->rss, io->rgs, io->ci,  hail ? hail->rhs : nullptr};
+  const double *const o[8] = {out->evap3d, out->rainfr, out->inprc, out->inprr, out->inpri,
+                              out->inprs,  out->inprg,  hail ? hail->inprh : nullptr};
+  for (int a = 0; a < 9; ++a) {
+    if (!s[a]) continue;
+    for (int b = 0; b < 9; ++b)
+      if (a != b && s[a] == w[b]) return true;
+    for (int b = 0; b < 8; ++b)
+      if (s[a] == o[b]) return true;
+  }
+  return false;
+}
+
 extern "C" int ice3_rain_ice_from(ice3_ctx *ctx, int prec, int ncol, int nlev, int ld, double dt,
                                   const ice3_rain_ice_in *in, const ice3_rain_ocnd2_in *in2,
                                   const ice3_rain_ice_src *src, const ice3_rain_ice_inout *io,
@@ -1510,6 +1531,7 @@ extern "C" int ice3_rain_ice_from(ice3_ctx *ctx, int prec, int ncol, int nlev, i
   if (!ctx || !in || !src || !io || !out || !known_prec(prec) || (in2 && hail) ||
       ((in2 || hail) && prec != ICE3_PREC_FP64))
     return ICE3_EINVAL;
+  if (!empty_domain(ncol, nlev, ld, dt) && crossed_sources(src, io, out, hail)) return ICE3_EINVAL;
   return rain_ice_call(ctx, prec, ncol, nlev, ld, dt, in, in2, src, io, out, hail, stats, stream);
 }
 

@@ -243,9 +243,10 @@ int ice3_rain_ice_hail(ice3_ctx *ctx, int ncol, int nlev, int ld, double dt,
                        const ice3_stats *stats, void *stream);
 
 /* RAIN_ICE with the sources read from src and written to io (and hail->rhs): ice3_rain_ice
- * without the copies that a caller who keeps the sources at entry would make.  Any array of src
- * may be the one io (hail) writes.  in2 (or NULL): as ice3_rain_ice_ocnd2; hail (or NULL): as
- * ice3_rain_ice_hail, its source read from src->rhs; not both, and in FP64. */
+ * without the copies that a caller who keeps the sources at entry would make.  Each array of src
+ * may be the one of the same name that io (hail) writes, and overlaps no other output: one that
+ * is another output's array returns ICE3_EINVAL.  in2 (or NULL): as ice3_rain_ice_ocnd2; hail (or
+ * NULL): as ice3_rain_ice_hail, its source read from src->rhs; not both, and in FP64. */
 typedef struct {
   const double *ths, *rvs, *rcs, *rrs, *ris, *rss, *rgs, *ci;
   const double *rhs;    /* with hail; else NULL */
