@@ -3,6 +3,7 @@ from __future__ import annotations
 
 import ctypes
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -64,9 +65,16 @@ def columns_of(fields: dict, layout: str, *, device):
     return out, fresh
 
 
-def column_shape(x, layout: str, name: str) -> tuple:
-    """The (nlev, ncol) shape as_columns(x) would have, without making it."""
-    shape = tuple(x.shape) if hasattr(x, "shape") else tuple(torch.as_tensor(x).shape)
+def column_shape(x, layout: str, name: str, *, device) -> tuple:
+    """The (nlev, ncol) shape as_columns(x) would have, without making it, of a field that no kernel
+    reads.  What as_columns refuses (a type, a dtype, strides or a device that it cannot convert) is
+    refused here too: an array is converted as far as the host goes, anything else altogether."""
+    if isinstance(x, np.ndarray):
+        x = torch.as_tensor(x, dtype=torch.float64)
+    elif type(x) is not torch.Tensor or x.layout is not torch.strided or x.is_quantized or \
+            x.device.type not in ("cuda", "cpu"):
+        return tuple(as_columns(x, layout, device=device, name=name).shape)
+    shape = tuple(x.shape)
     if layout == "columns":
         if len(shape) != 2:
             raise ValueError(f"{name}: expected a (nlev, ncol) array, got {shape}")

@@ -144,8 +144,10 @@ class RainIce(_Base):
         fresh = {k for k, v in read.items() if v in fresh}
         nlev, ncol = f["tht"].shape
         for k, v in self._UNREAD.items():  # taken for the interface: the kernels read none of them
-            if v in state and k not in f and column_shape(state[v], layout, v) != (nlev, ncol):
-                raise ValueError(f"{k}: shape {column_shape(state[v], layout, v)} != {(nlev, ncol)}")
+            if v in state and k not in f:
+                got = column_shape(state[v], layout, v, device=self.device)
+                if got != (nlev, ncol):
+                    raise ValueError(f"{k}: shape {got} != {(nlev, ncol)}")
         for k, v in f.items():
             if v.shape != (nlev, ncol):
                 raise ValueError(f"{k}: shape {tuple(v.shape)} != {(nlev, ncol)}")
@@ -214,7 +216,7 @@ class AdjustRainIce(_Base):
             if nlev < 2:
                 raise ValueError("the OCND2 branch needs at least two levels")
         for k, v in {**{k: v.shape for k, v in g.items()},
-                     "rhodj": column_shape(f["rhodj"], layout, "rhodj")}.items():
+                     "rhodj": column_shape(f["rhodj"], layout, "rhodj", device=self.device)}.items():
             if v != (nlev, ncol):
                 raise ValueError(f"{k}: shape {tuple(v)} != {(nlev, ncol)}")
         g.setdefault("rhodj", g["rhodref"])

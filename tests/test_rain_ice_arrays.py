@@ -56,3 +56,52 @@ def test_crossed_sources_are_refused(source):
 
 def test_empty_domain_follows_no_pointer():
     assert _from("rrs", "rss", ncol=0) == _lib.ICE3_OK
+
+
+UNREADABLE = {
+    "objects": lambda np, torch: np.full((3, 4), None, dtype=object),
+    "texts": lambda np, torch: np.full((3, 4), "1.0"),
+    "byte order": lambda np, torch: np.zeros((3, 4), dtype=">f8"),
+    "negative strides": lambda np, torch: np.zeros((3, 4))[::-1],
+    "no data": lambda np, torch: torch.zeros((3, 4), dtype=torch.float64, device="meta"),
+    "sparse": lambda np, torch: torch.zeros((3, 4), dtype=torch.float64).to_sparse(),
+    "ragged": lambda np, torch: [[0.0, 1.0], [0.0]],
+    "nothing": lambda np, torch: None,
+}
+READABLE = {
+    "tensor": lambda np, torch: torch.zeros((3, 4), dtype=torch.float64),
+    "single": lambda np, torch: torch.zeros((3, 4)),
+    "view": lambda np, torch: torch.zeros((4, 3), dtype=torch.float64).t(),
+    "array": lambda np, torch: np.zeros((3, 4), dtype=np.float32),
+    "integers": lambda np, torch: np.zeros((3, 4), dtype=np.int64),
+    "lists": lambda np, torch: [[0.0] * 4] * 3,
+}
+
+
+@pytest.mark.parametrize("layout", ["columns", "jax"])
+@pytest.mark.parametrize("form", [*UNREADABLE, *READABLE])
+def test_unread_fields_are_taken_and_refused_as_read_ones(form, layout):
+    """A field that the interface takes and no kernel reads (rhodj): its shape alone is looked at, and
+    it is refused where a field that is read would be."""
+    import numpy as np
+    import torch
+    from ice3_amd._fields import as_columns, column_shape
+    x = {**UNREADABLE, **READABLE}[form](np, torch)
+    if form in READABLE:
+        assert column_shape(x, layout, "x", device="cpu") == tuple(as_columns(x, layout, device="cpu", name="x").shape)
+        return
+    with pytest.raises(Exception) as read:
+        t = as_columns(x, layout, device="cpu", name="x")
+        t.data_ptr()  # what the call does with a field that it reads
+    with pytest.raises(read.type):
+        column_shape(x, layout, "x", device="cpu")
+
+
+@pytest.mark.parametrize("shape,layout", [((3,), "columns"), ((3,), "jax"), ((2, 3, 4), "columns")])
+def test_unread_fields_of_another_rank_are_refused(shape, layout):
+    import numpy as np
+    import torch
+    from ice3_amd._fields import column_shape
+    for x in (np.zeros(shape), torch.zeros(shape)):
+        with pytest.raises(ValueError, match="x: expected"):
+            column_shape(x, layout, "x", device="cpu")
