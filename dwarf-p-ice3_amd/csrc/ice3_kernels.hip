@@ -1205,9 +1205,9 @@ extern "C" int ice3_transpose_fields(int nfield, const double *const *src, doubl
     a.src[q] = src[q];
     a.dst[q] = dst[q];
   }
-  a.rows = rows; a.cols = cols; a.col_tiles = (cols + TR_COLS - 1) / TR_COLS;
+  a.rows = rows; a.cols = cols; a.col_tiles = (cols - 1) / TR_COLS + 1;
   const size_t blocks = ((size_t)rows + TR_ROWS - 1) / TR_ROWS * a.col_tiles;
-  if (blocks > 0x7fffffff) return ICE3_EINVAL;
+  if (blocks >= (size_t)1 << 24) return ICE3_EINVAL;  // a launch takes fewer than 2^32 threads along an axis
   hipLaunchKernelGGL(k_transpose, dim3((unsigned)blocks, nfield), dim3(256), 0, (hipStream_t)stream, a);
   HIPCHK(hipGetLastError());
   return ICE3_OK;

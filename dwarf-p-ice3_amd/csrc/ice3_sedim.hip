@@ -168,25 +168,25 @@ template <class R> __global__ void __launch_bounds__(256) k_sedim_walk(SedimArgs
 }
 
 template <class R> hipError_t sedim_launch(const SedimArgs &sa, int ncu, hipStream_t s) {
-  const dim3 g((sa.ncol + 63) / 64);
   if constexpr (sizeof(R) == sizeof(float)) {
     if (sa.ncol >= SEDIM_WALK_COLS * ncu) {
       hipLaunchKernelGGL(k_sedim_walk<R>, dim3((sa.ncol + 255) / 256), dim3(256), 0, s, sa);
       return hipGetLastError();
     }
   }
-  if constexpr (sizeof(R) == sizeof(double)) {
-    if (sa.src_rh) {
-      hipLaunchKernelGGL((k_sedim<double, false, true>), g, dim3(640), 0, s, sa);
-      return hipGetLastError();
-    }
-    if (sa.zzz) {
-      hipLaunchKernelGGL((k_sedim<double, true>), g, dim3(512), 0, s, sa);
-      return hipGetLastError();
-    }
+  for (int c = 0;;) {
+    const SedimArgs part = sedim_columns(sa, c, SEDIM_LAUNCH_COLS);
+    const dim3 g((part.ncol + 63) / 64);
+    if (sizeof(R) == sizeof(double) && part.src_rh)
+      hipLaunchKernelGGL((k_sedim<double, false, true>), g, dim3(640), 0, s, part);
+    else if (sizeof(R) == sizeof(double) && part.zzz)
+      hipLaunchKernelGGL((k_sedim<double, true>), g, dim3(512), 0, s, part);
+    else
+      hipLaunchKernelGGL(k_sedim<R>, g, dim3(512), 0, s, part);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || part.ncol == sa.ncol - c) return e;
+    c += part.ncol;
   }
-  hipLaunchKernelGGL(k_sedim<R>, g, dim3(512), 0, s, sa);
-  return hipGetLastError();
 }
 
 template hipError_t sedim_launch<double>(const SedimArgs &, int, hipStream_t);

@@ -12,6 +12,8 @@
 // these functions.  Everything here is force-inlined and every array index is a
 // compile-time constant after unrolling, so the state lives in registers.
 #pragma once
+#include <initializer_list>
+
 #include "../../include/ice3.h"
 #include "ice3_physics.hpp"
 
@@ -132,6 +134,22 @@ struct SedimArgs {
   const double *src_rh;  // hail (KRR=7): source in, source out, surface rate
   double *dst_rh, *inprh;
 };
+
+// Columns of a launch of k_sedim at most: it takes ten threads a column with hail, and a launch
+// fewer than 2^32 along an axis.
+constexpr int SEDIM_LAUNCH_COLS = 1 << 28;
+
+// At most n columns of a from column c on.
+inline SedimArgs sedim_columns(const SedimArgs &a, int c, int n) {
+  SedimArgs p = a;
+  p.ncol = a.ncol - c < n ? a.ncol - c : n;
+  for (const double **f : {&p.rhodref, &p.dzz, &p.src_rr, &p.src_ri, &p.src_rs, &p.src_rg, &p.src_rh})
+    if (*f) *f += c;
+  for (double **f : {&p.dst_rr, &p.dst_ri, &p.dst_rs, &p.dst_rg, &p.dst_rh, &p.inprc, &p.inprr, &p.inpri,
+                     &p.inprs, &p.inprg, &p.inprh, &p.zzz})
+    if (*f) *f += c;
+  return p;
+}
 
 // ICE4_SEDIMENTATION with CSEDIM='SPLI' (micro/mode_ice4_sedimentation.F90:196-219): the
 // split sedimentation of rain, pristine ice, snow, graupel (and hail) on the state at t, then

@@ -43,7 +43,8 @@ def columns_of(fields: dict, layout: str, *, device):
             t = torch.as_tensor(x, dtype=f64, device=device)
         if layout == "jax" and t.dim() >= 2 and t.is_contiguous() and t.device.type == "cuda":
             v = t.reshape(-1, t.shape[-1])
-            if not v.t().is_contiguous() and max(v.shape) < 2 ** 31:
+            # (below 2^28 either way ice3_transpose_fields' tiles, 32 by 128, fit its launch)
+            if not v.t().is_contiguous() and max(v.shape) < 2 ** 28:
                 batches.setdefault(tuple(v.shape), []).append((k, v))
                 out[k] = None  # keeps the order of the names
                 continue

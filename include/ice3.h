@@ -114,8 +114,9 @@ int ice3_count_nonfinite(int nfield, const double *const *fields, const int *row
 
 /* nfield (at most ICE3_MAX_CHECK_FIELDS) float64 device arrays (rows, cols), contiguous, written
  * transposed: dst[q][c*rows + r] = src[q][r*cols + c].  One launch; src and dst are host arrays
- * of device pointers, and no dst overlaps a src.  The Python drop-ins bring (..., nz) fields to
- * the (nlev, ncol) layout with it. */
+ * of device pointers, and no dst overlaps a src.  At most 2^24 - 1 tiles of 32 rows by 128 columns,
+ * else ICE3_EINVAL.  The Python drop-ins bring (..., nz) fields to the (nlev, ncol) layout with
+ * it. */
 int ice3_transpose_fields(int nfield, const double *const *src, double *const *dst, int rows,
                           int cols, void *stream);
 
