@@ -27,28 +27,38 @@ def as_columns(x, layout: str, *, device, name: str) -> torch.Tensor:
     return t.reshape(-1, t.shape[-1]).t().contiguous()
 
 
+def device_tensor(x, device) -> torch.Tensor:
+    """x as a float64 tensor on the device (a tensor that is one already passes a check only)."""
+    if type(x) is torch.Tensor and x.dtype is torch.float64 and x.device == device:
+        return x
+    return torch.as_tensor(x, dtype=torch.float64, device=device)
+
+
 def columns_of(fields: dict, layout: str, *, device):
     """as_columns of every field of a call, and the names of those that are fresh copies (the
     others share the caller's memory).  "jax" fields whose memory is (..., nz) in order are
     transposed together, one launch for each shape among them."""
     out, fresh, batches = {}, set(), {}
-    f64 = torch.float64
     for k, x in fields.items():
-        if type(x) is torch.Tensor and x.dtype is f64 and x.device == device:
-            t = x
-            if layout == "columns" and x.dim() == 2 and x.is_contiguous():
-                out[k] = x
+        t = device_tensor(x, device)
+        if layout == "columns":
+            if t is x and t.dim() == 2 and t.is_contiguous():
+                out[k] = t
                 continue
+            out[k] = as_columns(t, layout, device=device, name=k)
         else:
-            t = torch.as_tensor(x, dtype=f64, device=device)
-        if layout == "jax" and t.dim() >= 2 and t.is_contiguous() and t.device.type == "cuda":
+            if t.dim() < 2:
+                raise ValueError(f"{k}: expected a (..., nz) array, got {tuple(t.shape)}")
             v = t.reshape(-1, t.shape[-1])
-            # (below 2^28 either way ice3_transpose_fields' tiles, 32 by 128, fit its launch)
-            if not v.t().is_contiguous() and max(v.shape) < 2 ** 28:
-                batches.setdefault(tuple(v.shape), []).append((k, v))
-                out[k] = None  # keeps the order of the names
-                continue
-        out[k] = as_columns(t, layout, device=device, name=k)
+            c = v.t()
+            if not c.is_contiguous():
+                # (below 2^28 either way ice3_transpose_fields' tiles, 32 by 128, fit its launch)
+                if t.is_contiguous() and t.is_cuda and max(v.shape) < 2 ** 28:
+                    batches.setdefault(tuple(v.shape), []).append((k, v))
+                    out[k] = None  # keeps the order of the names
+                    continue
+                c = c.contiguous()
+            out[k] = c
         if out[k].data_ptr() != t.data_ptr():
             fresh.add(k)
     for (rows, cols), items in batches.items():
@@ -91,14 +101,19 @@ def column_shape(x, layout: str, name: str, *, device) -> tuple:
 def in_rows(fields: dict) -> bool:
     """Whether "jax" layout fields (device float64 tensors) are better taken as (ncol, nlev) rows,
     the vertical contiguous, than as (nlev, ncol) columns: True unless more of them already have
-    the columns' memory order (results of a columns call are such views)."""
-    score = 0
-    for t in fields.values():
-        if t.is_contiguous():
-            score += 1
-        elif t.dim() >= 2 and t.movedim(-1, 0).is_contiguous():
+    the columns' memory order (results of a columns call are such views) than the rows'.  Looks at
+    no more of them than decides it."""
+    others = [t for t in fields.values() if not t.is_contiguous()]
+    lead = len(fields) - 2 * len(others)  # of the rows, if all the others are in the columns' order
+    if lead >= 0:
+        return True
+    score = len(fields) - len(others)
+    for t in others:
+        if t.dim() >= 2 and t.movedim(-1, 0).is_contiguous():
             score -= 1
-    return score >= 0
+            if score < 0:
+                return False
+    return True
 
 
 def as_rows(t: torch.Tensor, name: str) -> torch.Tensor:

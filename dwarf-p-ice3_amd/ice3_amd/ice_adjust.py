@@ -20,7 +20,7 @@ import ctypes
 import torch
 
 from . import _lib
-from ._fields import (addresses, as_columns, as_rows, check_layout, columns_of, from_columns, in_rows,
+from ._fields import (addresses, as_columns, as_rows, check_layout, columns_of, device_tensor, from_columns, in_rows,
                       new_fields, ptr, resolve_layout, stream_ptr)
 
 _PREC = {"fp64": _lib.PREC_FP64, "mixed": _lib.PREC_MIXED}
@@ -115,7 +115,7 @@ class IceAdjust:
         are (ncol, nlev) rows ("jax" arrays as they are) instead of (nlev, ncol) columns."""
         rows = False
         if layout == "jax":
-            args = {k: torch.as_tensor(v, dtype=torch.float64, device=self.device) for k, v in args.items()}
+            args = {k: device_tensor(v, self.device) for k, v in args.items()}
             rows = in_rows(args)
         if rows:
             f = {k: as_rows(v, k) for k, v in args.items()}
