@@ -1268,14 +1268,14 @@ extern "C" int ice3_ice_adjust_ocnd2(ice3_ctx *ctx, int ncol, int nlev, int ld, 
 // ICE_ADJUST and the statistical sedimentation of the FP64 fused step; aa.rh (with sa.src_rh)
 // selects hail.  One column walk when there are enough columns to hide its latency: a lone
 // wavefront takes 6 us a level, so that 1,024 to 65,536 columns of 90 levels all take 0.53 to
-// 0.60 ms, against 0.08 to 0.44 ms for ICE_ADJUST point by point followed by k_sedim.  From
-// SEDIM_WALK_COLS (1.7 wavefronts per SIMD) on the walk saves more traffic than it waits: at
-// 98,304 columns 0.69 against 0.63 ms, at 106,496 0.71 against 0.69, at 114,688 0.715 against 0.737
+// 0.60 ms, against 0.08 to 0.44 ms for ICE_ADJUST point by point followed by k_sedim; or levels
+// so few that there is little to wait for (sedim_walk_cols).  From 432 columns a compute unit (1.7
+// wavefronts per SIMD) on the walk saves more traffic than it waits: at 98,304 columns 0.69 against 0.63 ms, at 106,496 0.71 against 0.69, at 114,688 0.715 against 0.737
 // (hail: 0.79 against 0.91), at 131,072 0.75 against 0.82, at 262,144 1.40 against 1.63.
 static hipError_t launch_adjust_sedim(const ice3_ctx *ctx, const AdjustArgs &aa, const SedimArgs &sa,
                                       hipStream_t s) {
   const dim3 gw((aa.ncol + 63) / 64), gp((aa.ncol + 255) / 256, aa.nlev);
-  if (aa.ncol >= SEDIM_WALK_COLS * ctx->ncu) {
+  if (aa.ncol >= (long long)sedim_walk_cols(SEDIM_FUSED, aa.nlev) * ctx->ncu) {
     if (aa.rh) hipLaunchKernelGGL(k_adjust_sedim_hail, gw, dim3(64), 0, s, aa, sa);
     else hipLaunchKernelGGL(k_adjust_sedim, gw, dim3(64), 0, s, aa, sa);
     return hipGetLastError();

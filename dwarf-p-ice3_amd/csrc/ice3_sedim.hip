@@ -24,9 +24,9 @@ namespace ice3 {
 //
 // Few columns: bound by the recurrence (pristine ice's two logarithms and exponential, about
 // 0.7 us a level).  1,024 columns of 90 levels take 59 us (one thread per column, four species
-// after one another: 292 us; four wavefronts without the own-content half split off: 104 us).
-// Many columns: bound by the VALU (76 % busy).  65,536 columns: 183 us (339), 262,144: 683 us
-// (705).  Groups of three levels keep four workgroups' LDS on a compute unit; four levels took
+// after one another: 186 us; four wavefronts without the own-content half split off: 104 us).
+// More columns: bound by the VALU (76 % busy).  65,536 columns: 179 us (223); from the counts of
+// sedim_walk_cols on one thread per column is the better form.  Groups of three levels keep four workgroups' LDS on a compute unit; four levels took
 // 206 us at 65,536 columns.  The Horner coefficients as scalars, hoisted out of the loop by
 // machine LICM, are worth 9 us at 1,024 columns and 20 us at 65,536 against vector ones.
 constexpr int SG = 3;  // levels of a group
@@ -158,38 +158,34 @@ __global__ void __launch_bounds__(128 * (HAIL ? 5 : 4)) k_sedim(SedimArgs a) {
   }
 }
 
-// One thread per column, walking it (the mixed path over many columns: float rates leave it
-// bound by HBM, 262,144 columns of 90 levels 0.39 ms against 0.44 ms in k_sedim<float>; at
-// 65,536 columns 0.165 against 0.104).
-template <class R> __global__ void __launch_bounds__(256) k_sedim_walk(SedimArgs a) {
+// One thread per column, walking it: few levels, which leave k_sedim's pipeline unfilled, and many
+// columns, which hide a column's latency without k_sedim's own-content wavefronts, LDS and barriers.
+// 262,144 columns of 90 levels: 559 us, k_sedim 640 (hail 694 and 1019, OCND2 587 and 698); 4 million
+// columns of one level: 0.10 ms and 0.60.  The scalar coefficients are worth 10 % here too (616 us without).
+template <class R, bool ZZZ = false, bool HAIL = false>
+__global__ void __launch_bounds__(256) k_sedim_walk(SedimArgs a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.ncol) return;
-  sedim_column<R>(a, i);
+  sedim_column<R, ZZZ, HAIL>(a, i);
 }
 
-template <class R> hipError_t sedim_launch(const SedimArgs &sa, int ncu, hipStream_t s) {
-  if constexpr (sizeof(R) == sizeof(float)) {
-    if (sa.ncol >= SEDIM_WALK_COLS * ncu) {
-      hipLaunchKernelGGL(k_sedim_walk<R>, dim3((sa.ncol + 255) / 256), dim3(256), 0, s, sa);
-      return hipGetLastError();
-    }
-  }
-  for (int c = 0;;) {
-    const SedimArgs part = sedim_columns(sa, c, SEDIM_LAUNCH_COLS);
-    const dim3 g((part.ncol + 63) / 64);
-    if (sizeof(R) == sizeof(double) && part.src_rh)
-      hipLaunchKernelGGL((k_sedim<double, false, true>), g, dim3(640), 0, s, part);
-    else if (sizeof(R) == sizeof(double) && part.zzz)
-      hipLaunchKernelGGL((k_sedim<double, true>), g, dim3(512), 0, s, part);
-    else
-      hipLaunchKernelGGL(k_sedim<R>, g, dim3(512), 0, s, part);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || part.ncol == sa.ncol - c) return e;
-    c += part.ncol;
-  }
+template <class R, bool ZZZ, bool HAIL>
+static hipError_t sedim_launch_as(const SedimArgs &sa, SedimForm form, int ncu, hipStream_t s) {
+  if (sa.ncol >= (long long)sedim_walk_cols(form, sa.nlev) * ncu)
+    hipLaunchKernelGGL((k_sedim_walk<R, ZZZ, HAIL>), dim3((sa.ncol - 1) / 256 + 1), dim3(256), 0, s, sa);
+  else
+    hipLaunchKernelGGL((k_sedim<R, ZZZ, HAIL>), dim3((sa.ncol - 1) / 64 + 1), dim3(HAIL ? 640 : 512), 0, s, sa);
+  return hipGetLastError();
 }
 
-template hipError_t sedim_launch<double>(const SedimArgs &, int, hipStream_t);
-template hipError_t sedim_launch<float>(const SedimArgs &, int, hipStream_t);
+template <> hipError_t sedim_launch<double>(const SedimArgs &sa, int ncu, hipStream_t s) {
+  if (sa.src_rh) return sedim_launch_as<double, false, true>(sa, SEDIM_HAIL, ncu, s);
+  if (sa.zzz) return sedim_launch_as<double, true, false>(sa, SEDIM_FP64, ncu, s);
+  return sedim_launch_as<double, false, false>(sa, SEDIM_FP64, ncu, s);
+}
+
+template <> hipError_t sedim_launch<float>(const SedimArgs &sa, int ncu, hipStream_t s) {
+  return sedim_launch_as<float, false, false>(sa, SEDIM_MIXED, ncu, s);
+}
 
 }  // namespace ice3

@@ -12,8 +12,6 @@
 // these functions.  Everything here is force-inlined and every array index is a
 // compile-time constant after unrolling, so the state lives in registers.
 #pragma once
-#include <initializer_list>
-
 #include "../../include/ice3.h"
 #include "ice3_physics.hpp"
 
@@ -135,20 +133,35 @@ struct SedimArgs {
   double *dst_rh, *inprh;
 };
 
-// Columns of a launch of k_sedim at most: it takes ten threads a column with hail, and a launch
-// fewer than 2^32 along an axis.
-constexpr int SEDIM_LAUNCH_COLS = 1 << 28;
-
-// At most n columns of a from column c on.
-inline SedimArgs sedim_columns(const SedimArgs &a, int c, int n) {
-  SedimArgs p = a;
-  p.ncol = a.ncol - c < n ? a.ncol - c : n;
-  for (const double **f : {&p.rhodref, &p.dzz, &p.src_rr, &p.src_ri, &p.src_rs, &p.src_rg, &p.src_rh})
-    if (*f) *f += c;
-  for (double **f : {&p.dst_rr, &p.dst_ri, &p.dst_rs, &p.dst_rg, &p.dst_rh, &p.inprc, &p.inprr, &p.inpri,
-                     &p.inprs, &p.inprg, &p.inprh, &p.zzz})
-    if (*f) *f += c;
-  return p;
+// Columns per compute unit from which the statistical sedimentation walks a column with one thread
+// (k_sedim_walk, or k_adjust_sedim with ICE_ADJUST), below which k_sedim takes 64 columns with a
+// wavefront per species and half.  Few levels leave k_sedim's pipeline of three levels a step
+// unfilled and its prologue unpaid; few columns leave the walk's chain of levels, 2 us each, uncovered.
+// The walk steps up whenever another wavefront a SIMD is needed (every 256 columns a compute unit).
+// 256 compute units, us of the walk / k_sedim; the form taken changes at each line's middle pair:
+//   FP64   2 levels:   8,192 columns 6/7,     16,384 6/7,      65,536 8/15
+//          5 levels:  32,768 15/13,           49,152 15/17,    65,536 15/23
+//         12 levels:  49,152 31/27,           65,536 32/35,    98,304 46/48
+//         20 levels:  65,536 54/52, 98,304 74/72,  110,000 76/82, 262,144 135/175
+//         90 levels:  98,304 308/252, 110,000 309/290, 131,072 319/320, 262,144 559/640
+//   hail   5 levels:  32,768 19/15,           49,152 19/21,    65,536 19/32
+//         20 levels:  49,152 65/50,           65,536 72/79,    98,304 93/112
+//         90 levels:  81,920 395/360,         98,304 398/411, 262,144 694/1019
+//   mixed  5 levels:  32,768 10/8,            49,152 10/10,    65,536 10/13
+//         90 levels:  65,536 140/97,         110,000 167/160
+//   fused, k_adjust_sedim / ICE_ADJUST and k_sedim: 2 levels 64 columns 11/14, 16,384 12/14;
+//          4 levels:  32,768 26/20,           49,152 27/24,    65,536 28/31;
+//          5 levels and more: from 432 columns a compute unit on (launch_adjust_sedim)
+// k_sedim never has 2^28 columns, at ten threads a column, in one launch: they are walked.
+enum SedimForm { SEDIM_FP64, SEDIM_HAIL, SEDIM_MIXED, SEDIM_FUSED };
+inline int sedim_walk_cols(SedimForm form, int nlev) {
+  if (form == SEDIM_FUSED) return nlev <= 2 ? 0 : nlev <= 4 ? 72 * (nlev - 1) : 432;
+  const int few = 48 * (nlev - 1);
+  const int many = form == SEDIM_MIXED  ? 432
+                   : form == SEDIM_HAIL ? (nlev < 51 ? 180 + 4 * nlev : 384)
+                   : nlev <= 12         ? 216
+                                        : (nlev < 76 ? 360 + 2 * nlev : 512);
+  return few < many ? few : many;
 }
 
 // ICE4_SEDIMENTATION with CSEDIM='SPLI' (micro/mode_ice4_sedimentation.F90:196-219): the

@@ -285,19 +285,5 @@ extern "C" void hst_log_f64(const double *x, double *y, long n) {
   for (long q = 0; q < n; ++q) y[q] = log_f64(x[q]);
 }
 
-// n columns of a sedimentation over ncol, from column c on (ice3_stages.hpp: sedim_columns), and the
-// most of a launch: pointers are byte offsets, 0 for an array that is not there.
-extern "C" int hst_sedim_columns(int ncol, int c, int n, const size_t *in, size_t *out) {
-  SedimArgs a = SedimArgs{};
-  a.ncol = ncol; a.nlev = 3; a.ld = ncol; a.dt = 50.;
-  const double **const from[] = {&a.rhodref, &a.dzz, &a.src_rr, &a.src_ri, &a.src_rs, &a.src_rg, &a.src_rh};
-  double **const to[] = {&a.dst_rr, &a.dst_ri, &a.dst_rs, &a.dst_rg, &a.dst_rh, &a.inprc, &a.inprr,
-                         &a.inpri, &a.inprs, &a.inprg, &a.inprh, &a.zzz};
-  for (int q = 0; q < 7; ++q) *from[q] = (const double *)in[q];
-  for (int q = 0; q < 12; ++q) *to[q] = (double *)in[7 + q];
-  a = sedim_columns(a, c, n);
-  for (int q = 0; q < 7; ++q) out[q] = (size_t)*from[q];
-  for (int q = 0; q < 12; ++q) out[7 + q] = (size_t)*to[q];
-  return a.nlev == 3 && a.ld == ncol && a.dt == 50. ? a.ncol : -1;
-}
-extern "C" int hst_sedim_launch_cols(void) { return SEDIM_LAUNCH_COLS; }
+// From how many columns a compute unit the sedimentation walks (ice3_stages.hpp: sedim_walk_cols).
+extern "C" int hst_sedim_walk_cols(int form, int nlev) { return sedim_walk_cols((SedimForm)form, nlev); }

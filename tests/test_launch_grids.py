@@ -1,31 +1,35 @@
-"""Launches of several threads a column: a launch takes fewer than 2^32 threads along an axis, so that
-many columns go in parts."""
+"""Which form the statistical sedimentation takes: one thread a column or several wavefronts for 64 of
+them, and that no launch has 2^32 threads along an axis."""
 import ctypes
 import os
 import sys
 
+import numpy as np
 import pytest
 
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "host_stages"))
 import host_lib  # noqa: E402
 
+FORMS = {"fp64": 0, "hail": 1, "mixed": 2, "fused": 3}
+DT = 50.0
 
-@pytest.mark.parametrize("ncol", [1, 2 ** 28 - 1, 2 ** 28, 2 ** 28 + 1, 2 ** 29 + 65, 2 ** 31 - 1])
-@pytest.mark.parametrize("hail", [False, True])
-def test_sedimentation_in_parts_covers_every_column(ncol, hail):
-    """Parts of whole workgroups' columns, each within a launch, one after the other, and every array
-    of a part from its first column on (hail's seven arrays apart from the others')."""
-    lib = host_lib.load()
-    most = lib.hst_sedim_launch_cols()
-    assert most % 64 == 0 and most // 64 * 640 < 2 ** 32
-    arrays = [0 if q in (6, 11, 17) and not hail else (q + 1) << 40 for q in range(19)]
-    given, part, c = (ctypes.c_size_t * 19)(*arrays), (ctypes.c_size_t * 19)(), 0
-    while c < ncol:
-        n = lib.hst_sedim_columns(ncol, c, most, given, part)
-        assert 0 < n == min(most, ncol - c)
-        assert list(part) == [a and a + 8 * c for a in arrays]
-        c += n
-    assert c == ncol
+
+@pytest.mark.parametrize("form", FORMS)
+def test_several_threads_a_column_fit_a_launch(form):
+    """A domain has at most 2^32 points (and a device far fewer than 4,096 compute units): the columns
+    below the walk's count, at ten threads each, stay within a launch at every number of levels."""
+    cols = host_lib.load().hst_sedim_walk_cols
+    for nlev in [*range(1, 300), 1000, 65535]:
+        most = min(cols(FORMS[form], nlev) * 4096, 2 ** 32 // nlev)
+        assert 0 <= most and -(-most // 64) * 640 < 2 ** 32, nlev
+
+
+def test_few_levels_walk_from_fewer_columns():
+    cols = host_lib.load().hst_sedim_walk_cols
+    for form in FORMS.values():
+        counts = [cols(form, n) for n in range(1, 300)]
+        assert counts[0] == 0                    # one level has nothing to wait for
+        assert counts == sorted(counts) and counts[-1] <= 512
 
 
 @pytest.mark.parametrize("rows,cols", [(2 ** 29, 2), (2 ** 31 - 1, 2), (2, 2 ** 31 - 1), (2 ** 24, 4096)])
@@ -64,3 +68,44 @@ def test_rain_ice_over_more_columns_than_one_axis_takes(ncol):
                 g, w = got[k].reshape(-1), want[k].reshape(-1)
                 assert bool((g[:ncol // n * n].view(-1, n) == w).all()) and torch.equal(g[ncol // n * n:], w[:ncol % n]), k
     assert float(diags["inprr"].max()) > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["plain", "hail", "ocnd2", "mixed"])
+@pytest.mark.parametrize("nlev", [1, 2, 3, 4, 7, 12, 40])
+def test_rain_ice_on_both_sides_of_the_walk(kind, nlev):
+    """RAIN_ICE over more columns than every form's walk begins at, against the same columns in calls of
+    fewer than any walk of two levels or more: every output bit for bit (OCND2's model level height,
+    the walk's and k_sedim's, through the microphysics that reads it)."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ice3_amd import RainIce, RainIceHail, RainIceOCND2, synthetic
+    ncu = torch.cuda.get_device_properties(0).multi_processor_count
+    ncol, part = 512 * ncu + 1, 47 * ncu - 1
+    f = synthetic.generate(2048, 90, seed=20260402, variant="pipeline")
+    f = {k: np.ascontiguousarray(v[:3 * nlev:3] if nlev <= 30 else v[:nlev]) for k, v in f.items() if v.ndim == 2}
+    rng = np.random.Generator(np.random.Philox(nlev))
+    names = dict(exn="exn", rhodref="rho_dry_ref", pres="pabs", dzz="dzz", th_t="th", rv_t="rv", rc_t="rc", rr_t="rr",
+                 ri_t="ri", rs_t="rs", rg_t="rg", ci_t="ci", sigs="sigs")
+    names.update({k: k for k in ("ths", "rvs", "rcs", "rrs", "ris", "rss", "rgs")})
+    s = {k: f[v] for k, v in names.items()}
+    if kind == "hail":
+        s["rh_t"], s["rhs"] = f["rg"] * 0.7, f["rg"] * 0.7 / DT
+    if kind == "ocnd2":
+        s.update(icldfr=rng.uniform(0, 1, f["th"].shape), ssio=rng.uniform(0, 0.2, f["th"].shape),
+                 ssiu=rng.uniform(-0.2, 0, f["th"].shape), ifr=np.full(f["th"].shape, 10.0))
+    # the columns over and over, thinned by as much as a column's own number says: none alike
+    thin = torch.linspace(0.5, 1.5, ncol, dtype=torch.float64, device="cuda")
+    s = {k: torch.from_numpy(v).cuda().repeat(1, -(-ncol // 2048))[:, :ncol].contiguous() for k, v in s.items()}
+    for k in ("rrs", "ris", "rss", "rgs", "dzz") + (("rhs",) if kind == "hail" else ()):
+        s[k] = s[k] * thin
+    call = {"plain": RainIce, "hail": RainIceHail, "ocnd2": RainIceOCND2, "mixed": RainIce}[kind]()
+    kw = {"precision": "mixed"} if kind == "mixed" else {}
+    whole, whole_d = call(s, DT, **kw)
+    for c in range(0, ncol, part):
+        new, diags = call({k: v[:, c:c + part].contiguous() for k, v in s.items()}, DT, **kw)
+        for k in ("ths", "rvs", "rcs", "rrs", "ris", "rss", "rgs", "ci_t", "evap3d") + (("rhs",) if kind == "hail" else ()):
+            assert torch.equal(new[k], whole[k][:, c:c + part]), (k, c)
+        for k in diags:
+            assert torch.equal(diags[k], whole_d[k][c:c + part]), (k, c)
