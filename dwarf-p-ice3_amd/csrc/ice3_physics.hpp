@@ -187,7 +187,9 @@ __device__ constexpr double ZSRC_1D[34] = {
 // table are clamped (the reference reads out of bounds there).
 __host__ __device__ __forceinline__ int tiwmx_index(double t) {
   const double jk = round(100. * t);  // NINT: half away from zero
-  return (int)(jk < ICE3_TIWMX_START ? ICE3_TIWMX_START : (jk > ICE3_TIWMX_STOP ? ICE3_TIWMX_STOP : jk)) -
+  return (int)(!(jk >= ICE3_TIWMX_START) ? ICE3_TIWMX_START  // a NaN too: the index stays in the table
+               : jk > ICE3_TIWMX_STOP    ? ICE3_TIWMX_STOP
+                                         : jk) -
          ICE3_TIWMX_START;
 }
 

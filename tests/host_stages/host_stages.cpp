@@ -287,3 +287,7 @@ extern "C" void hst_log_f64(const double *x, double *y, long n) {
 
 // From how many columns a compute unit the sedimentation walks (ice3_stages.hpp: sedim_walk_cols).
 extern "C" int hst_sedim_walk_cols(int form, int nlev) { return sedim_walk_cols((SedimForm)form, nlev); }
+
+// The OCND2 tables' index of a temperature, and their length (ice3_physics.hpp: tiwmx_index).
+extern "C" int hst_tiwmx_index(double t) { return tiwmx_index(t); }
+extern "C" int hst_tiwmx_n(void) { return ICE3_TIWMX_N; }
