@@ -128,6 +128,12 @@ __global__ void __launch_bounds__(256) k_count_nonfinite(CountArgs a) {
   if ((threadIdx.x & 63) == 0) atomicAdd(&a.counts[q], n);
 }
 
+// The kernels' division, value by value (ice3_divide, a test hook).
+__global__ void __launch_bounds__(256) k_divide(int n, const double *a, const double *b, double *q) {
+  const unsigned e = blockIdx.x * 256 + threadIdx.x;
+  if (e < (unsigned)n) q[e] = a[e] / by(b[e]);
+}
+
 // ---- k_transpose: fields (rows, cols) -> (cols, rows), all the fields of a call in one launch.
 // A workgroup takes TR_ROWS rows (model columns) and up to TR_COLS of their values (levels): a
 // run of memory that it reads in order, and writes through LDS in rows of TR_ROWS doubles (two
@@ -1189,6 +1195,14 @@ extern "C" int ice3_count_nonfinite(int nfield, const double *const *fields, con
   const int blocks = (ncol + 255) / 256;
   dim3 grid(blocks < 1024 ? blocks : 1024, nfield);
   hipLaunchKernelGGL(k_count_nonfinite, grid, dim3(256), 0, (hipStream_t)stream, a);
+  HIPCHK(hipGetLastError());
+  return ICE3_OK;
+}
+
+extern "C" int ice3_divide(int n, const double *a, const double *b, double *q, void *stream) {
+  if (n < 0 || (n > 0 && (!a || !b || !q))) return ICE3_EINVAL;
+  if (n == 0) return ICE3_OK;
+  hipLaunchKernelGGL(k_divide, dim3((n - 1) / 256 + 1), dim3(256), 0, (hipStream_t)stream, n, a, b, q);
   HIPCHK(hipGetLastError());
   return ICE3_OK;
 }

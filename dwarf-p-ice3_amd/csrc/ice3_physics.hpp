@@ -29,27 +29,34 @@ enum { ITH = 0, IRV = 1, IRC = 2, IRR = 3, IRI = 4, IRS = 5, IRG = 6, IRH = 7 };
 // ---------------------------------------------------------------- FP64 division
 // a / by(b).  On the device: the hardware reciprocal (relative error under 4.7e-8), one Newton
 // step, and the residual correction of the quotient, which squares the reciprocal's remaining
-// error (2e-15): the IEEE quotient but for operands within 1e-29 of a rounding boundary (equal to
-// it on 6.3e9 random pairs over 2^+-300).  Two fused operations fewer than the compiler's own
-// -fapprox-func sequence, which takes a second Newton step; and a divisor shared by several
-// quotients is one reciprocal wherever they stand.  A zero, infinite or NaN divisor gives NaN, as
-// the compiler's sequence does.  Divisions are a quarter of k_micro's VALU time: with this form
-// k_micro takes 2.85 ms at 512x512x90 instead of 2.95, results bit for bit the same.
+// error (2.4e-15): the IEEE quotient but for operands whose quotient is within 1e-29 of a rounding
+// boundary, and there one of the two neighbours.  Two fused operations fewer than the compiler's
+// own -fapprox-func sequence, which takes a second Newton step; and a divisor shared by several
+// quotients is one reciprocal wherever they stand.  A zero, infinite or NaN divisor gives NaN, and
+// so does an infinite dividend, as with the compiler's sequence.  Divisions are a quarter of
+// k_micro's VALU time: with this form k_micro takes 2.85 ms at 512x512x90 instead of 2.95, results
+// bit for bit the same.
 template <class T> struct By {
   T b, r;
 };
+// The divisor b with its reciprocal refined from an approximate one, and a quotient by it.
+__host__ __device__ __forceinline__ By<double> by_from(double b, double r0) {
+  return {b, fma(fma(-b, r0, 1.0), r0, r0)};
+}
+__host__ __device__ __forceinline__ double corrected_quotient(double a, const By<double> &d) {
+  const double q = a * d.r;
+  return fma(fma(-d.b, q, a), d.r, q);
+}
 __host__ __device__ __forceinline__ By<double> by(double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  const double r = __builtin_amdgcn_rcp(b);
-  return {b, fma(fma(-b, r, 1.0), r, r)};
+  return by_from(b, __builtin_amdgcn_rcp(b));
 #else
   return {b, 0.};
 #endif
 }
 __host__ __device__ __forceinline__ double operator/(double a, const By<double> &d) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  const double q = a * d.r;
-  return fma(fma(-d.b, q, a), d.r, q);
+  return corrected_quotient(a, d);
 #else
   return a / d.b;
 #endif

@@ -297,6 +297,12 @@ int ice3_ice_adjust_branches(ice3_ctx *ctx, int ncol, int nlev, int ld, double d
                              const ice3_ice_adjust_in *in, const double *rh,
                              const ice3_ice_adjust_out *out, unsigned *branches, void *stream);
 
+/* The kernels' FP64 division (no counterpart in the reference: a test hook): q[e] = a[e] / b[e] for
+ * n device values, the IEEE quotient for finite dividends and normal divisors whose quotient is
+ * normal and no closer than 1e-29 to a rounding boundary, one of its neighbours there; NaN for a
+ * zero, infinite or NaN divisor. */
+int ice3_divide(int n, const double *a, const double *b, double *q, void *stream);
+
 /* ---- fused ice_adjust + rain_ice (the "adjust then microphysics" time step) ----
  * ice_adjust runs on the state at t; its updated sources, times dt, are the
  * t-state of rain_ice (the synthetic and AROME-like inputs carry the state at t

@@ -291,3 +291,9 @@ extern "C" int hst_sedim_walk_cols(int form, int nlev) { return sedim_walk_cols(
 // The OCND2 tables' index of a temperature, and their length (ice3_physics.hpp: tiwmx_index).
 extern "C" int hst_tiwmx_index(double t) { return tiwmx_index(t); }
 extern "C" int hst_tiwmx_n(void) { return ICE3_TIWMX_N; }
+
+// The kernels' FP64 quotients a / b from given approximate reciprocals r0 (ice3_physics.hpp: by_from,
+// corrected_quotient); fma is the C library's.
+extern "C" void hst_quotients(const double *a, const double *b, const double *r0, double *q, long n) {
+  for (long e = 0; e < n; ++e) q[e] = corrected_quotient(a[e], by_from(b[e], r0[e]));
+}
