@@ -39,27 +39,32 @@ def columns_of(fields: dict, layout: str, *, device):
     others share the caller's memory).  "jax" fields whose memory is (..., nz) in order are
     transposed together, one launch for each shape among them."""
     out, fresh, batches = {}, set(), {}
+    if layout == "columns":
+        f64, tensor = torch.float64, torch.Tensor
+        for k, x in fields.items():
+            if type(x) is tensor and x.dtype is f64 and x.device == device and x.dim() == 2 and x.is_contiguous():
+                out[k] = x
+                continue
+            t = device_tensor(x, device)
+            out[k] = as_columns(t, layout, device=device, name=k)
+            if out[k].data_ptr() != t.data_ptr():
+                fresh.add(k)
+        return out, fresh
     for k, x in fields.items():
         t = device_tensor(x, device)
-        if layout == "columns":
-            if t is x and t.dim() == 2 and t.is_contiguous():
-                out[k] = t
+        if t.dim() < 2:
+            raise ValueError(f"{k}: expected a (..., nz) array, got {tuple(t.shape)}")
+        v = t.reshape(-1, t.shape[-1])
+        c = v.t()
+        if not c.is_contiguous():
+            # (below 2^28 either way ice3_transpose_fields' tiles, 32 by 128, fit its launch)
+            if t.is_contiguous() and t.is_cuda and max(v.shape) < 2 ** 28:
+                batches.setdefault(tuple(v.shape), []).append((k, v))
+                out[k] = None  # keeps the order of the names
                 continue
-            out[k] = as_columns(t, layout, device=device, name=k)
-        else:
-            if t.dim() < 2:
-                raise ValueError(f"{k}: expected a (..., nz) array, got {tuple(t.shape)}")
-            v = t.reshape(-1, t.shape[-1])
-            c = v.t()
-            if not c.is_contiguous():
-                # (below 2^28 either way ice3_transpose_fields' tiles, 32 by 128, fit its launch)
-                if t.is_contiguous() and t.is_cuda and max(v.shape) < 2 ** 28:
-                    batches.setdefault(tuple(v.shape), []).append((k, v))
-                    out[k] = None  # keeps the order of the names
-                    continue
-                c = c.contiguous()
-            out[k] = c
-        if out[k].data_ptr() != t.data_ptr():
+            c = c.contiguous()
+        out[k] = c
+        if c.data_ptr() != t.data_ptr():
             fresh.add(k)
     for (rows, cols), items in batches.items():
         for i in range(0, len(items), _lib.ICE3_MAX_CHECK_FIELDS):
@@ -80,11 +85,10 @@ def column_shape(x, layout: str, name: str, *, device) -> tuple:
     """The (nlev, ncol) shape as_columns(x) would have, without making it, of a field that no kernel
     reads.  What as_columns refuses (a type, a dtype, strides or a device that it cannot convert) is
     refused here too: an array is converted as far as the host goes, anything else altogether."""
-    if isinstance(x, np.ndarray):
+    if type(x) is not torch.Tensor or x.layout is not torch.strided or x.is_quantized or not (x.is_cuda or x.is_cpu):
+        if not isinstance(x, np.ndarray):
+            return tuple(as_columns(x, layout, device=device, name=name).shape)
         x = torch.as_tensor(x, dtype=torch.float64)
-    elif type(x) is not torch.Tensor or x.layout is not torch.strided or x.is_quantized or \
-            x.device.type not in ("cuda", "cpu"):
-        return tuple(as_columns(x, layout, device=device, name=name).shape)
     shape = tuple(x.shape)
     if layout == "columns":
         if len(shape) != 2:
