@@ -411,7 +411,7 @@ def ocnd2_step(lib, ctx, dev, g, cin, sp, stream, args, outputs, budget_err, sta
     return {"columns_per_s": ncol / (ms * 1e-3), "ms_per_step": ms, "speedup_vs_stat_krr6": ms_stat / ms,
             "stages_ms": stage_times_of(fn, args.steps, False),
             "water_budget_max_rel_err": budget_err(out),
-            "note": "fused step with PARAMI%LOCND2: k_ice_adjust_ocnd2, k_sedim<double> (which also "
+            "note": "fused step with PARAMI%LOCND2: k_ice_adjust_ocnd2, k_sedim_walk<double> (which also "
                     "writes the model level height), k_micro<double, OCND2> (persistent)"}
 
 

@@ -10,7 +10,8 @@
 //   k_adjust_sedim one thread per column: ICE_ADJUST and the sedimentation in one
 //                  top-down walk (the FP64 fused step over many columns);
 //   k_sedim<R>     (ice3_sedim.hip) the statistical sedimentation and the surface
-//                  precipitation, a wavefront per 64 columns and species;
+//                  precipitation, a wavefront per 64 columns, species and half, or
+//   k_sedim_walk<R>  one thread per column (few levels, many columns);
 //   k_micro<R>     persistent, one workgroup per compute unit, lookup tables in LDS:
 //                  the ICE4 time-split microphysics, total tendencies and negativity
 //                  correction per point, with the points of long time splittings

@@ -261,9 +261,10 @@ constexpr size_t MLP_BWD_LDS = (size_t)4 * BW_TILE * 2;
 // dW = H^T dZ the points are the contraction, so H and dZ of a layer go through LDS transposed;
 // dH = W dZ takes dZ from registers.  The backward tiles lie where the forward weights were, the
 // weights of a layer one layer ahead of their use.
-// 32,768 points (a tile for each compute unit), with the reduction: 51 us, against 208 us of
-// k_mlp_forward (34, with 100 MB of pre-activations and activations saved), k_mlp_backward (112)
-// and a serial sum of the partials (62).  Bound by the latency of its ten phases between
+// 32,768 points (a tile for each compute unit): 43 us a call among calls, 37 and, of the reduction, 10
+// as a profiler times the kernels one by one; 208 us of k_mlp_forward (34, with 100 MB of
+// pre-activations and activations saved), k_mlp_backward (112) and a serial sum of the partials
+// (62).  Bound by the latency of its ten phases between
 // barriers at two wavefronts a SIMD, and the 59 MB of partials written and read.
 struct MlpGradArgs {
   int npts;

@@ -284,7 +284,7 @@ struct MicroArgs {
   int max_calls;                 // sub-step cap per point
   unsigned long long *capped;    // context counter of capped points (always counted)
   // OCND2 branch only: ICE_ADJUST's OCND2 outputs, the TIWMX tables, and the model level
-  // height ZZZZ, which the sedimentation's column walk writes into rainfr before the
+  // height ZZZZ, which the sedimentation writes into rainfr before the
   // microphysics reads it and writes the rain fraction over it
   const double *icldfr, *ssio, *ssiu, *ifr, *tiwmx;
   unsigned *branches;  // test hook only (ice3_rain_ice_branches): per point, ICE3_BR_* bits

@@ -6,8 +6,9 @@ their updated values, ``evap3d``/``rainfr`` are added, and the diagnostics hold 
 surface precipitation ``inprc, inprr, inpri, inprs, inprg``.  Arithmetic is PHYEX
 RAIN_ICE (micro/rain_ice.F90) with the sedimentation before the microphysics, the
 per-point ICE4 time splitting, the total tendencies and the negativity correction,
-evaluated by the HIP kernels ``k_sedim`` (the statistical sedimentation, one column per
-thread) or ``k_sedim_split`` (``sedimentation="SPLI"``: the split scheme, one column per
+evaluated by the HIP kernels ``k_sedim`` (the statistical sedimentation, a wavefront per 64
+columns, species and half of the flux computation; ``k_sedim_walk``, one column per thread,
+over few levels or many columns) or ``k_sedim_split`` (``sedimentation="SPLI"``: the split scheme, one column per
 wavefront) and ``k_micro`` (the persistent per-point microphysics).
 
 State keys read (RainIceJAX names): exn, rhodref, pres, dzz, th_t, rv_t, rc_t, rr_t, ri_t,

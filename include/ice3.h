@@ -388,7 +388,9 @@ typedef struct {
 } ice3_surrogate;
 
 /* Fused step with the surrogate microphysics.  work: device scratch of
- * ice3_surrogate_work_bytes(ncol, nlev) bytes, 256-byte aligned (the fallback queue).  sg_counters (device, 5 entries, accumulated):
+ * ice3_surrogate_work_bytes(ncol, nlev) bytes, 256-byte aligned (101 bytes a point and 2 MiB, of
+ * which the step uses the fallback queue: 4 bytes a point and 67 KB).  sg_counters (device, 5
+ * entries, accumulated):
  * [0] points taken from the network, [1] out of range, [2] negative source,
  * [3] water residual, [4] no hydrometeor.  stats as for ice3_adjust_rain_ice (fallback
  * points only; network points report 0 calls). */

@@ -1,8 +1,10 @@
 // CPU build of the device stages of libice3_hip (dwarf-p-ice3_amd/csrc/ice3_stages.hpp),
-// for tests only: the same adjust_at / sedim_column / micro_at code the kernels run,
-// executed point by point in the kernels' launch order (all ICE_ADJUST points, then
-// every column's sedimentation, then every microphysics point), so that the kernel
-// source can be checked against the oracle and under sanitizers without a GPU.
+// for tests only: the adjust_at / sedim_column / micro_at code that the one-thread kernels
+// run (k_ice_adjust, k_sedim_walk, k_adjust_sedim, k_micro_points), executed point by point in
+// their launch order (all ICE_ADJUST points, then every column's sedimentation, then every
+// microphysics point), so that the kernel source can be checked against the oracle and under
+// sanitizers without a GPU.  k_sedim, k_sedim_split and k_micro arrange the same point
+// functions over wavefronts in code of their own, which GPU tests alone cover.
 // Entry points mirror include/ice3.h with host arrays and no context or stream.
 #include <cstdio>
 #include <cstdlib>
