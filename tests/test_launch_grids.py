@@ -109,3 +109,47 @@ def test_rain_ice_on_both_sides_of_the_walk(kind, nlev):
             assert torch.equal(new[k], whole[k][:, c:c + part]), (k, c)
         for k in diags:
             assert torch.equal(diags[k], whole_d[k][c:c + part]), (k, c)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hail", [False, True])
+@pytest.mark.parametrize("nlev", [1, 2, 3, 4, 5])
+def test_fused_step_of_few_levels(nlev, hail):
+    """The fused step over more columns than its walk of any number of levels begins at, against the same
+    columns in calls of fewer than its walk of three levels begins at (one and two levels are walked in
+    both: ICE_ADJUST, the sedimentation and the microphysics one by one stand beside them)."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ice3_amd import AdjustRainIce, AdjustRainIceHail, _lib, synthetic
+    from ice3_amd._fields import ptr
+    ncu = torch.cuda.get_device_properties(0).multi_processor_count
+    ncol, part = 432 * ncu + 1, 143 * ncu - 1
+    f = synthetic.generate(2048, 90, seed=20260404, variant="pipeline")
+    f = {k: v[:3 * nlev:3] if v.ndim == 2 else v for k, v in f.items()}
+    f["rhodref"] = f["rho_dry_ref"]
+    f["rh"] = f["rg"] * 0.7
+    f["rhs"] = f["rh"] / DT
+    f = {k: torch.from_numpy(np.ascontiguousarray(v)).cuda() for k, v in f.items()}
+    f = {k: v.repeat((1,) * (v.dim() - 1) + (-(-ncol // 2048),))[..., :ncol].contiguous() for k, v in f.items()}
+    for k in ("rrs", "ris", "rss", "rgs", "dzz"):
+        f[k] = f[k] * torch.linspace(0.5, 1.5, ncol, dtype=torch.float64, device="cuda")
+    call = AdjustRainIceHail() if hail else AdjustRainIce()
+    whole = call(f, DT)
+    for c in range(0, ncol, part):
+        res = call({k: v[..., c:c + part].contiguous() for k, v in f.items()}, DT)
+        for k, v in res.items():
+            assert torch.equal(v, whole[k][..., c:c + part]), (k, c)
+    if hail:
+        return
+    out = {k: torch.empty((nlev, ncol), dtype=torch.float64, device="cuda") for k in _lib.PIPE_OUT_FIELDS[:15]}
+    out.update({k: torch.empty(ncol, dtype=torch.float64, device="cuda") for k in _lib.PIPE_OUT_FIELDS[15:]})
+    fin = _lib.PipeIn(*[ptr(f[k]) for k in _lib.PIPE_IN_FIELDS])
+    fout = _lib.PipeOut(*[ptr(out[k]) for k in _lib.PIPE_OUT_FIELDS])
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for stage in (_lib.STAGE_ADJUST, _lib.STAGE_SEDIMENTATION, _lib.STAGE_MICROPHYSICS):
+        assert _lib.load().ice3_adjust_rain_ice_stages(_lib.context(0), _lib.PREC_FP64, ncol, nlev, ncol, DT,
+                                                       ctypes.byref(fin), ctypes.byref(fout), None, stage,
+                                                       stream) == _lib.ICE3_OK
+    for k, v in out.items():
+        assert torch.equal(v, whole[k]), k
